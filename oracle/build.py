@@ -21,6 +21,11 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 REFERENCE = "/root/reference"
 
 
+def have_reference() -> bool:
+    """The reference's headers are there (the folder may exist and be empty)."""
+    return os.path.exists(os.path.join(REFERENCE, "Complex.h"))
+
+
 def build_oracle(verbose: bool = True) -> str:
     out = os.path.join(HERE, "liboracle.so")
     cmd = ["gcc", "-O2", "-fPIC", "-shared", "-Wall", "-o", out, os.path.join(HERE, "oracle.c"), "-lm"]
@@ -32,7 +37,7 @@ def build_oracle(verbose: bool = True) -> str:
 
 def build_ref(verbose: bool = True) -> str | None:
     """Compile the reference-header checker, if the reference tree is present."""
-    if not os.path.isdir(REFERENCE):
+    if not have_reference():
         if verbose:
             print("reference tree absent: oracle/_ref not rebuilt", flush=True)
         return None
@@ -50,7 +55,7 @@ def build_dropin(verbose: bool = True) -> str | None:
     the reference tree and a built estl_amd/libestl_hip.so)."""
     repo = os.path.dirname(HERE)
     lib = os.path.join(repo, "estl_amd", "libestl_hip.so")
-    if not os.path.isdir(REFERENCE) or not os.path.exists(lib):
+    if not have_reference() or not os.path.exists(lib):
         if verbose:
             print("reference tree or libestl_hip.so absent: oracle/_ref/dropin_check not rebuilt", flush=True)
         return None
