@@ -22,6 +22,7 @@
 //   * k_conv_rows on binary16 rows, k_filter_l1, k_spec_l1, k_conv_scales: the FP16-storage
 //                   variant (and group forms of the last three for request groups).
 #include "fft_block.h"
+#include "fft_wave.h"
 #include "internal.h"
 
 namespace estl {
@@ -90,8 +91,17 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
         spec = const_cast<float2 *>(group->spec[q]);
     }
     float2 v[E];
+    if (k <= N) {
+        // every value is one tap or none: all of a thread's loads in flight at once
 #pragma unroll
-    for (int i = 0; i < E; ++i) v[i] = make_float2(fold_tap(h, k, N, shift, tl + TPT * i), 0.0f);
+        for (int i = 0; i < E; ++i) {
+            const long e = (tl + TPT * i + shift) & (N - 1);
+            v[i] = make_float2(e < k ? h[e] : 0.0f, 0.0f);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < E; ++i) v[i] = make_float2(fold_tap(h, k, N, shift, tl + TPT * i), 0.0f);
+    }
     // kSpecTw: the power table below 4096 points, the block table from 4096
     block_fft<LOG2N, -1, kLdsPad, false, kSpecTw<LOG2N>>(v, lds, tl, tw, false);
     if (normalize) {
@@ -124,8 +134,22 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
             if (tl == 0) *l1_single = make_float2(L, l1);
         }
     }
+    if constexpr (LOG2N >= kWaveMinLog2) {
+        // bins to the order k_conv_rows and k_conv_ols of this length read them in
+        using P = Lds<kLdsPad>;
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < E; ++i) spec[tl + TPT * i] = v[i];
+        for (int i = 0; i < E; ++i) lds[P::idx(tl + TPT * i)] = v[i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const int pos = tl + TPT * i;
+            spec[pos] = lds[P::idx(wave_bin<LOG2N>(pos))];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < E; ++i) spec[tl + TPT * i] = v[i];
+    }
 }
 
 // l1_single (one filter, FP16 storage, N >= 2^12): the spectrum divided by its L and
@@ -155,14 +179,64 @@ __device__ __forceinline__ float ld_real(const _Float16 *p) { return (float)*p; 
 __device__ __forceinline__ void st_real(float *p, float v) { st_stream_f(p, v); }
 __device__ __forceinline__ void st_real(_Float16 *p, float v) { *p = (_Float16)v; }
 
-// Persistent over pairs of real rows (TPW pairs per workgroup, four resident rounds of
-// workgroups; one workgroup per group measured within 2 % either way at 1024-8192
-// points, so the grid stays).  With
-// a request group, `rows` counts the group's pairs twice and each slot takes its pair's
-// member: input rows, spectrum and output rows.  R: the stored real type, float or
-// _Float16 (FP16 storage: the spectrum has been divided by the filter's L1 norm, so
-// every stored output lies in [-1, 1] (|y| <= sum |h| max |x|); the caller's per-row
-// scales carry the magnitudes).
+// Pairs of real rows of N >= 2^10 values, TPW = max(1, 256 / T) pairs per workgroup and
+// one workgroup per group of pairs: forward transform, multiply, inverse transform in
+// registers (wave_fft), each value read and written once.  With a request group, `rows`
+// counts the group's pairs twice and each slot takes its pair's member: input rows,
+// spectrum and output rows.  R: the stored real type, float or _Float16 (FP16 storage: the
+// spectrum has been divided by the filter's L1 norm, so every stored output lies in
+// [-1, 1] (|y| <= sum |h| max |x|); the caller's per-row scales carry the magnitudes).
+// Bound by HBM and VALU alike: 75 vector instructions per complex value at 2^10 points and
+// no barrier (16 values per thread and three exchanges across the workgroup took 105).
+// 30001 rows of 1024 values: 55.8 -> 49.2 us (4.40 -> 4.99 TB/s).
+template <int LOG2N, int TPW, bool CORR, typename R>
+__global__ void __launch_bounds__(WaveGeom<LOG2N>::T * TPW) __attribute__((amdgpu_waves_per_eu(4)))
+k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 *__restrict__ spec,
+            const float2 *__restrict__ tw, float scale, const ConvGroup *__restrict__ group) {
+    using G = WaveGeom<LOG2N>;
+    constexpr int N = G::N, T = G::T;
+    __shared__ float lds[TPW * G::lds_floats];
+    const int w = TPW > 1 ? threadIdx.x / T : 0, t = TPW > 1 ? threadIdx.x % T : threadIdx.x;
+    const long pairs = (rows + 1) / 2;
+    const long pr = (long)blockIdx.x * TPW + w;
+    const bool active = pr < pairs;
+    long r1 = active ? 2 * pr : 0, nrows = rows;
+    if (group) {
+        const int q = active ? conv_group_member(group, pr) : 0;
+        r1 = active ? 2 * (pr - group->pair_start[q]) : 0;
+        nrows = group->real_rows[q];
+        x = static_cast<const R *>(group->x[q]);
+        y = static_cast<R *>(group->y[q]);
+        spec = group->spec[q];
+    }
+    // a last pair of one row computes that row twice and stores it once
+    const bool two = active && r1 + 1 < nrows;
+    const R *x1 = global_ptr(x) + r1 * N + t, *x2 = two ? x1 + N : x1;
+    spec = global_ptr(spec);
+    float2 v[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) v[i] = make_float2(ld_real(x1 + T * i), ld_real(x2 + T * i));
+    float *slice = lds + w * G::lds_floats;
+    wave_fft<LOG2N>(v, slice, t, tw, false);
+#pragma unroll
+    for (int r = 0; r < 32; ++r) {
+        const float2 hk = spec[t + T * r];
+        v[r] = CORR ? cmulc(v[r], hk) : cmul(v[r], hk);
+    }
+    wave_ifft<LOG2N>(v, slice, t, tw);
+    if (active) {
+        R *y1 = global_ptr(y) + r1 * N + t;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) st_real(y1 + T * i, v[i].x * scale);
+        if (two) {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) st_real(y1 + N + T * i, v[i].y * scale);
+        }
+    }
+}
+
+// The same for rows of N < 2^10 values (16 values per thread, bins in natural order),
+// persistent over the pairs (four resident rounds of workgroups).
 template <int LOG2N, int TPW, bool CORR, typename R>
 __global__ void __launch_bounds__(BlockGeom<LOG2N>::TPT * TPW) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_rows(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 *__restrict__ spec,
@@ -386,61 +460,92 @@ struct OlsArgs {
     int pre;      // first valid position in a window
 };
 
-// Four waves per SIMD (at most 128 VGPRs): two 512-thread workgroups per CU at L = 2^13,
-// one of 1024 threads at 2^14.
+// One workgroup per pair of windows, 32 values per thread, at most 128 VGPRs and 33 / 66
+// KiB of LDS: four waves per SIMD, four workgroups per CU at L = 2^13 and two at 2^14, so
+// one's loads and stores overlap another's arithmetic.  Bound by the vector instructions
+// (~110 per complex value and two transforms; 16 values per thread took ~148, with twelve
+// barriers a window pair instead of seven).  63 rows of 2^20 values and 2049 taps (2^13
+// windows): 203 -> 154 us; 101 binary16 rows of 2^18 and 6001 taps (2^14), spectrum
+// included: 153 -> 96 us.
 template <int LOG2L, bool CORR, typename R>
-__global__ void __launch_bounds__(BlockGeom<LOG2L>::TPT) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(WaveGeom<LOG2L>::T) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *__restrict__ spec,
            const float2 *__restrict__ tw, float scale) {
-    using G = BlockGeom<LOG2L>;
-    constexpr int E = G::E, TPT = G::TPT;
-    __shared__ float2 lds[Lds<kLdsPad>::size(G::N)];
+    using G = WaveGeom<LOG2L>;
+    constexpr int T = G::T, L = G::N;
+    __shared__ float lds[G::lds_floats];
+    const int t = threadIdx.x;
     if (a.s_out && blockIdx.x == 0) {
         // FP16 storage: the output row scales, s_in times L (the value after the
         // spectrum's L bins), as k_conv_scales computes them
-        const float L = spec[(size_t)1 << LOG2L].x;
-        for (long r = threadIdx.x; r < a.rows; r += TPT) a.s_out[r] = a.s_in[r] * L;
+        const float l1 = spec[(size_t)L].x;
+        for (long r = t; r < a.rows; r += T) a.s_out[r] = a.s_in[r] * l1;
     }
-    const long windows = a.rows * a.W;
-    const long pairs = (windows + 1) / 2;
-    // offsets inside a row in 32 bits (n <= 2^30): the row bases are workgroup-uniform,
-    // so loads and stores take a scalar base and a 32-bit lane offset; x[(s + i) mod n]
-    // with s >= -pre wraps correctly in unsigned arithmetic because n divides 2^32
-    const unsigned nm = (unsigned)((1L << a.log2n) - 1);
-    for (long pr = blockIdx.x; pr < pairs; pr += gridDim.x) {  // uniform across the workgroup
-        const int tl = opaque_lane(threadIdx.x);
-        const long w0 = 2 * pr, w1 = w0 + 1;
-        const bool two = w1 < windows;
-        // rows and windows, held in scalar registers (rows < 2^31, windows per row < 2^17)
-        const int r0 = __builtin_amdgcn_readfirstlane((int)(w0 / a.W));
-        const int b0 = __builtin_amdgcn_readfirstlane((int)(w0 - (long)r0 * a.W));
-        const int r1 = two ? __builtin_amdgcn_readfirstlane((int)(w1 / a.W)) : r0;
-        const int b1 = two ? __builtin_amdgcn_readfirstlane((int)(w1 - (long)r1 * a.W)) : b0;
-        const R *x0 = x + ((long)r0 << a.log2n), *x1 = x + ((long)r1 << a.log2n);
-        const unsigned m0 = (unsigned)b0 * (unsigned)a.M, m1 = (unsigned)b1 * (unsigned)a.M;  // first outputs
-        const unsigned s0 = m0 - (unsigned)a.pre + (unsigned)tl, s1 = m1 - (unsigned)a.pre + (unsigned)tl;
-        float2 v[E];
+    // rows and windows in scalar registers, offsets inside a row in 32 bits (n <= 2^30):
+    // loads and stores take a scalar base and a 32-bit lane offset
+    const unsigned W = (unsigned)a.W, windows = (unsigned)a.rows * W;
+    const unsigned w0 = 2u * blockIdx.x;
+    const bool two = w0 + 1u < windows;  // a lone last window is computed twice, stored once
+    const unsigned w1 = two ? w0 + 1u : w0;
+    const unsigned r0 = __builtin_amdgcn_readfirstlane(w0 / W), b0 = w0 - r0 * W;
+    const unsigned r1 = __builtin_amdgcn_readfirstlane(w1 / W), b1 = w1 - r1 * W;
+    const R *x0 = x + ((long)r0 << a.log2n), *x1 = x + ((long)r1 << a.log2n);
+    R *y0 = y + ((long)r0 << a.log2n), *y1 = y + ((long)r1 << a.log2n);
+    const int n = 1 << a.log2n;
+    const unsigned nm = (unsigned)n - 1u;
+    const int m0 = (int)b0 * a.M, m1 = (int)b1 * a.M;  // first outputs
+    const int s0 = m0 - a.pre, s1 = m1 - a.pre;        // first inputs; < 0 or past n - L: wraps
+    float2 v[32];
+    if (s0 >= 0 && s0 <= n - L) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            v[e] = make_float2(ld_real(x0 + ((s0 + (unsigned)(TPT * e)) & nm)),
-                               two ? ld_real(x1 + ((s1 + (unsigned)(TPT * e)) & nm)) : 0.0f);
-        }
-        block_fft<LOG2L, -1, kLdsPad, false, kTwPowers>(v, lds, tl, tw, true);
+        for (int e = 0; e < 32; ++e) v[e].x = ld_real(x0 + (s0 + T * e) + t);
+    } else {
+        // x[(s + i) mod n] wraps correctly in unsigned arithmetic: n divides 2^32
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const float2 hk = spec[tl + TPT * e];
-            v[e] = CORR ? cmulc(v[e], hk) : cmul(v[e], hk);
-        }
-        block_fft<LOG2L, +1, kLdsPad, false, kTwPowers>(v, lds, tl, tw, true);
-        const unsigned n = nm + 1u, osh = (unsigned)a.oshift;
-        R *y0 = y + ((long)r0 << a.log2n), *y1 = y + ((long)r1 << a.log2n);
+        for (int e = 0; e < 32; ++e) v[e].x = ld_real(x0 + ((unsigned)(s0 + t + T * e) & nm));
+    }
+    if (s1 >= 0 && s1 <= n - L) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const int q = tl + TPT * e - a.pre;  // position in the window's valid outputs
-            if (q < 0 || q >= a.M) continue;
-            const unsigned p0 = m0 + (unsigned)q, p1 = m1 + (unsigned)q;
-            if (p0 < n) st_real(y0 + ((p0 + osh) & nm), v[e].x * scale);
-            if (two && p1 < n) st_real(y1 + ((p1 + osh) & nm), v[e].y * scale);
+        for (int e = 0; e < 32; ++e) v[e].y = ld_real(x1 + (s1 + T * e) + t);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 32; ++e) v[e].y = ld_real(x1 + ((unsigned)(s1 + t + T * e) & nm));
+    }
+    wave_fft<LOG2L>(v, lds, t, tw, false);
+#pragma unroll
+    for (int r = 0; r < 32; ++r) {
+        const float2 hk = spec[t + T * r];
+        v[r] = CORR ? cmulc(v[r], hk) : cmul(v[r], hk);
+    }
+    wave_ifft<LOG2L>(v, lds, t, tw);
+    const int osh = (int)a.oshift;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        if (half && !two) break;
+        const int m = half ? m1 : m0;
+        R *yr = half ? y1 : y0;
+        const int live = n - m < a.M ? n - m : a.M;  // outputs of this window
+        if (m + osh + live <= n || m + osh >= n) {
+            // no output wraps: a scalar base, and a lane test only where the valid part ends
+            R *base = yr + (m + osh >= n ? m + osh - n : m + osh) - a.pre;
+#pragma unroll
+            for (int e = 0; e < 32; ++e) {
+                const int lo = T * e;
+                if (lo + T <= a.pre || lo >= a.pre + live) continue;
+                const float o = (half ? v[e].y : v[e].x) * scale;
+                if (lo >= a.pre && lo + T <= a.pre + live) {
+                    st_real(base + lo + t, o);
+                } else if (lo + t >= a.pre && lo + t < a.pre + live) {
+                    st_real(base + lo + t, o);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 32; ++e) {
+                const int q = t + T * e - a.pre;  // position in the window's valid outputs
+                if (q >= 0 && q < live)
+                    st_real(yr + ((unsigned)(m + q + osh) & nm), (half ? v[e].y : v[e].x) * scale);
+            }
         }
     }
 }
@@ -448,14 +553,11 @@ k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *
 template <int LOG2L, bool CORR, typename R>
 static hipError_t launch_conv_ols_t(const void *x, void *y, const OlsArgs &a, const float2 *spec, const float2 *tw,
                                     hipStream_t st) {
-    using G = BlockGeom<LOG2L>;
-    auto kernel = k_conv_ols<LOG2L, CORR, R>;
-    const long resident = conv_resident(kernel, G::TPT);
+    using G = WaveGeom<LOG2L>;
     const long pairs = (a.rows * a.W + 1) / 2;
-    long blocks = pairs;
-    if (blocks > 4 * resident) blocks = 4 * resident;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(G::TPT), 0, st, static_cast<const R *>(x),
-                       static_cast<R *>(y), a, spec, tw, 1.0f / (float)G::N);
+    if (a.rows > 0x7fffffffL || pairs > 0x3fffffffL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_conv_ols<LOG2L, CORR, R>), dim3((unsigned)pairs), dim3(G::T), 0, st,
+                       static_cast<const R *>(x), static_cast<R *>(y), a, spec, tw, 1.0f / (float)G::N);
     return hipGetLastError();
 }
 
@@ -487,9 +589,8 @@ static hipError_t launch_conv_ols_l(bool fp16, bool corr, const void *x, void *y
                 : launch_conv_ols_t<LOG2L, false, float>(x, y, a, spec, tw, st);
 }
 
-// x, y: rows of n FP32 (fp16 = false) or binary16 reals; spectrum and power table
-// (block_fft kTwPowers) of L = 2^log2L, log2L = 13 (512-thread workgroups, two per CU)
-// or 14 (1024 threads, one).  FP16 storage: s_in / s_out the per-row scales (the
+// x, y: rows of n FP32 (fp16 = false) or binary16 reals; spectrum and roots (wave_table)
+// of L = 2^log2L, log2L = 13 or 14.  FP16 storage: s_in / s_out the per-row scales (the
 // launch also writes s_out = s_in x L, L stored after the spectrum); null for FP32.
 hipError_t launch_conv_ols(bool fp16, bool corr, int log2L, const void *x, void *y, long rows, int log2n, long k,
                            long oshift, const float2 *spec, const float2 *tw, const float *s_in, float *s_out,
@@ -501,33 +602,29 @@ hipError_t launch_conv_ols(bool fp16, bool corr, int log2L, const void *x, void 
     return hipErrorInvalidValue;
 }
 
-template <int LOG2N, bool CORR>
-static hipError_t launch_conv_rows_t(const float *x, float *y, long rows, const float2 *spec, const float2 *tw,
-                                     float scale, hipStream_t st, const ConvGroup *group) {
-    using G = BlockGeom<LOG2N>;
-    constexpr int TPW = (G::TPT >= 256) ? 1 : 256 / G::TPT;
-    auto kernel = k_conv_rows<LOG2N, TPW, CORR, float>;
-    const long resident = conv_resident(kernel, G::TPT * TPW);
-    const long pairs = (rows + 1) / 2;
-    long blocks = (pairs + TPW - 1) / TPW;
-    if (blocks > 4 * resident) blocks = 4 * resident;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(G::TPT * TPW), 0, st, x, y, rows, spec, tw, scale, group);
-    return hipGetLastError();
-}
-
-template <int LOG2N, bool CORR>
-static hipError_t launch_conv_rows_h_t(const void *x, void *y, long rows, const float2 *spec, const float2 *tw,
-                                       float scale, hipStream_t st, const ConvGroup *group) {
-    using G = BlockGeom<LOG2N>;
-    constexpr int TPW = (G::TPT >= 256) ? 1 : 256 / G::TPT;
-    auto kernel = k_conv_rows<LOG2N, TPW, CORR, _Float16>;
-    const long resident = conv_resident(kernel, G::TPT * TPW);
-    const long pairs = (rows + 1) / 2;
-    long blocks = (pairs + TPW - 1) / TPW;
-    if (blocks > 4 * resident) blocks = 4 * resident;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(G::TPT * TPW), 0, st, static_cast<const _Float16 *>(x),
-                       static_cast<_Float16 *>(y), rows, spec, tw, scale, group);
-    return hipGetLastError();
+template <int LOG2N, bool CORR, typename R>
+static hipError_t launch_conv_rows_t(const R *x, R *y, long rows, const float2 *spec, const float2 *tw, float scale,
+                                     hipStream_t st, const ConvGroup *group) {
+    if constexpr (LOG2N >= kWaveMinLog2) {
+        using G = WaveGeom<LOG2N>;
+        constexpr int TPW = (G::T >= 256) ? 1 : 256 / G::T;
+        const long pairs = (rows + 1) / 2, groups = (pairs + TPW - 1) / TPW;
+        if (groups > 0x7fffffffL) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((k_conv_wave<LOG2N, TPW, CORR, R>), dim3((unsigned)groups), dim3(G::T * TPW), 0, st, x, y,
+                           rows, spec, tw, scale, group);
+        return hipGetLastError();
+    } else {
+        using G = BlockGeom<LOG2N>;
+        constexpr int TPW = (G::TPT >= 256) ? 1 : 256 / G::TPT;
+        auto kernel = k_conv_rows<LOG2N, TPW, CORR, R>;
+        const long resident = conv_resident(kernel, G::TPT * TPW);
+        const long pairs = (rows + 1) / 2;
+        long blocks = (pairs + TPW - 1) / TPW;
+        if (blocks > 4 * resident) blocks = 4 * resident;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(G::TPT * TPW), 0, st, x, y, rows, spec, tw, scale,
+                           group);
+        return hipGetLastError();
+    }
 }
 
 template <bool CORR>
@@ -535,7 +632,9 @@ static hipError_t launch_conv_rows_h_c(int log2n, const void *x, void *y, long r
                                        const float2 *tw, float scale, hipStream_t st, const ConvGroup *group) {
     switch (log2n) {
 #define CONV_H_CASE(L) \
-    case L: return launch_conv_rows_h_t<L, CORR>(x, y, rows, spec, tw, scale, st, group);
+    case L:                                                                                                   \
+        return launch_conv_rows_t<L, CORR>(static_cast<const _Float16 *>(x), static_cast<_Float16 *>(y), rows, spec, \
+                                           tw, scale, st, group);
         CONV_H_CASE(1) CONV_H_CASE(2) CONV_H_CASE(3) CONV_H_CASE(4) CONV_H_CASE(5) CONV_H_CASE(6) CONV_H_CASE(7)
         CONV_H_CASE(8) CONV_H_CASE(9) CONV_H_CASE(10) CONV_H_CASE(11) CONV_H_CASE(12) CONV_H_CASE(13)
 #undef CONV_H_CASE

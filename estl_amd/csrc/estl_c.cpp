@@ -110,6 +110,33 @@ int power_table(int device, int log2n, const float2 **out) {
     return ESTL_OK;
 }
 
+// Roots of the convolutions' transforms (WaveRoots, fft_wave.h): w, w^4, w^16 of
+// w = W_N^t, t in [0, N / 32), then of w = W_N^(32 t), t in [0, N / 1024).
+int wave_table(int device, int log2n, const float2 **out) {
+    auto &c = twcache();
+    std::lock_guard<std::mutex> lk(c.mu);
+    auto key = std::make_tuple(device, 3, (long)log2n, 0L, 0L);
+    auto it = c.tables.find(key);
+    if (it != c.tables.end()) {
+        *out = it->second;
+        return ESTL_OK;
+    }
+    if (log2n < kWaveMinLog2 || log2n > kOlsWideLog2)
+        return set_error(ESTL_ERR_UNSUPPORTED, "no roots table for log2n=%d", log2n);
+    const long N = 1L << log2n, T = N / 32, Q = T / 32;
+    float2 *d = nullptr;
+    hipStream_t ts = table_stream(device);
+    HIP_TRY(hipMalloc(&d, sizeof(float2) * 3 * (T + Q)));
+    for (int e = 0; e < 3; ++e) {
+        HIP_TRY(launch_twiddle(d + e * T, T, 1, 1, 1L << (2 * e), N, ts));
+        HIP_TRY(launch_twiddle(d + 3 * T + e * Q, Q, 1, 1, 32L << (2 * e), N, ts));
+    }
+    HIP_TRY(hipStreamSynchronize(ts));
+    c.tables[key] = d;
+    *out = d;
+    return ESTL_OK;
+}
+
 // Table of BlockGeom<log2n>: W_{N_q}^{g s} at [(s-1) A_q + g] per pass q >= 1.
 int block_table(int device, int log2n, const float2 **out) {
     auto &c = twcache();

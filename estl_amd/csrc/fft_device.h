@@ -80,6 +80,14 @@ __device__ __forceinline__ void st_elem(f16x2 *p, float2 x) {
     __builtin_nontemporal_store(h, p);
 }
 
+// p as a pointer to global memory, for pointers whose origin the compiler does not see (one
+// read from a descriptor, or behind an asm): it would access generic ones with flat
+// instructions, whose loads also count as LDS accesses and hold up the waits for those.
+template <class T>
+__device__ __forceinline__ T *global_ptr(T *p) {
+    return (T *)(T __attribute__((address_space(1))) *)reinterpret_cast<uintptr_t>(p);
+}
+
 // Returns p unchanged, but hides from the optimiser that it is loop-invariant.  Used on
 // twiddle-table pointers inside loops over rows/items: otherwise every twiddle load of a
 // pass is hoisted out of the loop and ~30 float2 stay live for the whole kernel, which
@@ -87,7 +95,7 @@ __device__ __forceinline__ void st_elem(f16x2 *p, float2 x) {
 template <class T>
 __device__ __forceinline__ const T *opaque(const T *p) {
     asm volatile("" : "+s"(p));
-    return p;
+    return global_ptr(p);
 }
 // Same for a per-lane value (the thread index): in loops whose body dispatches on a
 // size class, addresses derived from the thread index alone would otherwise be hoisted

@@ -1,0 +1,188 @@
+// fft_wave.h -- transforms whose order of bins does not matter (the convolutions'), with
+// one exchange across the workgroup and the rest inside waves.
+//
+// A transform of N = 2^LOG2N points (2^10 .. 2^14) is spread over T = N / 32 threads, 32
+// values per thread, and runs decimation in frequency: with n = t + T i and
+// k = k1 + 32 k',
+//
+//   X[k1 + 32 k'] = sum_t W_T^{t k'} ( W_N^{t k1} sum_i x[t + T i] W_32^{i k1} )
+//
+// the inner sum is a 32-point DFT in registers, and what is left are 32 independent
+// transforms of T points, one per k1, each over Q = T / 32 neighbouring threads -- threads
+// of one wave.  They run the same step again (t = t' + Q i', k' = k2 + 32 k3) and end in
+// transforms of Q points in registers.  So only the hand-over of the first step crosses
+// the workgroup (and nothing does up to N = 2^11); the second stays inside a wave and needs
+// no barrier.  The inverse runs the steps backwards (decimation in time), from the order
+// in which the forward left the bins: thread u = k1 Q + t' holds in register r = m Q + k3
+// bin k1 + 32 (m + (32 / Q) t') + 1024 k3, stored at r T + u in a spectrum.
+//
+// The exchanges send real and imaginary parts one after the other through half the LDS:
+// 66 KiB at 2^14 points, two workgroups per CU at four waves per SIMD, where the whole
+// values need 139 KiB and leave one.
+#pragma once
+
+#include "fft_device.h"
+#include "internal.h"
+
+namespace estl {
+
+template <int LOG2N>
+struct WaveGeom {
+    static_assert(LOG2N >= 10 && LOG2N <= 14, "32 values per thread, rows of Q <= 16 threads");
+    static constexpr int N = 1 << LOG2N, E = 32;
+    static constexpr int T = N / E;  // threads per transform
+    static constexpr int Q = T / 32;  // threads per row (the T-point transform of one k1)
+    static constexpr bool in_wave = T <= 64;
+    // Floats from one row's LDS slice to the next.  A row holds its T values (first
+    // exchange), or them with one float of padding after every 32 (second).  33 Q puts the
+    // 32 / Q rows of 32 lanes on distinct groups of Q banks: no access of either exchange
+    // has a bank conflict.
+    static constexpr int RS = 33 * Q;
+    static constexpr int lds_floats = 32 * RS;
+};
+
+// the bin that position pos = r T + u of such a spectrum holds
+template <int LOG2N>
+__host__ __device__ constexpr int wave_bin(int pos) {
+    using G = WaveGeom<LOG2N>;
+    const int r = pos / G::T, u = pos % G::T;
+    return u / G::Q + 32 * (r / G::Q + (32 / G::Q) * (u % G::Q)) + 1024 * (r % G::Q);
+}
+
+// Orders this wave's LDS accesses (a wave's LDS operations execute in order; the
+// compiler must not move them across).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <bool IN_WAVE>
+__device__ __forceinline__ void exchange_sync() {
+    if constexpr (IN_WAVE) wave_lds_fence();
+    else __syncthreads();
+}
+
+// Twiddle roots of a transform (wave_table): w, w^4 and w^16 of w = W_N^t for t in [0, T),
+// three arrays of T values, then of w = W_T^t' for t' in [0, Q), each value correctly
+// rounded.
+template <int LOG2N>
+struct WaveRoots {
+    static constexpr int first = 0, second = 3 * WaveGeom<LOG2N>::T;
+    static constexpr int size = 3 * (WaveGeom<LOG2N>::T + WaveGeom<LOG2N>::Q);
+};
+
+// v[k] *= w^k (its conjugate for DIR > 0) for k in [0, 32), with w, w^4, w^16 read from
+// `roots` at a stride of STRIDE: k = a + 4 b + 16 c, each factor at most two products from
+// a rounded root, and the roots' errors grow by 3 + 3 + 1 at most (by 31 as powers of w
+// alone, which a 32-point step at full length shows in the result).
+template <int DIR, int STRIDE>
+__device__ __forceinline__ void twiddle32(float2 (&v)[32], const float2 *__restrict__ roots, int t) {
+    // read and raised anew at each use: kept from the forward transform for the inverse
+    // the powers would take 60 registers
+    const float2 *p = opaque(roots);
+    float2 lo[4], hi[8];
+    lo[1] = p[t];
+    hi[1] = p[STRIDE + t];
+    hi[4] = p[2 * STRIDE + t];
+    lo[2] = cmul(lo[1], lo[1]);
+    lo[3] = cmul(lo[2], lo[1]);
+    hi[2] = cmul(hi[1], hi[1]);
+    hi[3] = cmul(hi[2], hi[1]);
+    StaticFor<5, 8>::run([&](auto ac) { hi[decltype(ac)::value] = cmul(hi[4], hi[decltype(ac)::value - 4]); });
+    StaticFor<0, 8>::run([&](auto ac) {
+        constexpr int a = decltype(ac)::value;
+        if constexpr (a > 0) v[4 * a] = ctw<DIR>(v[4 * a], hi[a]);
+        StaticFor<1, 4>::run([&](auto bc) {
+            constexpr int b = decltype(bc)::value;
+            float2 w = lo[b];
+            if constexpr (a > 0) w = cmul(hi[a], lo[b]);
+            v[4 * a + b] = ctw<DIR>(v[4 * a + b], w);
+        });
+    });
+}
+
+// v[i] = x[t + T i] on entry, bin k1 + 32 (m + (32 / Q) t') + 1024 k3 in v[m Q + k3] on exit.
+// `lds` holds WaveGeom::lds_floats floats of this transform.  All threads of the
+// workgroup call it together; `tw` is the table of WaveRoots.  With lds_busy, other threads may still be reading the slice.
+template <int LOG2N>
+__device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, const float2 *__restrict__ tw, bool lds_busy) {
+    using G = WaveGeom<LOG2N>;
+    constexpr int T = G::T, Q = G::Q, RS = G::RS;
+    float *row = lds + (t / Q) * RS;
+    const int tq = t % Q;
+    Dft<32, -1>::run(v);
+    twiddle32<-1, T>(v, tw + WaveRoots<LOG2N>::first, t);
+    if (lds_busy) exchange_sync<G::in_wave>();
+#pragma unroll
+    for (int k = 0; k < 32; ++k) lds[k * RS + t] = v[k].x;
+    exchange_sync<G::in_wave>();
+#pragma unroll
+    for (int i = 0; i < 32; ++i) v[i].x = row[tq + Q * i];
+    exchange_sync<G::in_wave>();
+#pragma unroll
+    for (int k = 0; k < 32; ++k) lds[k * RS + t] = v[k].y;
+    exchange_sync<G::in_wave>();
+#pragma unroll
+    for (int i = 0; i < 32; ++i) v[i].y = row[tq + Q * i];
+    Dft<32, -1>::run(v);
+    if constexpr (Q > 1) {
+        twiddle32<-1, Q>(v, tw + WaveRoots<LOG2N>::second, tq);
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < 32; ++k) row[k * Q + (k * Q >> 5) + tq] = v[k].x;
+        wave_lds_fence();
+#pragma unroll
+        for (int r = 0; r < 32; ++r) v[r].x = row[33 * tq + r];
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < 32; ++k) row[k * Q + (k * Q >> 5) + tq] = v[k].y;
+        wave_lds_fence();
+#pragma unroll
+        for (int r = 0; r < 32; ++r) v[r].y = row[33 * tq + r];
+        StaticFor<0, 32 / Q>::run([&](auto mc) { Dft<Q, -1>::run(v + Q * decltype(mc)::value); });
+    }
+}
+
+// The unnormalised inverse: bins in the order wave_fft leaves them to x[t + T i] in v[i].
+// The caller's own wave was the last to read its rows of the slice (wave_fft's end state).
+template <int LOG2N>
+__device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, const float2 *__restrict__ tw) {
+    using G = WaveGeom<LOG2N>;
+    constexpr int T = G::T, Q = G::Q, RS = G::RS;
+    float *row = lds + (t / Q) * RS;
+    const int tq = t % Q;
+    if constexpr (Q > 1) {
+        StaticFor<0, 32 / Q>::run([&](auto mc) { Dft<Q, +1>::run(v + Q * decltype(mc)::value); });
+        wave_lds_fence();
+#pragma unroll
+        for (int r = 0; r < 32; ++r) row[33 * tq + r] = v[r].x;
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < 32; ++k) v[k].x = row[k * Q + (k * Q >> 5) + tq];
+        wave_lds_fence();
+#pragma unroll
+        for (int r = 0; r < 32; ++r) row[33 * tq + r] = v[r].y;
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < 32; ++k) v[k].y = row[k * Q + (k * Q >> 5) + tq];
+        twiddle32<+1, Q>(v, tw + WaveRoots<LOG2N>::second, tq);
+    }
+    Dft<32, +1>::run(v);
+    wave_lds_fence();
+#pragma unroll
+    for (int i = 0; i < 32; ++i) row[tq + Q * i] = v[i].x;
+    exchange_sync<G::in_wave>();
+#pragma unroll
+    for (int k = 0; k < 32; ++k) v[k].x = lds[k * RS + t];
+    exchange_sync<G::in_wave>();
+#pragma unroll
+    for (int i = 0; i < 32; ++i) row[tq + Q * i] = v[i].y;
+    exchange_sync<G::in_wave>();
+#pragma unroll
+    for (int k = 0; k < 32; ++k) v[k].y = lds[k * RS + t];
+    twiddle32<+1, T>(v, tw + WaveRoots<LOG2N>::first, t);
+    Dft<32, +1>::run(v);
+}
+
+}  // namespace estl

@@ -117,6 +117,9 @@ constexpr int kSpecBlockTwLog2 = 12;  // filter spectra of at least 2^12 points 
 constexpr int kMaxPassLog2 = 13;   // largest radix of a global pass
 constexpr int kMaxPassTileLog2 = 14;  // a pass tile holds at most 2^14 values (~139 KiB of LDS)
 constexpr int kMaxPassCols = 6;    // at most 2^6 columns per tile
+// convolutions of 2^10 values and more (k_conv_wave, k_conv_ols) keep 32 values per thread
+// and a spectrum in the order their transform leaves it (fft_wave.h)
+constexpr int kWaveMinLog2 = 10;
 constexpr int kOlsLog2 = 13;       // overlap-save convolution windows of 2^13 values
 constexpr int kOlsWideLog2 = 14;   // and of 2^14 values (rows of n >= 2^15)
 #ifndef ESTL_OLS_MAX_TAPS

@@ -73,6 +73,7 @@ inline size_t planar_bytes(long count) {
 int current_device();
 int block_table(int device, int log2n, const float2 **out);
 int power_table(int device, int log2n, const float2 **out);  // block_fft's kTwPowers table
+int wave_table(int device, int log2n, const float2 **out);   // fft_wave.h's roots, log2n = 10..14
 int linear_table(int device, long count, long mult, long nq, const float2 **out);
 std::vector<int> default_pass_split(int log2n);
 int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned flags, const std::vector<int> *split,
@@ -100,7 +101,8 @@ struct ConvShape {
     unsigned flags = 0;
     bool corr = false, fused = false;
     float scale = 1.0f;
-    const float2 *tw_rows = nullptr;  // power table of the fused rows kernel (n <= 2^13)
+    const float2 *tw_rows = nullptr;  // table of the fused rows kernel (n <= 2^13): roots from
+                                      // 2^10 values (k_conv_wave), the power table below
     Plan spec_plan;                  // forward FFT of the folded filter (batch 1)
     const float2 *tw_spec = nullptr;  // k_filter_spectrum's table when spec_plan is a rows plan
     std::vector<PassStep> fwd, inv;  // multi-pass pipeline (n > 2^13): fwd, mid, inv
@@ -113,9 +115,9 @@ struct ConvShape {
     bool half = false;
     Plan half_fwd, half_inv;
     // tables of the overlap-save windows of 2^13 (n > 2^13) and 2^14 (n > 2^14) values:
-    // block tables (the filter's window spectrum, kSpecTw) and power tables (k_conv_ols)
+    // block tables (the filter's window spectrum, kSpecTw) and roots (k_conv_ols)
     const float2 *tw_ols[2] = {nullptr, nullptr};
-    const float2 *tw_ols_pow[2] = {nullptr, nullptr};
+    const float2 *tw_ols_roots[2] = {nullptr, nullptr};
 };
 bool conv_half_path(long n, long rows, int precision);
 // Rows longer than an overlap-save window convolved with a filter of at most
