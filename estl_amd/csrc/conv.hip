@@ -179,6 +179,22 @@ __device__ __forceinline__ float ld_real(const _Float16 *p) { return (float)*p; 
 __device__ __forceinline__ void st_real(float *p, float v) { st_stream_f(p, v); }
 __device__ __forceinline__ void st_real(_Float16 *p, float v) { *p = (_Float16)v; }
 
+// v[r] times bin r T + t of a spectrum (its conjugate with CORR), eight bins in flight at a
+// time: the compiler's schedule has all 32 and spills for them.
+template <bool CORR, int T>
+__device__ __forceinline__ void multiply_spectrum(float2 (&v)[32], const float2 *__restrict__ spec, int t) {
+#pragma unroll
+    for (int c = 0; c < 32; c += 8) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = c; r < c + 8; ++r) {
+            const float2 hk = spec[t + T * r];
+            v[r] = CORR ? cmulc(v[r], hk) : cmul(v[r], hk);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // Pairs of real rows of N >= 2^10 values, TPW = max(1, 256 / T) pairs per workgroup and
 // one workgroup per group of pairs: forward transform, multiply, inverse transform in
 // registers (wave_fft), each value read and written once.  With a request group, `rows`
@@ -186,9 +202,9 @@ __device__ __forceinline__ void st_real(_Float16 *p, float v) { *p = (_Float16)v
 // spectrum and output rows.  R: the stored real type, float or _Float16 (FP16 storage: the
 // spectrum has been divided by the filter's L1 norm, so every stored output lies in
 // [-1, 1] (|y| <= sum |h| max |x|); the caller's per-row scales carry the magnitudes).
-// Bound by HBM and VALU alike: 75 vector instructions per complex value at 2^10 points and
+// Bound by HBM and VALU alike: 65 vector instructions per complex value at 2^10 points and
 // no barrier (16 values per thread and three exchanges across the workgroup took 105).
-// 30001 rows of 1024 values: 55.8 -> 49.2 us (4.40 -> 4.99 TB/s).
+// 30001 rows of 1024 values: 55.3 -> 49.7 us (4.44 -> 4.94 TB/s); 4001 rows of 8192: 83 -> 59 us.
 template <int LOG2N, int TPW, bool CORR, typename R>
 __global__ void __launch_bounds__(WaveGeom<LOG2N>::T * TPW) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 *__restrict__ spec,
@@ -218,11 +234,7 @@ k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
     for (int i = 0; i < 32; ++i) v[i] = make_float2(ld_real(x1 + T * i), ld_real(x2 + T * i));
     float *slice = lds + w * G::lds_floats;
     wave_fft<LOG2N>(v, slice, t, tw, false);
-#pragma unroll
-    for (int r = 0; r < 32; ++r) {
-        const float2 hk = spec[t + T * r];
-        v[r] = CORR ? cmulc(v[r], hk) : cmul(v[r], hk);
-    }
+    multiply_spectrum<CORR, T>(v, spec, t);
     wave_ifft<LOG2N>(v, slice, t, tw);
     if (active) {
         R *y1 = global_ptr(y) + r1 * N + t;
@@ -463,10 +475,11 @@ struct OlsArgs {
 // One workgroup per pair of windows, 32 values per thread, at most 128 VGPRs and 33 / 66
 // KiB of LDS: four waves per SIMD, four workgroups per CU at L = 2^13 and two at 2^14, so
 // one's loads and stores overlap another's arithmetic.  Bound by the vector instructions
-// (~110 per complex value and two transforms; 16 values per thread took ~148, with twelve
-// barriers a window pair instead of seven).  63 rows of 2^20 values and 2049 taps (2^13
-// windows): 203 -> 154 us; 101 binary16 rows of 2^18 and 6001 taps (2^14), spectrum
-// included: 153 -> 96 us.
+// (~92 per complex value and two transforms; 16 values per thread took ~148, with twelve
+// barriers a window pair instead of seven), which keep the SIMDs 96 % busy while four
+// waves each are resident, at a clock that power holds to 2.0-2.3 GHz; the rest is the last
+// round.  63 rows of 2^20 values and 2049 taps (2^13 windows): 201 -> 147 us; 101 binary16
+// rows of 2^18 and 6001 taps (2^14), spectrum included: 153 -> 94 us.
 template <int LOG2L, bool CORR, typename R>
 __global__ void __launch_bounds__(WaveGeom<LOG2L>::T) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *__restrict__ spec,
@@ -512,11 +525,7 @@ k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *
         for (int e = 0; e < 32; ++e) v[e].y = ld_real(x1 + ((unsigned)(s1 + t + T * e) & nm));
     }
     wave_fft<LOG2L>(v, lds, t, tw, false);
-#pragma unroll
-    for (int r = 0; r < 32; ++r) {
-        const float2 hk = spec[t + T * r];
-        v[r] = CORR ? cmulc(v[r], hk) : cmul(v[r], hk);
-    }
+    multiply_spectrum<CORR, T>(v, spec, t);
     wave_ifft<LOG2L>(v, lds, t, tw);
     const int osh = (int)a.oshift;
 #pragma unroll

@@ -81,7 +81,8 @@ static hipStream_t table_stream(int device) {
 }
 
 // Power table of BlockGeom<log2n> (block_fft's kTwPowers): W_{N_q}^g at powoff(q) + g,
-// g in [0, A_q), per pass q >= 1; FP64 on the device, rounded once.
+// g in [0, A_q), per pass q >= 1, then their fourth powers in the same order; FP64 on the
+// device, rounded once.
 int power_table(int device, int log2n, const float2 **out) {
     auto &c = twcache();
     std::lock_guard<std::mutex> lk(c.mu);
@@ -97,21 +98,21 @@ int power_table(int device, int log2n, const float2 **out) {
     hipStream_t ts = table_stream(device);
     HIP_TRY(hipMalloc(&d, sizeof(float2) * (count > 0 ? count : 1)));
     long off = 0;
-    for (int q = 1; q < rows_pass_count(log2n); ++q) {
-        long A;
-        int B;
-        rows_pass_params(log2n, q, &A, &B);
-        HIP_TRY(launch_twiddle(d + off, A, 1, A, 1, A * B, ts));
-        off += A;
-    }
+    for (int e = 1; e <= 4; e += 3)
+        for (int q = 1; q < rows_pass_count(log2n); ++q) {
+            long A;
+            int B;
+            rows_pass_params(log2n, q, &A, &B);
+            HIP_TRY(launch_twiddle(d + off, A, 1, A, e, A * B, ts));
+            off += A;
+        }
     HIP_TRY(hipStreamSynchronize(ts));
     c.tables[key] = d;
     *out = d;
     return ESTL_OK;
 }
 
-// Roots of the convolutions' transforms (WaveRoots, fft_wave.h): w, w^4, w^16 of
-// w = W_N^t, t in [0, N / 32), then of w = W_N^(32 t), t in [0, N / 1024).
+// Roots of the convolutions' transforms, in the order of WaveRoots (fft_wave.h).
 int wave_table(int device, int log2n, const float2 **out) {
     auto &c = twcache();
     std::lock_guard<std::mutex> lk(c.mu);
@@ -126,10 +127,14 @@ int wave_table(int device, int log2n, const float2 **out) {
     const long N = 1L << log2n, T = N / 32, Q = T / 32;
     float2 *d = nullptr;
     hipStream_t ts = table_stream(device);
-    HIP_TRY(hipMalloc(&d, sizeof(float2) * 3 * (T + Q)));
+    const long bin = 96, pos = bin + 2048, point = pos + 3 * Q;
+    HIP_TRY(hipMalloc(&d, sizeof(float2) * (point + 3 * T)));
     for (int e = 0; e < 3; ++e) {
-        HIP_TRY(launch_twiddle(d + e * T, T, 1, 1, 1L << (2 * e), N, ts));
-        HIP_TRY(launch_twiddle(d + 3 * T + e * Q, Q, 1, 1, 32L << (2 * e), N, ts));
+        const long power = 1L << (2 * e);
+        HIP_TRY(launch_twiddle(d + 32 * e, 32, 1, 1, N / 1024 * power, N, ts));
+        if (e < 2) HIP_TRY(launch_twiddle(d + bin + 1024 * e, 1024, 2, Q, power, N, ts));
+        HIP_TRY(launch_twiddle(d + pos + Q * e, Q, 1, 1, 32 * power, N, ts));
+        HIP_TRY(launch_twiddle(d + point + T * e, T, 1, 1, power, N, ts));
     }
     HIP_TRY(hipStreamSynchronize(ts));
     c.tables[key] = d;

@@ -44,13 +44,13 @@ struct BlockGeom {
     }
     static constexpr long twsize = twoff(P);
     // the power table (TwPowers): W_{N_q}^g for g in [0, A_q) per pass q >= 1, at
-    // powoff(q)
+    // powoff(q), and their fourth powers powsum further on
     static constexpr long powoff(int q) {
         long o = 0;
         for (int p = 1; p < q; ++p) o += A(p);
         return o;
     }
-    static constexpr long powsize = powoff(P);
+    static constexpr long powsum = powoff(P), powsize = 2 * powsum;
     static constexpr bool uses_lds = TPT > 1;
 };
 
@@ -58,19 +58,17 @@ struct BlockGeom {
 // W_{N_q}^{g s} for s in [1, B_q)):
 //   kTwBlock:  every W_{N_q}^{g s} read from the block table (B_q - 1 reads per
 //              butterfly; the table is N values, 128 KiB at N = 2^14);
-//   kTwPowers: one read, w = W_{N_q}^g from the power table (sum of the A_q, 34 KiB at
-//              2^14, mostly cache-resident); w^(2^k) by squaring, and w^s as the product
-//              of the w^(2^k) of the set bits of s -- at most six products deep from the
-//              correctly rounded w (a few ulp), with only the log2 B powers live.  Trades
-//              the long-latency reads of a table too big for L1 for VALU work.
+//   kTwPowers: two reads, w = W_{N_q}^g and w^4 from the power table (twice the sum of the
+//              A_q, 68 KiB at 2^14, mostly cache-resident); w^2 and w^8 by squaring, and the
+//              twiddles of each level of the DFT from them (dft_twiddled).  Trades the long-latency reads of
+//              a table too big for L1 for VALU work.
 enum { kTwBlock = 0, kTwPowers = 1 };
 // Twiddle source of the rows kernels (k_fft_rows, _planar, _h): powers at every
-// row length (a rows plan's table is the power table, estl_c.cpp).  With powers the
-// rows kernel of 4096 and 8192 points needs 68-75 VGPRs; the block table's twiddles
-// kept in registers across rows had needed 167-206 (three waves per SIMD at 4096 points,
-// two at 8192) and measured 6-9 % slower, and read again for each row from L2 they cost
-// more.  The price is a few ulp per twiddle: rel-L2 against FP64 1.2e-7 -> 3.0e-7 at
-// 4096 points (the bound is 1.2e-5).
+// row length (a rows plan's table is the power table, estl_c.cpp).  The block table's
+// twiddles kept in registers across rows needed 167-206 VGPRs and measured 6-9 % slower at
+// 4096 and 8192 points, and read again for each row from L2 they cost more.  Rel-L2
+// against FP64 is 1.6e-7 at 4096 points (the bound is 1.2e-5): 3.0e-7 when every power
+// came from w alone, 1.2e-7 with the block table's rounded values.
 template <int LOG2N>
 constexpr int kRowsTw = kTwPowers;
 // Twiddle source of the filter spectrum (k_filter_spectrum): the block table from 4096
@@ -79,27 +77,6 @@ constexpr int kRowsTw = kTwPowers;
 // spectrum -- and the convolution by it -- within 2e-6 of the shifted input.
 template <int LOG2N>
 constexpr int kSpecTw = LOG2N < kSpecBlockTwLog2 ? kTwPowers : kTwBlock;
-template <int B, int DIR>
-__device__ __forceinline__ void apply_twiddle_powers(float2 (&u)[B], float2 w) {
-    constexpr int LB = __builtin_ctz(B);
-    float2 p[LB > 0 ? LB : 1];
-    p[0] = w;
-    StaticFor<1, LB>::run([&](auto kc) {
-        constexpr int k = decltype(kc)::value;
-        p[k] = cmul(p[k - 1], p[k - 1]);
-    });
-    StaticFor<1, B>::run([&](auto sc) {
-        constexpr int s = decltype(sc)::value;
-        constexpr int lo = __builtin_ctz(s);
-        float2 t = p[lo];
-        StaticFor<lo + 1, LB>::run([&](auto bc) {
-            constexpr int b = decltype(bc)::value;
-            if constexpr ((s >> b) & 1) t = cmul(t, p[b]);
-        });
-        u[s] = ctw<DIR>(u[s], t);
-    });
-}
-
 // LDS layouts of a sequence's exchange buffer.
 //  kLdsPad: one float2 of padding after every 16 values; addresses stay base + constant,
 //           so the exchange reads use immediate offsets (fewest VGPRs);
@@ -115,6 +92,12 @@ template <>
 struct Lds<kLdsPad> {
     static constexpr int size(int n) { return n + (n >> 4); }
     static __device__ __forceinline__ int idx(int i) { return i + (i >> 4); }
+    // idx(i + off), given idx(i), where adding off to i carries nothing into bit 4 (off a
+    // multiple of 16, or i + off within the 16 values of i): one add with a constant, which
+    // the LDS instructions take as their offset.  Formed from i + off, each address cost two
+    // to four instructions (the 4096-point rows kernel had 845 vector instructions; 619
+    // with these and dft_dit's folded twiddles).
+    static __device__ __forceinline__ constexpr int step(int at, int off) { return at + off + (off >> 4); }
 };
 template <>
 struct Lds<kLdsXor> {
@@ -153,8 +136,12 @@ __device__ __forceinline__ void block_fft(float2 (&v)[BlockGeom<LOG2N>::E], floa
             });
         } else {
             if (q > 1 || lds_busy) __syncthreads();
+            const int at = Lds<LAYOUT>::idx(tl);
 #pragma unroll
-            for (int i = 0; i < E; ++i) lds[Lds<LAYOUT>::idx(tl + TPT * i)] = v[i];
+            for (int i = 0; i < E; ++i) {
+                if constexpr (LAYOUT == kLdsPad && TPT % 16 == 0) lds[Lds<kLdsPad>::step(at, TPT * i)] = v[i];
+                else lds[Lds<LAYOUT>::idx(tl + TPT * i)] = v[i];
+            }
             __syncthreads();
             StaticFor<0, NB>::run([&](auto bc) {
                 constexpr int b = decltype(bc)::value;
@@ -162,16 +149,23 @@ __device__ __forceinline__ void block_fft(float2 (&v)[BlockGeom<LOG2N>::E], floa
                 const int g = j / S, z = j % S;   // S is a power of two
                 const int base = S * B * g + z;
                 float2 u[B];
+                const int from = Lds<LAYOUT>::idx(base);
 #pragma unroll
-                for (int s = 0; s < B; ++s) u[s] = lds[Lds<LAYOUT>::idx(base + S * s)];
+                for (int s = 0; s < B; ++s) {
+                    // base is a multiple of S B plus z < S: S s (a multiple of 16, or less
+                    // than 16 - z within the aligned 16 of S B >= 16 or S B < 16 values)
+                    if constexpr (LAYOUT == kLdsPad) u[s] = lds[Lds<kLdsPad>::step(from, S * s)];
+                    else u[s] = lds[Lds<LAYOUT>::idx(base + S * s)];
+                }
                 if constexpr (TWSRC == kTwPowers) {
-                    apply_twiddle_powers<B, DIR>(u, (HOIST_TW ? tw : opaque(tw))[G::powoff(q) + g]);
+                    const float2 *w = (HOIST_TW ? tw : opaque(tw)) + G::powoff(q) + g;
+                    dft_twiddled<B, DIR>(u, w, w + G::powsum);
                 } else {
                     const float2 *twq = (HOIST_TW ? tw : opaque(tw)) + G::twoff(q) + g;
 #pragma unroll
                     for (int s = 1; s < B; ++s) u[s] = ctw<DIR>(u[s], twq[(s - 1) * Aq]);
+                    Dft<B, DIR>::run(u);
                 }
-                Dft<B, DIR>::run(u);
 #pragma unroll
                 for (int h = 0; h < B; ++h) v[b + NB * h] = u[h];
             });

@@ -5,8 +5,8 @@
 // * compile-time twiddle constants W_R^k = exp(DIR * 2 pi i k / R), evaluated in double
 //   by constexpr series and rounded once to float (the reference printed them with six
 //   significant digits, KernelGenerator.h:60-66; here they are correctly rounded);
-// * register-resident DFTs of size 2..64 (natural order in and out) built from radix-4
-//   and radix-2 decimation-in-time steps with the constant twiddles folded in.  They
+// * register-resident DFTs of size 2..32 (natural order in and out), plain or with their
+//   inputs' twiddles folded into the butterflies.  They
 //   play the role of OpenCLFFTAlgorithm::generateLocalFFTKernel (OpenCLFFTAlgorithm.h:14-43)
 //   and of the +-1/+-i shortcuts of KomplexConstMultiplication (KernelGenerator.h:100-142),
 //   as C++ templates instead of generated OpenCL strings.
@@ -207,67 +207,105 @@ struct StaticFor {
 };
 
 // ---------------------------------------------------------------- register DFTs
-// In-place DFT of R elements x[0..R) (natural order), sign DIR, unnormalised.
-template <int R, int DIR>
-struct Dft;
+// Transforms of R <= 32 values in registers, natural order in and out, unnormalised, as
+// radix-2 decimation in time.  A butterfly with twiddle w is six fused multiply-adds,
+// a' = a + w b (two per component) and 2 a - a': with 3 log2 R instructions per value,
+// twiddles included, fewer than higher radices with their products apart (a twiddled
+// 16-point transform: 217 instructions with its twiddles' generation; as radix 4 after
+// 15 products by powers of w: 276).
 
-template <int DIR>
-struct Dft<1, DIR> {
-    static __device__ __forceinline__ void run(float2 *) {}
-};
+// a + w b and a - w b; w as tabulated for the forward direction (DIR > 0 takes its
+// conjugate), a quarter turn further with ROT.
+template <int DIR, bool ROT>
+__device__ __forceinline__ void butterfly(float2 a, float2 b, float2 w, float2 &sum, float2 &diff) {
+    // the twiddle's real part c, and s: w = c + i s
+    const float c = ROT ? (DIR < 0 ? w.y : w.y) : w.x;
+    const float s = ROT ? (DIR < 0 ? -w.x : w.x) : (DIR < 0 ? w.y : -w.y);
+    const float2 t = make_float2(fmaf(-s, b.y, fmaf(c, b.x, a.x)), fmaf(s, b.x, fmaf(c, b.y, a.y)));
+    sum = t;
+    diff = make_float2(fmaf(2.0f, a.x, -t.x), fmaf(2.0f, a.y, -t.y));
+}
 
-template <int DIR>
-struct Dft<2, DIR> {
-    static __device__ __forceinline__ void run(float2 *x) {
-        float2 a = x[0], b = x[1];
-        x[0] = cadd(a, b);
-        x[1] = csub(a, b);
+// The twiddles of a DFT of R values weighted by w^i: on the level that joins transforms of
+// r / 2 to r, w^(R/r) W_r^k for k < r / 4 (the next r / 4 are a quarter turn further), at
+// r / 4 + k; for r = 2 at 0.
+template <int R>
+struct LevelTw {
+    static constexpr int count = R > 4 ? R / 2 : R == 4 ? 2 : 1;
+    float2 t[count];
+    // from p[l] = w^(2^l), l < log2 R
+    __device__ __forceinline__ explicit LevelTw(const float2 *p) {
+        constexpr int LR = __builtin_ctz(R);
+        t[0] = p[LR - 1];
+        StaticFor<2, LR + 1>::run([&](auto lc) {
+            constexpr int l = decltype(lc)::value, r = 1 << l;
+            StaticFor<0, r / 4>::run([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                t[r / 4 + k] = twc<k, r, -1>(p[LR - l]);
+            });
+        });
     }
 };
 
-template <int DIR>
-struct Dft<4, DIR> {
-    static __device__ __forceinline__ void run(float2 *x) {
-        float2 a0 = cadd(x[0], x[2]), a1 = csub(x[0], x[2]);
-        float2 a2 = cadd(x[1], x[3]), a3 = twc<1, 4, DIR>(csub(x[1], x[3]));
-        x[0] = cadd(a0, a2);
-        x[2] = csub(a0, a2);
-        x[1] = cadd(a1, a3);
-        x[3] = csub(a1, a3);
+template <int R, int DIR, bool TW>
+__device__ __forceinline__ void dft_dit(float2 (&x)[R], const float2 *tw) {
+    static_assert(R >= 1 && (R & (R - 1)) == 0, "radix must be a power of two");
+    if constexpr (R > 1) {
+        float2 e[R / 2], o[R / 2];
+        StaticFor<0, R / 2>::run([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            e[i] = x[2 * i];
+            o[i] = x[2 * i + 1];
+        });
+        dft_dit<R / 2, DIR, TW>(e, tw);
+        dft_dit<R / 2, DIR, TW>(o, tw);
+        StaticFor<0, R / 2>::run([&](auto kc) {
+            constexpr int k = decltype(kc)::value;
+            if constexpr (TW) {
+                constexpr bool rot = R >= 4 && k >= R / 4;
+                butterfly<DIR, rot>(e[k], o[k], tw[R / 4 + (rot ? k - R / 4 : k)], x[k], x[k + R / 2]);
+            } else if constexpr ((4 * k) % R == 0) {
+                const float2 b = twc<k, R, DIR>(o[k]);
+                x[k] = cadd(e[k], b);
+                x[k + R / 2] = csub(e[k], b);
+            } else {
+                constexpr float c = float(ct::cos2pi(k, R)), s = -float(ct::sin2pi(k, R));
+                butterfly<DIR, false>(e[k], o[k], make_float2(c, s), x[k], x[k + R / 2]);
+            }
+        });
     }
-};
+}
 
-// R = 4 M (R >= 8): y_r[m] = x[4 m + r], Y_r = DFT_M(y_r),
-// X[k + M q] = sum_r W_R^{r k} Y_r[k] W_4^{r q}.
+// In-place DFT of x[0..R), sign DIR.
 template <int R, int DIR>
 struct Dft {
-    static_assert(R >= 8 && (R & (R - 1)) == 0, "radix must be a power of two");
-    static constexpr int M = R / 4;
     static __device__ __forceinline__ void run(float2 *x) {
-        float2 y[4][M];
-        StaticFor<0, 4>::run([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            StaticFor<0, M>::run([&](auto mc) {
-                constexpr int m = decltype(mc)::value;
-                y[r][m] = x[4 * m + r];
-            });
-            Dft<M, DIR>::run(y[r]);
-        });
-        StaticFor<0, M>::run([&](auto kc) {
-            constexpr int k = decltype(kc)::value;
-            float2 a0 = y[0][k];
-            float2 a1 = twc<k, R, DIR>(y[1][k]);
-            float2 a2 = twc<2 * k, R, DIR>(y[2][k]);
-            float2 a3 = twc<3 * k, R, DIR>(y[3][k]);
-            float2 b0 = cadd(a0, a2), b1 = csub(a0, a2);
-            float2 b2 = cadd(a1, a3), b3 = twc<1, 4, DIR>(csub(a1, a3));
-            x[k] = cadd(b0, b2);
-            x[k + 2 * M] = csub(b0, b2);
-            x[k + M] = cadd(b1, b3);
-            x[k + 3 * M] = csub(b1, b3);
-        });
+        float2 y[R];
+        StaticFor<0, R>::run([&](auto ic) { y[decltype(ic)::value] = x[decltype(ic)::value]; });
+        dft_dit<R, DIR, false>(y, nullptr);
+        StaticFor<0, R>::run([&](auto ic) { x[decltype(ic)::value] = y[decltype(ic)::value]; });
     }
 };
+
+__device__ __forceinline__ float2 csquare(float2 a) {
+    return make_float2(fmaf(a.x, a.x, -a.y * a.y), 2.0f * a.x * a.y);
+}
+
+// In-place DFT of x_i w^i (conj(w)^i for DIR > 0), R <= 16, with w^4 given too (read only
+// for R >= 8): w^2 and w^8 are then one squaring away from a rounded value, and the
+// twiddles' error stays below that of products of powers of w alone.
+template <int R, int DIR>
+__device__ __forceinline__ void dft_twiddled(float2 (&x)[R], const float2 *__restrict__ w1, const float2 *__restrict__ w4) {
+    constexpr int LR = __builtin_ctz(R);
+    static_assert(LR >= 1 && LR <= 4, "radix 2 to 16");
+    float2 p[4];
+    p[0] = *w1;
+    if constexpr (LR > 1) p[1] = csquare(p[0]);
+    if constexpr (LR > 2) p[2] = *w4;
+    if constexpr (LR > 3) p[3] = csquare(p[2]);
+    const LevelTw<R> tw(p);
+    dft_dit<R, DIR, true>(x, tw.t);
+}
 
 // ---------------------------------------------------------------- synthetic data
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {

@@ -63,43 +63,53 @@ __device__ __forceinline__ void exchange_sync() {
     else __syncthreads();
 }
 
-// Twiddle roots of a transform (wave_table): w, w^4 and w^16 of w = W_N^t for t in [0, T),
-// three arrays of T values, then of w = W_T^t' for t' in [0, Q), each value correctly
-// rounded.
+// Twiddles go to the inputs of each step, as powers of one root per transform, which
+// dft_dit folds into its butterflies: before the second step value i' of row k1 has
+// W_N^{t k1} = W_N^{t' k1} (W_1024^{k1})^{i'}, and the first factor waits for the third,
+// where value t' of (k1, k2) has (W_N^{k1 + 32 k2})^{t'}; backwards, the roots are W_T^{t'}
+// (powers k2) and W_N^t (powers k1).  The roots' table (wave_table), each value correctly
+// rounded, with the fourth and sixteenth powers beside the roots so that no power is
+// squared twice:
+//   row:   W_1024^{e k1}, k1 < 32, for e = 1, 4, 16
+//   bin:   W_N^{e (k1 + 32 k2)} at (k2 mod 32 / Q) T + thread, for e = 1, 4
+//   pos:   W_T^{e t'}, t' < Q, for e = 1, 4, 16
+//   point: W_N^{e t}, t < T, for e = 1, 4, 16
 template <int LOG2N>
 struct WaveRoots {
-    static constexpr int first = 0, second = 3 * WaveGeom<LOG2N>::T;
-    static constexpr int size = 3 * (WaveGeom<LOG2N>::T + WaveGeom<LOG2N>::Q);
+    static constexpr int row = 0, bin = 96, pos = bin + 2048, point = pos + 3 * WaveGeom<LOG2N>::Q;
+    static constexpr int size = point + 3 * WaveGeom<LOG2N>::T;
 };
 
-// v[k] *= w^k (its conjugate for DIR > 0) for k in [0, 32), with w, w^4, w^16 read from
-// `roots` at a stride of STRIDE: k = a + 4 b + 16 c, each factor at most two products from
-// a rounded root, and the roots' errors grow by 3 + 3 + 1 at most (by 31 as powers of w
-// alone, which a 32-point step at full length shows in the result).
+// In-place DFT of v[i] w^i (conjugated for DIR > 0), i < 32; w, w^4, w^16 at roots[t],
+// [STRIDE + t], [2 STRIDE + t].
 template <int DIR, int STRIDE>
-__device__ __forceinline__ void twiddle32(float2 (&v)[32], const float2 *__restrict__ roots, int t) {
-    // read and raised anew at each use: kept from the forward transform for the inverse
-    // the powers would take 60 registers
-    const float2 *p = opaque(roots);
-    float2 lo[4], hi[8];
-    lo[1] = p[t];
-    hi[1] = p[STRIDE + t];
-    hi[4] = p[2 * STRIDE + t];
-    lo[2] = cmul(lo[1], lo[1]);
-    lo[3] = cmul(lo[2], lo[1]);
-    hi[2] = cmul(hi[1], hi[1]);
-    hi[3] = cmul(hi[2], hi[1]);
-    StaticFor<5, 8>::run([&](auto ac) { hi[decltype(ac)::value] = cmul(hi[4], hi[decltype(ac)::value - 4]); });
-    StaticFor<0, 8>::run([&](auto ac) {
-        constexpr int a = decltype(ac)::value;
-        if constexpr (a > 0) v[4 * a] = ctw<DIR>(v[4 * a], hi[a]);
-        StaticFor<1, 4>::run([&](auto bc) {
-            constexpr int b = decltype(bc)::value;
-            float2 w = lo[b];
-            if constexpr (a > 0) w = cmul(hi[a], lo[b]);
-            v[4 * a + b] = ctw<DIR>(v[4 * a + b], w);
-        });
-    });
+__device__ __forceinline__ void dft32_rooted(float2 (&v)[32], const float2 *__restrict__ roots, int t) {
+    // read anew at each use: kept from one use to the next their powers would take
+    // tens of registers
+    const float2 *q = opaque(roots);
+    float2 p[5];
+    p[0] = q[t];
+    p[2] = q[STRIDE + t];
+    p[4] = q[2 * STRIDE + t];
+    p[1] = csquare(p[0]);
+    p[3] = csquare(p[2]);
+    const LevelTw<32> tw(p);
+    dft_dit<32, DIR, true>(v, tw.t);
+}
+
+// The same for x[i] w^i, i < Q <= 16; w and w^4 at roots[t] and [1024 + t].
+template <int Q, int DIR>
+__device__ __forceinline__ void dft_rooted(float2 *x, const float2 *__restrict__ roots, int t) {
+    constexpr int LQ = __builtin_ctz(Q);
+    float2 p[4], y[Q];
+    p[0] = roots[t];
+    p[1] = csquare(p[0]);
+    if constexpr (LQ > 2) p[2] = roots[1024 + t];
+    if constexpr (LQ > 3) p[3] = csquare(p[2]);
+    const LevelTw<Q> tw(p);
+    StaticFor<0, Q>::run([&](auto ic) { y[decltype(ic)::value] = x[decltype(ic)::value]; });
+    dft_dit<Q, DIR, true>(y, tw.t);
+    StaticFor<0, Q>::run([&](auto ic) { x[decltype(ic)::value] = y[decltype(ic)::value]; });
 }
 
 // v[i] = x[t + T i] on entry, bin k1 + 32 (m + (32 / Q) t') + 1024 k3 in v[m Q + k3] on exit.
@@ -111,8 +121,8 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
     constexpr int T = G::T, Q = G::Q, RS = G::RS;
     float *row = lds + (t / Q) * RS;
     const int tq = t % Q;
+    using W = WaveRoots<LOG2N>;
     Dft<32, -1>::run(v);
-    twiddle32<-1, T>(v, tw + WaveRoots<LOG2N>::first, t);
     if (lds_busy) exchange_sync<G::in_wave>();
 #pragma unroll
     for (int k = 0; k < 32; ++k) lds[k * RS + t] = v[k].x;
@@ -125,9 +135,8 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
     exchange_sync<G::in_wave>();
 #pragma unroll
     for (int i = 0; i < 32; ++i) v[i].y = row[tq + Q * i];
-    Dft<32, -1>::run(v);
+    dft32_rooted<-1, 32>(v, tw + W::row, t / Q);
     if constexpr (Q > 1) {
-        twiddle32<-1, Q>(v, tw + WaveRoots<LOG2N>::second, tq);
         wave_lds_fence();
 #pragma unroll
         for (int k = 0; k < 32; ++k) row[k * Q + (k * Q >> 5) + tq] = v[k].x;
@@ -140,7 +149,10 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
         wave_lds_fence();
 #pragma unroll
         for (int r = 0; r < 32; ++r) v[r].y = row[33 * tq + r];
-        StaticFor<0, 32 / Q>::run([&](auto mc) { Dft<Q, -1>::run(v + Q * decltype(mc)::value); });
+        StaticFor<0, 32 / Q>::run([&](auto mc) {
+            constexpr int m = decltype(mc)::value;
+            dft_rooted<Q, -1>(v + Q * m, tw + W::bin + T * m, t);
+        });
     }
 }
 
@@ -149,6 +161,7 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
 template <int LOG2N>
 __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, const float2 *__restrict__ tw) {
     using G = WaveGeom<LOG2N>;
+    using W = WaveRoots<LOG2N>;
     constexpr int T = G::T, Q = G::Q, RS = G::RS;
     float *row = lds + (t / Q) * RS;
     const int tq = t % Q;
@@ -166,9 +179,10 @@ __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, co
         wave_lds_fence();
 #pragma unroll
         for (int k = 0; k < 32; ++k) v[k].y = row[k * Q + (k * Q >> 5) + tq];
-        twiddle32<+1, Q>(v, tw + WaveRoots<LOG2N>::second, tq);
+        dft32_rooted<+1, Q>(v, tw + W::pos, tq);
+    } else {
+        Dft<32, +1>::run(v);
     }
-    Dft<32, +1>::run(v);
     wave_lds_fence();
 #pragma unroll
     for (int i = 0; i < 32; ++i) row[tq + Q * i] = v[i].x;
@@ -181,8 +195,7 @@ __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, co
     exchange_sync<G::in_wave>();
 #pragma unroll
     for (int k = 0; k < 32; ++k) v[k].y = lds[k * RS + t];
-    twiddle32<+1, T>(v, tw + WaveRoots<LOG2N>::first, t);
-    Dft<32, +1>::run(v);
+    dft32_rooted<+1, T>(v, tw + W::point, t);
 }
 
 }  // namespace estl

@@ -22,6 +22,8 @@ namespace estl {
 // ------------------------------------------------------------------ twiddles
 // mode 0 (per-pass layout of BlockGeom): entry e -> s = e / A + 1, g = e % A, m = g*s
 // mode 1 (linear): entry e -> m = e * mult
+// mode 2 (the bin roots of WaveRoots, Q = A): entry e = r T + u, T = 32 Q ->
+//         m = mult * bin, bin = u / Q + 32 (r + (32 / Q) (u mod Q))
 // value = exp(-2 pi i m / nq), computed as sincospi(2 m / nq) in double.
 __global__ void k_twiddle(float2 *__restrict__ dst, long count, int mode, long A, long mult, long nq) {
     long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -30,6 +32,9 @@ __global__ void k_twiddle(float2 *__restrict__ dst, long count, int mode, long A
     if (mode == 0) {
         long s = e / A + 1, g = e % A;
         m = (g * s) % nq;
+    } else if (mode == 2) {
+        const long r = e / (32 * A), u = e % (32 * A);
+        m = (u / A + 32 * (r + 32 / A * (u % A))) * mult % nq;
     } else {
         m = (e * mult) % nq;
     }
@@ -98,8 +103,9 @@ hipError_t launch_stream_copy(const void *src, void *dst, long n16, bool nontemp
 // whole transform in registers and padded LDS, one HBM read and one HBM write per
 // value, nontemporal loads and stores.  A partial last group computes its missing rows
 // on a copy of the last row and stores nothing for them.  With twiddles by powers
-// (kRowsTw) the kernel holds 68 VGPRs at 4096 points and 75 at 8192, so LDS alone
-// bounds residency (four 34 KiB groups per CU; two 8192-point rows).  Measured against
+// (kRowsTw) the kernel holds 58 VGPRs at 4096 and 8192 points, so LDS alone bounds
+// residency (four 34 KiB groups per CU; two 8192-point rows), and it runs at the copy's
+// rate: 4096 x 16384 in 167-175 us between devices, 6.1-6.4 TB/s of the copy's 6.55.  Measured against
 // the earlier persistent grid (four resident rounds of workgroups, the next group
 // prefetched into registers; at 4096 and 8192 points the block table's twiddles held in
 // registers across rows, 167 / 206 VGPRs): 6.5 % faster at 4096 x 16384 and 9 % at
