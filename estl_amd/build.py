@@ -28,6 +28,8 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
 SOURCES = [("kernels.hip", [], "kernels"),
            ("pass.hip", ["-DESTL_PASS_DIR=-1"], "pass_fwd"),
            ("pass.hip", ["-DESTL_PASS_DIR=+1"], "pass_bwd"),
+           ("pass_wide.hip", ["-DESTL_PASS_DIR=-1"], "pass_wide_fwd"),
+           ("pass_wide.hip", ["-DESTL_PASS_DIR=+1"], "pass_wide_bwd"),
            ("workqueue.hip", [], "workqueue"),
            ("fp16.hip", [], "fp16"),
            ("conv.hip", [], "conv"),

@@ -77,6 +77,24 @@ bool spectrum_skips_first_pass(const Plan &spec, long k, long shift) {
     return k <= (spec.n >> spec.steps.front().log2b);
 }
 
+// The passes of a convolution's plan, with the radices of conv_pass_split, in k_fft_pass:
+// its input and output modes are that kernel's, and a row has to come out the same to the
+// last bit whatever runs beside it.
+static int build_conv_plan(Plan *p, long n, long batch, int dir, int precision, const std::vector<int> *split = nullptr) {
+    int log2n = 0;
+    while ((1L << log2n) < n) ++log2n;
+    std::vector<int> bits;
+    if (split) bits = *split;
+    else if (log2n > kMaxRowsLog2) bits = conv_pass_split(log2n);
+    if (int rc = build_plan(p, n, batch, dir, precision, 0, bits.empty() ? nullptr : &bits)) return rc;
+    for (PassStep &s : p->steps) {
+        s.args.wide = 0;
+        s.log2t = default_pass_tile(s.log2b, log2n - s.log2b, batch * (n >> s.log2b));
+        s.args.xcd_remap = 0;
+    }
+    return ESTL_OK;
+}
+
 // The passes of a spectrum plan over the filter(s) given by `taps` (rin, fk, fshift, or a
 // group descriptor): the first reads the taps (io_in = 3), or, when `skip`, the second
 // does (io_in = 4); with `divide_l1` the last stores each group member's spectrum
@@ -107,7 +125,7 @@ static int spectrum_passes(const Plan &plan, const PassArgs &taps, bool skip, bo
 }
 
 int group_spectrum_plan(Plan *p, long n, long filters) {
-    int rc = build_plan(p, n, filters, ESTL_FORWARD, ESTL_PRECISION_FP32, 0, nullptr);
+    int rc = build_conv_plan(p, n, filters, ESTL_FORWARD, ESTL_PRECISION_FP32);
     if (rc) return rc;
     if (p->kind != Plan::PASSES) return set_error(ESTL_ERR_UNSUPPORTED, "group spectra need a multi-pass size");
     PassStep &s0 = p->steps.front();
@@ -134,7 +152,7 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
     while ((1L << c->log2n) < n) ++c->log2n;
     c->scale = 1.0f / (float)n;
     c->spec_bytes = sizeof(float2) * (size_t)(h ? n + 1 : n);
-    int rc = build_plan(&c->spec_plan, n, 1, ESTL_FORWARD, ESTL_PRECISION_FP32, 0, nullptr);
+    int rc = build_conv_plan(&c->spec_plan, n, 1, ESTL_FORWARD, ESTL_PRECISION_FP32);
     if (rc) return rc;
     if (c->spec_plan.kind == Plan::PASSES) {
         // the first pass builds the filter from its taps through its direct load path
@@ -166,11 +184,11 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
     // FP16 storage: every pass stores 1/sqrt(radix) of its result, so the forward and
     // inverse passes together scale by exactly 1/n
     Plan f, b;
-    rc = build_plan(&f, n, c->pairs, ESTL_FORWARD, precision, 0, nullptr);
+    rc = build_conv_plan(&f, n, c->pairs, ESTL_FORWARD, precision);
     if (rc) return rc;
     std::vector<int> rev;
     for (auto it = f.steps.rbegin(); it != f.steps.rend(); ++it) rev.push_back(it->log2b);
-    rc = build_plan(&b, n, c->pairs, ESTL_BACKWARD, precision, 0, &rev);
+    rc = build_conv_plan(&b, n, c->pairs, ESTL_BACKWARD, precision, &rev);
     if (rc) return rc;
     const size_t P = f.steps.size();
     if (P < 2 || b.steps.size() != P) return set_error(ESTL_ERR_UNSUPPORTED, "convolution of n=%ld needs >= 2 passes", n);
@@ -195,9 +213,9 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
     c->scratch_bytes = (h ? 4 : sizeof(float2)) * (size_t)n * (size_t)c->pairs;
     if (conv_half_path(n, rows, precision)) {
         // the half-length transforms (their scratch, n/2 values, fits the pair's)
-        rc = build_plan(&c->half_fwd, n / 2, 1, ESTL_FORWARD, ESTL_PRECISION_FP32, 0, nullptr);
+        rc = build_conv_plan(&c->half_fwd, n / 2, 1, ESTL_FORWARD, ESTL_PRECISION_FP32);
         if (rc) return rc;
-        rc = build_plan(&c->half_inv, n / 2, 1, ESTL_BACKWARD, ESTL_PRECISION_FP32, 0, nullptr);
+        rc = build_conv_plan(&c->half_inv, n / 2, 1, ESTL_BACKWARD, ESTL_PRECISION_FP32);
         if (rc) return rc;
         c->half = true;
     }
@@ -412,16 +430,20 @@ int conv_run_group_half(const Plan &fwd, const Plan &inv, const ConvGroup *d_gro
         return set_error(ESTL_ERR_INVALID, "not a half-length group plan pair for n=%ld", n);
     if (members < 1 || members > kGroupMax || !z || !ws) return set_error(ESTL_ERR_INVALID, "bad request group");
     const int P = (int)fwd.steps.size();
+    auto tile = [&](const PassStep &s) {
+        return default_pass_tile(s.log2b, fwd.log2n - s.log2b, (long)members << (fwd.log2n - s.log2b));
+    };
     const float2 *src = nullptr;  // the first pass reads the members' rows
     for (int q = 0; q < P; ++q) {
         PassArgs a = fwd.steps[q].args;
         a.batch = members;
+        a.wide = a.xcd_remap = 0;  // as the request alone (build_conv_plan)
         if (q == 0) {
             a.io_in = 5;
             a.group = d_group;
         }
         float2 *dst = ((P - 1 - q) & 1) ? ws : z;
-        hipError_t e = launch_pass(fwd.steps[q].log2b, fwd.steps[q].log2t, ESTL_FORWARD, src, dst, a, st);
+        hipError_t e = launch_pass(fwd.steps[q].log2b, tile(fwd.steps[q]), ESTL_FORWARD, src, dst, a, st);
         if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group half-length forward pass: %s", hipGetErrorString(e));
         src = dst;
     }
@@ -431,13 +453,14 @@ int conv_run_group_half(const Plan &fwd, const Plan &inv, const ConvGroup *d_gro
     for (int q = 0; q < P; ++q) {
         PassArgs a = inv.steps[q].args;
         a.batch = members;
+        a.wide = a.xcd_remap = 0;
         float2 *dst = (q & 1) ? z : ws;
         if (q == P - 1) {
             a.io_out = 3;
             a.group = d_group;
             dst = nullptr;  // the last pass writes the members' outputs
         }
-        e = launch_pass(inv.steps[q].log2b, inv.steps[q].log2t, ESTL_BACKWARD, src, dst, a, st);
+        e = launch_pass(inv.steps[q].log2b, tile(inv.steps[q]), ESTL_BACKWARD, src, dst, a, st);
         if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group half-length inverse pass: %s", hipGetErrorString(e));
         src = dst;
     }

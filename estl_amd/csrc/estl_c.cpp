@@ -11,6 +11,7 @@
 //                 A_q / N_q prefix products (computeParameters, OpenCLFFTAlgorithm.h:9-12).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <cstdio>
@@ -198,29 +199,90 @@ static int ilog2(long n) {
     return l;
 }
 
-// Split log2n into passes of at most 9 bits, as evenly as possible, smaller radices
-// first (a 512-point radix still leaves room for a 16-column tile in 64 KiB of LDS;
-// measured on MI355X, the first pass -- the one without pre-twiddles -- is the
-// cheapest place for the smaller radix).
-std::vector<int> default_pass_split(int log2n) {
-    int P = (log2n + 8) / 9;
-    if (P < 2) P = 2;
-    std::vector<int> bits(P, log2n / P);
-    for (int i = 0; i < log2n % P; ++i) bits[P - 1 - i]++;
-    return bits;
-}
-
 // Columns per workgroup for a pass of radix 2^log2b over `cols` columns in total:
 // as wide as a 2^13-value tile (64 KiB of LDS) allows (wider tiles mean longer
 // contiguous runs per load and store), capped at 64, narrowed while that leaves fewer
-// than 512 tiles to spread over the CUs (small problems are latency-bound).
+// than 512 tiles to spread over the CUs (small problems are latency-bound), to 8: narrower
+// ones share their 128-byte lines three ways and more (2^18 x 4: 22.4 us with 4 columns,
+// 13.6 with 8).  Tiles of radices above 2^11 hold 2^14 values, not to be narrower still.
 int default_pass_tile(int log2b, int log2cpr, long total_cols) {
-    int lt = 13 - log2b;
+    int lt = (log2b > 10 ? 14 : 13) - log2b;
     if (lt > kMaxPassCols) lt = kMaxPassCols;
     if (lt > log2cpr) lt = log2cpr;
     if (lt < 0) lt = 0;
-    while (lt > 2 && (total_cols >> lt) < 512) --lt;
+    while (lt > 3 && (total_cols >> lt) < 512) --lt;
     return lt;
+}
+
+// The tile (log2 columns) k_pass_wide takes a pass of radix 2^log2b in, 0: none.  Measured on
+// MI355X (2^25 values a pass): tiles of 2^13 values (2^14 for radices 2^9 and 2^10, whose 16
+// and 32 columns keep runs of 128 and 256 bytes) at 5.1-5.8 TB/s against 4.5-5.4 in
+// k_fft_pass; 2^12 values are slower than it (4.6-5.1).  FP16 storage halves a run's bytes:
+// radix 2^8 takes 64 columns.  Last passes read P = 2^log2b / 32 contiguous values per
+// column, 32 bytes for radix 2^7 (4.3 TB/s against 5.4), which stays with k_fft_pass, as
+// does 2^6 (5.4 against 5.9).
+static int wide_tile_log2(int log2b, bool last, bool fp16) {
+    switch (log2b) {
+        case 7: return last ? 0 : 6;
+        case 8: return fp16 && !last ? 6 : 5;
+        case 9: return 5;
+        case 10: return 4;
+        default: return 0;
+    }
+}
+
+// Whether k_pass_wide has a pass: a compiled radix and tile, rows at least a tile apart (any
+// pass but a last one) or contiguous (S = 1) and at least a tile of them.
+static bool pass_is_wide(int log2b, int log2t, long A, int log2S) {
+    bool have = false;
+    for (const int bt : {0x76, 0x85, 0x86, 0x94, 0x95, 0xa4}) have |= bt == log2b * 16 + log2t;
+    return have && (log2S >= log2t || (log2S == 0 && (A >> log2t) > 0 && log2b >= 8));
+}
+
+// A pass's tile, unless `tiled` (a caller's), its kernel, and its pre-twiddle tables
+// (two-level, W_{A B}; k_pass_wide reads them in a first pass too).
+int finish_pass(PassStep *s, int device, bool tiled, bool fp16) {
+    PassArgs &a = s->args;
+    const int cpr = a.log2n - s->log2b;
+    const long cols = a.batch << cpr;
+    if (!tiled) {
+        s->log2t = default_pass_tile(s->log2b, cpr, cols);
+        // wide tiles as long as every CU has two, or the radix has no other FP16 kernel
+        const int w = wide_tile_log2(s->log2b, a.A > 1 && a.log2S == 0, fp16);
+        for (int lt = w; lt > 0 && lt >= w - 1; --lt)
+            if (pass_is_wide(s->log2b, lt, a.A, a.log2S) && ((cols >> lt) >= 512 || s->log2b == 10)) {
+                s->log2t = lt;
+                break;
+            }
+        a.xcd_remap = s->log2t < 4 ? 1 : 0;
+    }
+    a.wide = pass_is_wide(s->log2b, s->log2t, a.A, a.log2S);
+    if (a.A == 1 && !a.wide) return ESTL_OK;
+    const long nq = a.A << s->log2b;
+    a.lobits = ilog2(nq) <= 12 ? ilog2(nq) : (ilog2(nq) + 1) / 2;  // short ones in one level
+    int rc = linear_table(device, 1L << a.lobits, 1, nq, &a.tw_lo);
+    if (!rc) rc = linear_table(device, nq >> a.lobits, 1L << a.lobits, nq, &a.tw_hi);
+    return rc;
+}
+
+// The passes of a plan of `batch` rows.  Up to 2^18 values two passes; 2^19 and 2^20 two of
+// radices 2^9 and 2^10 where k_pass_wide fills the device (2^20 x 33: 300 us in three
+// passes, 210 in two; a single 2^20 is 10 % faster in three), then as few as radices of 2^9
+// allow, evenly split, smaller ones first (a first pass has no pre-twiddles).  A last pass
+// of radix 2^9 reads runs of 16 values per column where smaller ones read 8 or less, which
+// counts where a value is 4 bytes (binary16 2^16 x 300: 75 us as 2^8 2^8, 65 as 2^7 2^9;
+// 2^24 x 2: 178 us as 2^8 2^8 2^8, 165 as 2^7 2^8 2^9) and, in FP32, for rows of 2^15 and 2^16 (2^15 x 1000:
+// 186 -> 177 us).
+static std::vector<int> plan_pass_split(int log2n, long batch, bool fp16) {
+    const long values = batch << log2n;
+    if ((log2n == 19 || log2n == 20) && batch > 1) return {log2n - 10, 10};
+    const int P = std::max(2, (log2n + 8) / 9);
+    const bool last9 = fp16 ? P <= 3 && values >= (1L << 20) : P == 2 && log2n >= 15 && values >= (1L << 23);
+    if (!last9 || (log2n - 9 + P - 2) / (P - 1) > 9) return conv_pass_split(log2n);
+    std::vector<int> bits(P, 9);
+    const int rest = log2n - 9;
+    for (int i = 0; i + 1 < P; ++i) bits[i] = rest / (P - 1) + (i >= P - 1 - rest % (P - 1) ? 1 : 0);
+    return bits;
 }
 
 int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned flags, const std::vector<int> *split,
@@ -259,7 +321,7 @@ int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned fla
         return power_table(p->device, p->log2n, &p->tw_rows);
     }
     p->kind = Plan::PASSES;
-    std::vector<int> bits = (split && !split->empty()) ? *split : default_pass_split(p->log2n);
+    std::vector<int> bits = (split && !split->empty()) ? *split : plan_pass_split(p->log2n, batch, fp16);
     int total = 0;
     const int max_b = fp16 ? max_pass_log2_fp16() : kMaxPassLog2;
     for (int b : bits) {
@@ -280,9 +342,8 @@ int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned fla
         st.args.log2n = p->log2n;
         st.args.log2S = ilog2(n / (A * B));
         st.args.scale = fp16 ? (float)(1.0 / std::sqrt((double)B)) : (q + 1 == bits.size()) ? p->scale : 1.0f;
-        st.log2t = default_pass_tile(bits[q], p->log2n - bits[q], batch * (n / B));
-        st.args.xcd_remap = 0;
-        if (tiles && tiles->size() == bits.size()) {
+        const bool tiled = tiles && tiles->size() == bits.size();
+        if (tiled) {
             const int lt = (*tiles)[q];
             if (lt < 0 || lt > kMaxPassCols || lt + bits[q] > kMaxPassTileLog2 || lt > p->log2n - bits[q])
                 return set_error(ESTL_ERR_UNSUPPORTED, "tile 2^%d invalid for pass radix 2^%d", lt, bits[q]);
@@ -292,15 +353,8 @@ int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned fla
         }
         int rc = power_table(p->device, bits[q], &st.args.tw_local);
         if (rc) return rc;
-        if (A > 1) {
-            const long nq = A * B;
-            const int lnq = ilog2(nq);
-            st.args.lobits = (lnq + 1) / 2;
-            rc = linear_table(p->device, 1L << st.args.lobits, 1, nq, &st.args.tw_lo);
-            if (rc) return rc;
-            rc = linear_table(p->device, nq >> st.args.lobits, 1L << st.args.lobits, nq, &st.args.tw_hi);
-            if (rc) return rc;
-        }
+        rc = finish_pass(&st, p->device, tiled, fp16);
+        if (rc) return rc;
         p->steps.push_back(st);
         A *= B;
     }
@@ -502,6 +556,10 @@ int estl_plan_create_split(estl_plan_t *plan, long n, long batch, int direction,
     if (npasses < 0 || npasses > 16 || (npasses > 0 && !log2radices))
         return set_error(ESTL_ERR_INVALID, "bad pass split");
     std::vector<int> split(log2radices, log2radices + npasses);
+    if (precision == ESTL_PRECISION_FP16)
+        for (int b : split)
+            if (b > kMaxSplitLog2Fp16)
+                return set_error(ESTL_ERR_UNSUPPORTED, "pass radix 2^%d outside [2^4, 2^%d]", b, kMaxSplitLog2Fp16);
     std::vector<int> tiles;
     if (log2tiles && npasses > 0) tiles.assign(log2tiles, log2tiles + npasses);
     Plan *p = new Plan();

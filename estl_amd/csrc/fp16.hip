@@ -230,9 +230,9 @@ k_fft_pass_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, PassArgs a) 
     pass_tile<LOG2B, DIR, LOG2T, MID, f16x2>(in, out, a, tile, lds, false);
 }
 
-// FP16 passes: radices 2^4 .. 2^9 (every split the default planner makes), tiles of at
+// FP16 passes: radices 2^4 .. 2^9 here (2^10 in k_pass_wide only), tiles of at
 // most 2^14 values
-constexpr int kMaxPassLog2Fp16 = 9;
+constexpr int kMaxPassLog2Fp16 = 10;
 
 template <int LOG2B, int DIR, int LOG2T, bool MID>
 static hipError_t launch_pass_h_t(const f16x2 *in, f16x2 *out, const PassArgs &a, hipStream_t st) {
@@ -278,6 +278,7 @@ static hipError_t launch_pass_h_d(int log2b, int log2t, const f16x2 *in, f16x2 *
 
 hipError_t launch_pass_fp16(int log2b, int log2t, int dir, const void *in16, void *out16, const PassArgs &a,
                             hipStream_t st) {
+    if (a.wide) return launch_pass_wide(log2b, log2t, dir, true, in16, out16, a, st);
     const f16x2 *in = static_cast<const f16x2 *>(in16);
     f16x2 *out = static_cast<f16x2 *>(out16);
     return dir < 0 ? launch_pass_h_d<-1>(log2b, log2t, in, out, a, st) : launch_pass_h_d<+1>(log2b, log2t, in, out, a, st);

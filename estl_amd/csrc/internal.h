@@ -39,6 +39,7 @@ struct PassArgs {
     int log2S;               // S = n / (A_q B_q) = 2^log2S
     int lobits;              // two-level pre-twiddle split: m = (hi << lobits) | lo
     int xcd_remap;           // deal consecutive tiles to the same XCD
+    int wide;                // run by k_pass_wide (complex rows, no io_in or io_out mode)
     float scale;             // applied to the stored values (1 = none)
     const float2 *tw_local;  // power table of the radix-B DFT (block_fft kTwPowers)
     const float2 *tw_lo;     // W_{A B}^{lo}, lo < 2^lobits
@@ -83,6 +84,17 @@ long co_resident_blocks(const void *kernel, int block_threads);
 // rows kernel on the tile-planarized layout (kernels.hip)
 hipError_t launch_rows_planar(int log2n, int dir, const float2 *in, float2 *out, long batch, const float2 *tw,
                               float scale, hipStream_t st);
+// pass_wide.hip: passes with args.wide set (pass_is_wide says which radices, tiles and
+// strides it has); buffers of float2, or of binary16 pairs with fp16
+hipError_t launch_pass_wide_fwd(int log2b, int log2t, bool fp16, const void *in, void *out, const PassArgs &a,
+                                hipStream_t st);
+hipError_t launch_pass_wide_bwd(int log2b, int log2t, bool fp16, const void *in, void *out, const PassArgs &a,
+                                hipStream_t st);
+inline hipError_t launch_pass_wide(int log2b, int log2t, int dir, bool fp16, const void *in, void *out,
+                                   const PassArgs &a, hipStream_t st) {
+    return dir < 0 ? launch_pass_wide_fwd(log2b, log2t, fp16, in, out, a, st)
+                   : launch_pass_wide_bwd(log2b, log2t, fp16, in, out, a, st);
+}
 hipError_t launch_pass_fwd(int log2b, int log2t, const float2 *in, float2 *out, const PassArgs &a, hipStream_t st);
 hipError_t launch_pass_bwd(int log2b, int log2t, const float2 *in, float2 *out, const PassArgs &a, hipStream_t st);
 // FP16 storage (fp16.hip): buffers of (re, im) binary16 pairs, passed untyped
@@ -100,6 +112,7 @@ int max_pass_log2_fp16();
 hipError_t launch_pass_mid(int log2b, int log2t, const float2 *in, float2 *out, const PassArgs &a, hipStream_t st);
 inline hipError_t launch_pass(int log2b, int log2t, int dir, const float2 *in, float2 *out, const PassArgs &a,
                               hipStream_t st) {
+    if (a.wide) return launch_pass_wide(log2b, log2t, dir, false, in, out, a, st);
     return dir < 0 ? launch_pass_fwd(log2b, log2t, in, out, a, st) : launch_pass_bwd(log2b, log2t, in, out, a, st);
 }
 hipError_t launch_twiddle(float2 *dst, long count, int mode, long A, long mult, long nq, hipStream_t st);
@@ -115,6 +128,7 @@ int rows_pass_count(int log2n);
 constexpr int kMaxRowsLog2 = 13;   // largest single-launch row length
 constexpr int kSpecBlockTwLog2 = 12;  // filter spectra of at least 2^12 points read the block table
 constexpr int kMaxPassLog2 = 13;   // largest radix of a global pass
+constexpr int kMaxSplitLog2Fp16 = 9;  // largest radix of an FP16 pass that a caller can ask for
 constexpr int kMaxPassTileLog2 = 14;  // a pass tile holds at most 2^14 values (~139 KiB of LDS)
 constexpr int kMaxPassCols = 6;    // at most 2^6 columns per tile
 // convolutions of 2^10 values and more (k_conv_wave, k_conv_ols) keep 32 values per thread

@@ -75,7 +75,22 @@ int block_table(int device, int log2n, const float2 **out);
 int power_table(int device, int log2n, const float2 **out);  // block_fft's kTwPowers table
 int wave_table(int device, int log2n, const float2 **out);   // fft_wave.h's roots, log2n = 10..14
 int linear_table(int device, long count, long mult, long nq, const float2 **out);
-std::vector<int> default_pass_split(int log2n);
+// Split log2n into passes of at most 9 bits, as evenly as possible, smaller radices first
+// (a 512-point radix still leaves room for a 16-column tile in 64 KiB of LDS; the first
+// pass -- the one without pre-twiddles -- is the cheapest place for the smaller radix).
+// The convolutions' passes take it for every number of rows: a request group's rows are
+// computed by the same radices as a request's alone.
+inline std::vector<int> conv_pass_split(int log2n) {
+    int P = (log2n + 8) / 9;
+    if (P < 2) P = 2;
+    std::vector<int> bits(P, log2n / P);
+    for (int i = 0; i < log2n % P; ++i) bits[P - 1 - i]++;
+    return bits;
+}
+// columns per workgroup (log2) of k_fft_pass (estl_c.cpp)
+int default_pass_tile(int log2b, int log2cpr, long total_cols);
+// a pass's tile (unless `tiled`), kernel (args.wide) and pre-twiddle tables
+int finish_pass(PassStep *s, int device, bool tiled, bool fp16);
 int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned flags, const std::vector<int> *split,
                const std::vector<int> *tiles = nullptr);
 int execute_plan(Plan *p, const float2 *in, float2 *out, hipStream_t st);

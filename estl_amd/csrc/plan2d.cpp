@@ -22,8 +22,6 @@
 
 namespace estl {
 
-int default_pass_tile(int log2b, int log2cpr, long total_cols);
-
 struct Plan2D {
     long nx = 0, ny = 0, batch = 0;
     int dir = ESTL_FORWARD;
@@ -85,7 +83,7 @@ static int build_plan2d(Plan2D *p, long nx, long ny, long batch, int dir, unsign
             s.args.batch = batch;
             s.args.xcd_remap = 0;
             s.args.scale = (q + 1 == p->cols.steps.size()) ? scale : 1.0f;
-            s.log2t = default_pass_tile(s.log2b, s.args.log2n - s.log2b, batch * ((nx * ny) >> s.log2b));
+            if ((rc = finish_pass(&s, p->cols.device, false, false))) return rc;
         }
         p->cols.n = nx * ny;
         p->cols.batch = batch;

@@ -515,7 +515,10 @@ class Server {
         auto it = half_plans_.find(key);
         if (it != half_plans_.end()) return it->second.get();
         std::unique_ptr<Plan> p(new Plan());
-        if (build_plan(p.get(), m, batch, dir, ESTL_PRECISION_FP32, 0, nullptr)) return nullptr;
+        int log2m = 0;
+        while ((1L << log2m) < m) ++log2m;
+        const std::vector<int> split = conv_pass_split(log2m);  // as the request alone
+        if (build_plan(p.get(), m, batch, dir, ESTL_PRECISION_FP32, 0, &split)) return nullptr;
         if (p->kind != Plan::PASSES) return nullptr;
         Plan *raw = p.get();
         half_plans_[key] = std::move(p);

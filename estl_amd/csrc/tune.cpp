@@ -145,18 +145,19 @@ std::vector<Choice> candidates(int log2n, int max_b) {
 
 }  // namespace
 
-int default_pass_tile(int log2b, int log2cpr, long total_cols);
-
 int execute_plan_fp16(Plan *p, const void *in, const float *in_scale, void *out, float *out_scale, hipStream_t st);
 
 // Time one candidate: median-free minimum of `reps` runs after a warm-up.  FP16
 // candidates run through the FP16 entry point (`scales`: two arrays of batch floats).
-static int time_candidate(const Choice &c, long n, long batch, int dir, int precision, float2 *in, float2 *out,
+// A candidate without tiles takes on those the plan chose.
+static int time_candidate(Choice &c, long n, long batch, int dir, int precision, float2 *in, float2 *out,
                           float *scales, hipStream_t st, hipEvent_t e0, hipEvent_t e1, double *us) {
     Plan p;
     int rc = build_plan(&p, n, batch, dir, precision, 0, c.rows ? nullptr : &c.split,
                         c.tiles.empty() ? nullptr : &c.tiles);
     if (rc) return rc;
+    if (!c.rows && c.tiles.empty())
+        for (const PassStep &s : p.steps) c.tiles.push_back(s.log2t);
     double best = 1e30;
     const int reps = 4;
     for (int r = 0; r < reps + 1; ++r) {
@@ -240,11 +241,6 @@ int tune_plan(long n, long batch, int dir, int precision, bool *rows, std::vecto
         rc = time_candidate(c, n, batch, dir, precision, in, out, scales, st, e0, e1, &us);
         if (rc) continue;  // a split without kernels for this size: skip it
         c.us = us;
-        if (!c.rows) {
-            // record the tile widths the plan used
-            c.tiles.clear();
-            for (int b : c.split) c.tiles.push_back(default_pass_tile(b, log2n - b, batch * (n >> b)));
-        }
         char buf[256];
         std::string s = c.rows ? "\"rows\"" : "[";
         if (!c.rows) {
