@@ -73,17 +73,73 @@ __global__ void __launch_bounds__(256) k_maxabs(const float2 *__restrict__ x, in
 
 // y = x / m_t in FP16; scale[t] = m_t (1 for an all-zero transform).  `scale` holds the
 // atomicMax results (float bits) on entry and is rewritten in place with the same bits.
-__global__ void k_pack(const float2 *__restrict__ x, f16x2 *__restrict__ y, int log2n, long batch,
-                       float *__restrict__ scale) {
+// A workgroup takes 256 kPackU consecutive values, the workgroups from the last to the first:
+// what k_maxabs read last is still in the memory-side cache.
+// Eight values a thread: one each left the launch bound by its workgroups' dispatch
+// (2^18 x 101 with k_maxabs 98 -> 90 us, 2^26 266 -> 248; chunks that both kernels take in turn
+// were slower).
+constexpr int kPackU = 8;
+__global__ void __launch_bounds__(256) k_pack(const float2 *__restrict__ x, f16x2 *__restrict__ y, int log2n,
+                                              long batch, float *__restrict__ scale) {
     const long count = batch << log2n;
-    const long stride = (long)gridDim.x * blockDim.x;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride) {
-        const long t = i >> log2n;
-        const float m = scale[t];
-        const float d = m > 0.0f ? m : 1.0f;
-        const float2 v = ld_stream(x + i);
-        st_elem(y + i, make_float2(v.x / d, v.y / d));
-        if ((i & ((1L << log2n) - 1)) == 0 && !(m > 0.0f)) scale[t] = 1.0f;
+    const long base = (long)(gridDim.x - 1 - blockIdx.x) * (256 * kPackU) + threadIdx.x;
+    float2 v[kPackU];
+    float m[kPackU];
+#pragma unroll
+    for (int u = 0; u < kPackU; ++u) {
+        const long i = base + 256 * u;
+        if (i < count) {
+            v[u] = ld_stream(x + i);
+            m[u] = scale[i >> log2n];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kPackU; ++u) {
+        const long i = base + 256 * u;
+        if (i < count) {
+            const float d = m[u] > 0.0f ? m[u] : 1.0f;
+            st_elem(y + i, make_float2(v[u].x / d, v[u].y / d));
+            if ((i & ((1L << log2n) - 1)) == 0 && !(m[u] > 0.0f)) scale[i >> log2n] = 1.0f;
+        }
+    }
+}
+
+// The two steps above for transforms of 2^8 to 2^14 values in one launch that reads them
+// once: 16 values per thread, TPT = N / 16 threads per transform, the maximum by xor shuffles
+// inside a wave and through LDS across a transform's waves (a maximum is order-free: the
+// scales and values of the separate steps).  HBM-bound, 12 B per value against 20:
+// 2^12 x 5000 80 -> 38 us, one row of 2^10 14 -> 7.
+template <int LOG2N>
+__global__ void __launch_bounds__((BlockGeom<LOG2N>::TPT > 256 ? BlockGeom<LOG2N>::TPT : 256))
+k_pack_rows(const float2 *__restrict__ x, f16x2 *__restrict__ y, long batch, float *__restrict__ scale) {
+    constexpr int N = 1 << LOG2N, TPT = N / 16, NT = TPT > 256 ? TPT : 256, TPW = NT / TPT;
+    constexpr int WAVES = TPT > 64 ? TPT / 64 : 1;
+    __shared__ float wmax[NT / 64];
+    const int t = threadIdx.x, w = t / TPT, tl = t % TPT;
+    const long want = (long)blockIdx.x * TPW + w;
+    const long row = want < batch ? want : batch - 1;
+    const float2 *src = x + row * N + tl;
+    float2 v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = ld_stream(src + TPT * i);
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) m = fmaxf(m, fmaxf(fabsf(v[i].x), fabsf(v[i].y)));
+#pragma unroll
+    for (int off = 1; off < (TPT < 64 ? TPT : 64); off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
+    if constexpr (WAVES > 1) {
+        if ((t & 63) == 0) wmax[t >> 6] = m;
+        __syncthreads();
+        m = wmax[w * WAVES];
+#pragma unroll
+        for (int i = 1; i < WAVES; ++i) m = fmaxf(m, wmax[w * WAVES + i]);
+    }
+    const float d = m > 0.0f ? m : 1.0f;
+    if (want < batch) {
+        if (tl == 0) scale[row] = d;
+        f16x2 *dst = y + row * N + tl;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st_elem(dst + TPT * i, make_float2(v[i].x / d, v[i].y / d));
     }
 }
 
@@ -112,13 +168,28 @@ static unsigned grid_for(long count, long per_block) {
 
 hipError_t launch_pack_fp16(const float2 *x, void *y16, float *scale, int log2n, long batch, hipStream_t st) {
     f16x2 *y = static_cast<f16x2 *>(y16);
+    switch (log2n) {
+#define PACK_CASE(L)                                                                                             \
+    case L: {                                                                                                    \
+        constexpr int TPT = BlockGeom<L>::TPT, NT = TPT > 256 ? TPT : 256;                                       \
+        const long groups = (batch + NT / TPT - 1) / (NT / TPT);                                                 \
+        if (groups > 0x7fffffffL) return hipErrorInvalidValue;                                                   \
+        hipLaunchKernelGGL(k_pack_rows<L>, dim3((unsigned)groups), dim3(NT), 0, st, x, y, batch, scale);         \
+        return hipGetLastError();                                                                                \
+    }
+        PACK_CASE(8) PACK_CASE(9) PACK_CASE(10) PACK_CASE(11) PACK_CASE(12) PACK_CASE(13) PACK_CASE(14)
+#undef PACK_CASE
+        default: break;
+    }
     unsigned *umax = reinterpret_cast<unsigned *>(scale);
     hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(batch, 256)), dim3(256), 0, st, umax, batch);
     const int clog = log2n < kMaxAbsChunkLog2 ? log2n : kMaxAbsChunkLog2;
     const int per_log = clog > 8 ? clog - 8 : 0;
     const long blocks = ((batch << log2n) + (1L << (per_log + 8)) - 1) >> (per_log + 8);
     hipLaunchKernelGGL(k_maxabs, dim3((unsigned)blocks), dim3(256), 0, st, x, log2n, batch, umax);
-    hipLaunchKernelGGL(k_pack, dim3(grid_for(batch << log2n, 256)), dim3(256), 0, st, x, y, log2n, batch, scale);
+    const long pb = ((batch << log2n) + 256 * kPackU - 1) / (256 * kPackU);
+    if (pb > 0x7fffffffL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_pack, dim3((unsigned)pb), dim3(256), 0, st, x, y, log2n, batch, scale);
     return hipGetLastError();
 }
 
@@ -139,7 +210,7 @@ hipError_t launch_scale_mul(const float *in, float *out, float f, long batch, hi
 template <int LOG2N, int DIR, int TPW>
 __global__ void __launch_bounds__(BlockGeom<LOG2N>::TPT * TPW)
 k_fft_rows_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, long batch, const float2 *__restrict__ tw,
-             float scale) {
+             float scale, const float *__restrict__ s_in, float *__restrict__ s_out, float s_factor) {
     using G = BlockGeom<LOG2N>;
     constexpr int N = G::N, E = G::E, TPT = G::TPT;
     constexpr int SLICE = G::uses_lds ? Lds<kLdsPad>::size(N) : 0;
@@ -159,6 +230,7 @@ k_fft_rows_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, long batch, 
         f16x2 *dst = out + row * N + tl;
 #pragma unroll
         for (int i = 0; i < E; ++i) st_elem(dst + TPT * i, cscale(v[i], scale));
+        if (s_out && tl == 0) s_out[row] = s_in[row] * s_factor;
         return;
     }
     const long groups = (batch + TPW - 1) / TPW;
@@ -178,13 +250,14 @@ k_fft_rows_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, long batch, 
             f16x2 *dst = out + row * N + tl;
 #pragma unroll
             for (int i = 0; i < E; ++i) st_elem(dst + TPT * i, cscale(v[i], scale));
+            if (s_out && tl == 0) s_out[row] = s_in[row] * s_factor;
         }
     }
 }
 
 template <int LOG2N, int DIR>
 static hipError_t launch_rows_h_t(const f16x2 *in, f16x2 *out, long batch, const float2 *tw, float scale,
-                                  hipStream_t st) {
+                                  hipStream_t st, const float *s_in, float *s_out, float s_factor) {
     using G = BlockGeom<LOG2N>;
     constexpr int TPW = (G::TPT >= 256) ? 1 : 256 / G::TPT;
     auto kernel = k_fft_rows_h<LOG2N, DIR, TPW>;
@@ -192,16 +265,17 @@ static hipError_t launch_rows_h_t(const f16x2 *in, f16x2 *out, long batch, const
     // 1024 points, 1-3 % at 4096 and 8192)
     const long groups = (batch + TPW - 1) / TPW;
     if (groups > 0x7fffffffL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(G::TPT * TPW), 0, st, in, out, batch, tw, scale);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(G::TPT * TPW), 0, st, in, out, batch, tw, scale, s_in,
+                       s_out, s_factor);
     return hipGetLastError();
 }
 
 template <int DIR>
 static hipError_t launch_rows_h_d(int log2n, const f16x2 *in, f16x2 *out, long batch, const float2 *tw, float scale,
-                                  hipStream_t st) {
+                                  hipStream_t st, const float *s_in, float *s_out, float s_factor) {
     switch (log2n) {
 #define ROWS_H_CASE(L) \
-    case L: return launch_rows_h_t<L, DIR>(in, out, batch, tw, scale, st);
+    case L: return launch_rows_h_t<L, DIR>(in, out, batch, tw, scale, st, s_in, s_out, s_factor);
         ROWS_H_CASE(1) ROWS_H_CASE(2) ROWS_H_CASE(3) ROWS_H_CASE(4) ROWS_H_CASE(5) ROWS_H_CASE(6) ROWS_H_CASE(7)
         ROWS_H_CASE(8) ROWS_H_CASE(9) ROWS_H_CASE(10) ROWS_H_CASE(11) ROWS_H_CASE(12) ROWS_H_CASE(13)
 #undef ROWS_H_CASE
@@ -210,11 +284,11 @@ static hipError_t launch_rows_h_d(int log2n, const f16x2 *in, f16x2 *out, long b
 }
 
 hipError_t launch_rows_fp16(int log2n, int dir, const void *in16, void *out16, long batch, const float2 *tw, float scale,
-                            hipStream_t st) {
+                            hipStream_t st, const float *s_in, float *s_out, float s_factor) {
     const f16x2 *in = static_cast<const f16x2 *>(in16);
     f16x2 *out = static_cast<f16x2 *>(out16);
-    return dir < 0 ? launch_rows_h_d<-1>(log2n, in, out, batch, tw, scale, st)
-                   : launch_rows_h_d<+1>(log2n, in, out, batch, tw, scale, st);
+    return dir < 0 ? launch_rows_h_d<-1>(log2n, in, out, batch, tw, scale, st, s_in, s_out, s_factor)
+                   : launch_rows_h_d<+1>(log2n, in, out, batch, tw, scale, st, s_in, s_out, s_factor);
 }
 
 // ------------------------------------------------------------------ global passes
@@ -227,6 +301,7 @@ k_fft_pass_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, PassArgs a) 
         const long nb = gridDim.x;
         if ((nb & 7) == 0) tile = (tile & 7) * (nb >> 3) + (tile >> 3);
     }
+    row_scale<LOG2B, LOG2T>(a, tile);
     pass_tile<LOG2B, DIR, LOG2T, MID, f16x2>(in, out, a, tile, lds, false);
 }
 

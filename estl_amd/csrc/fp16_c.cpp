@@ -27,9 +27,11 @@ int execute_plan_fp16(Plan *p, const void *in, const float *in_scale, void *out,
     switch (p->kind) {
         case Plan::COPY:
             if (in != out) e = hipMemcpyAsync(out, in, 4 * (size_t)p->batch, hipMemcpyDeviceToDevice, st);
+            if (e == hipSuccess) e = launch_scale_mul(in_scale, out_scale, (float)p->out_factor, p->batch, st);
             break;
         case Plan::ROWS:
-            e = launch_rows_fp16(p->log2n, p->dir, in, out, p->batch, p->tw_rows, p->scale, st);
+            e = launch_rows_fp16(p->log2n, p->dir, in, out, p->batch, p->tw_rows, p->scale, st, in_scale, out_scale,
+                                 (float)p->out_factor);
             break;
         case Plan::PASSES: {
             const int P = (int)p->steps.size();
@@ -45,13 +47,18 @@ int execute_plan_fp16(Plan *p, const void *in, const float *in_scale, void *out,
             }
             const void *src = in;
             for (int q = 0; q < P && e == hipSuccess; ++q) {
-                e = launch_pass_fp16(p->steps[q].log2b, p->steps[q].log2t, p->dir, src, dst[q], p->steps[q].args, st);
+                PassArgs a = p->steps[q].args;
+                if (q == P - 1) {  // the output scales in the same launch
+                    a.s_in = in_scale;
+                    a.s_out = out_scale;
+                    a.s_factor = (float)p->out_factor;
+                }
+                e = launch_pass_fp16(p->steps[q].log2b, p->steps[q].log2t, p->dir, src, dst[q], a, st);
                 src = dst[q];
             }
             break;
         }
     }
-    if (e == hipSuccess) e = launch_scale_mul(in_scale, out_scale, (float)p->out_factor, p->batch, st);
     if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "FP16 transform launch: %s", hipGetErrorString(e));
     return ESTL_OK;
 }

@@ -69,6 +69,9 @@ struct PassArgs {
     void *rout16;
     int planar_in;           // `in` / `out` use the tile-planarized layout (FP32 only)
     int planar_out;
+    const float *s_in;       // FP16 storage, a plan's last pass: the output scales it also
+    float *s_out;            // writes, s_in times s_factor per row (null: none)
+    float s_factor;
     const float2 *spectrum;
     long fk, fshift;         // io_in = 3, 4: taps and rotation of the filter
     // convolution passes of a request group: rows index the group's batch, and the
@@ -101,8 +104,9 @@ hipError_t launch_pass_bwd(int log2b, int log2t, const float2 *in, float2 *out, 
 hipError_t launch_pack_fp16(const float2 *x, void *y16, float *scale, int log2n, long batch, hipStream_t st);
 hipError_t launch_unpack_fp16(const void *y16, const float *scale, float2 *x, int log2n, long batch, hipStream_t st);
 hipError_t launch_scale_mul(const float *in, float *out, float f, long batch, hipStream_t st);
+// (s_out: the output row scales, s_in times s_factor, written by the same launch)
 hipError_t launch_rows_fp16(int log2n, int dir, const void *in16, void *out16, long batch, const float2 *tw, float scale,
-                            hipStream_t st);
+                            hipStream_t st, const float *s_in = nullptr, float *s_out = nullptr, float s_factor = 1.0f);
 hipError_t launch_pass_fp16(int log2b, int log2t, int dir, const void *in16, void *out16, const PassArgs &a,
                             hipStream_t st);
 hipError_t launch_pass_mid_fp16(int log2b, int log2t, const void *in16, void *out16, const PassArgs &a,

@@ -44,6 +44,15 @@ __device__ __forceinline__ int group_member(const ConvGroup *g, long row) {
     return q;
 }
 
+// FP16 storage: the output scale of the row that `tile` is the first of (plans whose last
+// pass carries s_out).
+template <int LOG2B, int LOG2T>
+__device__ __forceinline__ void row_scale(const PassArgs &a, long tile) {
+    const int per = a.log2n - LOG2B - LOG2T;
+    if (a.s_out && threadIdx.x == 0 && (tile & ((1L << per) - 1)) == 0)
+        a.s_out[tile >> per] = a.s_in[tile >> per] * a.s_factor;
+}
+
 // Geometry of tile `tile` for the calling thread: the row, the tile's first column j0,
 // the thread's column j = j0 + c, its g = j / S and z = j mod S, and tl.
 template <int LOG2B, int LOG2T>

@@ -21,6 +21,7 @@
 #pragma once
 
 #include "fft_block.h"
+#include "pass_tile.h"
 #include "internal.h"
 
 namespace estl {

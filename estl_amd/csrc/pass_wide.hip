@@ -12,6 +12,7 @@ template <int LOG2B, int DIR, int LOG2T, int MODE, typename ST>
 __global__ void __launch_bounds__(1 << (LOG2B - 5 + LOG2T)) __attribute__((amdgpu_waves_per_eu(4)))
 k_pass_wide(const ST *__restrict__ in, ST *__restrict__ out, PassArgs a) {
     __shared__ float lds[WideTile<LOG2B, LOG2T, MODE>::lds_floats];
+    if constexpr (!__is_same(ST, float2)) row_scale<LOG2B, LOG2T>(a, blockIdx.x);
     wide_tile<LOG2B, DIR, LOG2T, MODE>(in, out, a, blockIdx.x, lds);
 }
 
