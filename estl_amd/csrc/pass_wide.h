@@ -12,6 +12,8 @@
 // as one product of a two-level table (by squaring, the errors of 2^20 points were 8 %
 // larger).
 //
+// (lds_busy: the slice may still be being read on entry.)
+//
 // A tile is T = 2^LOG2T adjacent columns over P T threads.  Lanes run over columns where
 // the rows of a tile's input lie T values apart in memory (S >= T), and after the exchange
 // always, so every store and these loads move T consecutive values; in a last pass (S = 1)
@@ -47,10 +49,10 @@ __device__ __forceinline__ float2 pass_root(const PassArgs &a, unsigned m) {
 
 template <int LOG2B, int DIR, int LOG2T, int MODE, typename ST>
 __device__ __forceinline__ void wide_tile(const ST *__restrict__ in, ST *__restrict__ out, const PassArgs &a, long tile,
-                                          float *lds) {
+                                          float *lds, bool lds_busy = false) {
     using G = WideTile<LOG2B, LOG2T, MODE>;
     constexpr int P = G::P, T = G::T, LOG2P = LOG2B - 5;
-    const int th = threadIdx.x;
+    const int th = opaque_lane(threadIdx.x);
     const int lcpr = a.log2n - LOG2B;  // columns per row = 2^lcpr
     const long row = tile >> (lcpr - LOG2T);
     const int j0 = int(tile - (row << (lcpr - LOG2T))) << LOG2T;
@@ -95,6 +97,7 @@ __device__ __forceinline__ void wide_tile(const ST *__restrict__ in, ST *__restr
             dft_dit<32, DIR, true>(v, tw.t);
         }
         const int at = c * G::SC + t * G::ST;
+        if (lds_busy) __syncthreads();  // the previous tile's last reads
 #pragma unroll
         for (int k = 0; k < 32; ++k) lds[k * G::RS + at] = v[k].x;
         __syncthreads();

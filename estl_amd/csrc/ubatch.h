@@ -6,14 +6,19 @@
 namespace estl {
 
 // work-queue workgroup size 2^kUThreadsLog2 (see workqueue.hip)
-#ifndef ESTL_UBATCH_TLOG
-#define ESTL_UBATCH_TLOG 9
-#endif
-constexpr int kUThreadsLog2 = ESTL_UBATCH_TLOG;
+constexpr int kUThreadsLog2 = 9;
 constexpr int kUMaxLog2 = 20;  // largest transform of an uneven batch
-// up to here a work item is a group of rows (a large item must fill a workgroup's tile:
-// 2^(kUThreadsLog2 + 4) values)
-constexpr int kUMaxSmallLog2 = kUThreadsLog2 + 3 > 12 ? kUThreadsLog2 + 3 : 12;
+// up to here a work item is a group of rows (16 values per thread)
+constexpr int kUMaxSmallLog2 = kUThreadsLog2 + 4;
+
+// First radix of the large sizes' two passes.  Measured on MI355X (1 GiB of one size per
+// launch): the even split beats skewed ones -- a radix-16 first pass with 256-column tiles
+// and a 2^10..2^12 second pass was 1.7x (L = 14) to 6x (L = 16) slower, a 2^9 second pass
+// 2-20 % slower.
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+constexpr int ubatch_split(int L) { return L / 2; }
 
 // One work item: `count` transforms of size 2^log2n, the `first`-th.. of the
 // size-sorted offset list (count = 1 for large sizes).
@@ -29,6 +34,10 @@ struct UTables {
     // power tables (block_fft kTwPowers) of BlockGeom<log2>, log2 0..kUMaxSmallLog2: the
     // small transforms and the radices of the large ones' passes
     const float2 *pow[kUMaxSmallLog2 + 1];
+    // W_B^m, m < B = 2^log2, of the first passes in k_pass_wide's form, and the one entry
+    // (1) of their second level
+    const float2 *first[kUMaxLog2 / 2 + 1];
+    const float2 *one;
     const float2 *lo[kUMaxLog2 + 1];          // pre-twiddle tables of the second pass
     const float2 *hi[kUMaxLog2 + 1];
     int lobits[kUMaxLog2 + 1];

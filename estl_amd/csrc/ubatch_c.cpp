@@ -2,7 +2,7 @@
 //
 // create: validate the (size, offset) descriptors, sort the transforms by size
 //         (largest first), cut them into work items (groups of same-size rows for
-//         n <= 2^12, one transform per item above), upload the item list, the sorted
+//         n <= 2^13, one transform per item above), upload the item list, the sorted
 //         offsets and the twiddle-table pointers, allocate the scratch used by the
 //         two-pass transforms and the two ticket counters (zeroed once; the kernel
 //         leaves them zero);
@@ -148,6 +148,13 @@ static int ubatch_create(UBatch **out, int count, const long *sizes, const long 
         bool used = false;
         for (auto &it : u->items) used |= (it.log2n == L);
         if (!used) continue;
+        const int b = ubatch_split(L);
+        int rf = linear_table(u->device, 1L << b, 1, 1L << b, &tw.first[b]);
+        if (!rf) rf = linear_table(u->device, 1, 1, 1, &tw.one);
+        if (rf) {
+            ubatch_free(u);
+            return rf;
+        }
         const long nq = 1L << L;
         tw.lobits[L] = (L + 1) / 2;
         int rc = linear_table(u->device, 1L << tw.lobits[L], 1, nq, &tw.lo[L]);

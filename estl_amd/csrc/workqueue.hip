@@ -5,8 +5,8 @@
 // serves mixed sizes with one FFT object -- one plan, one program, one launch per pass --
 // per size (tests/Test.cpp:48-53).  Here a descriptor list holds every transform of the
 // batch and one launch computes them all:
-//   * a work item is either a group of same-size rows (n <= 2^12: kUThreads/TPT rows computed
-//     like k_fft_rows) or one whole large transform (2^13 <= n <= 2^20: both passes of a
+//   * a work item is either a group of same-size rows (n <= 2^13: kUThreads/TPT rows computed
+//     like k_fft_rows) or one whole large transform (2^14 <= n <= 2^20: both passes of a
 //     two-pass plan, tile by tile, through a scratch region, with a workgroup barrier
 //     between the passes -- no dependency crosses workgroups);
 //   * items are ordered largest first and handed out by an atomic ticket, so workgroups
@@ -16,6 +16,7 @@
 #include <utility>
 
 #include "pass_tile.h"
+#include "pass_wide.h"
 #include "ubatch.h"
 
 namespace estl {
@@ -25,13 +26,6 @@ namespace estl {
 // 2^U{8..18}): 512 threads at four waves per SIMD 2.53 ms, 256 threads 3.42 ms (its
 // 8-column tiles of radix 2^9 read 64-byte runs), 512 threads at three waves 2.97 ms.
 constexpr int kUThreads = 1 << kUThreadsLog2;
-static_assert(kUThreadsLog2 + 4 <= kUMaxSmallLog2 + 1, "every large size must fill a workgroup's tile");
-
-// pass split of the large sizes: 2^L = 2^(L/2) x 2^(L - L/2).  Measured on MI355X
-// (1 GiB of one size per launch): the even split beats skewed ones -- a radix-16 first
-// pass with 256-column tiles and a 2^10..2^12 second pass was 1.7x (L = 14) to 6x
-// (L = 16) slower, a 2^9 second pass 2-20 % slower.
-__host__ __device__ constexpr int ubatch_split(int L) { return L / 2; }
 
 template <int L>
 struct USmall {
@@ -40,12 +34,27 @@ struct USmall {
     static constexpr int slice = G::uses_lds ? Lds<kLdsPad>::size(G::N) : 0;
     static constexpr int lds = TPW * slice;
 };
+// Transforms of 2^17 values and more keep 32 values per thread (wide_tile, tiles of 2^14
+// values: twice the bytes in flight at the same four waves per SIMD): 500 of 2^17
+// 476-520 -> 457-476 us, 60 of 2^20 2.08 -> 1.31 ms, 8192 of 2^8 .. 2^18 2.43 -> 2.31 ms.  With so
+// few tiles a transform, 2^15 and 2^16 are 7 % slower that way (as 2^8 2^8 or with a
+// second radix of 2^9).
 template <int L>
 struct ULarge {
+    static constexpr bool wide = L >= 17;
     static constexpr int B1 = ubatch_split(L), B2 = L - B1;
-    static constexpr int T1 = kUThreadsLog2 + 4 - B1, T2 = kUThreadsLog2 + 4 - B2;  // threads = T B / 16
-    static constexpr int lds = PassTile<B1, T1>::lds_size > PassTile<B2, T2>::lds_size ? PassTile<B1, T1>::lds_size
-                                                                                        : PassTile<B2, T2>::lds_size;
+    static constexpr int per = kUThreadsLog2 + (wide ? 5 : 4);  // values of a tile
+    static constexpr int T1 = per - B1, T2 = per - B2;
+    static constexpr int floats() {
+        if constexpr (wide) {
+            const int f = WideTile<B1, T1, kWideFirst>::lds_floats, l = WideTile<B2, T2, kWideLast>::lds_floats;
+            return f > l ? f : l;
+        } else {
+            const int f = PassTile<B1, T1>::lds_size, l = PassTile<B2, T2>::lds_size;
+            return 2 * (f > l ? f : l);
+        }
+    }
+    static constexpr int lds = (floats() + 1) / 2;
 };
 
 template <int... Ls>
@@ -64,7 +73,7 @@ constexpr int large_lds_max(std::integer_sequence<int, Ls...>) {
 constexpr int kULdsSmall = small_lds_max(std::make_integer_sequence<int, kUMaxSmallLog2>{});
 constexpr int kULdsLarge = large_lds_max(std::make_integer_sequence<int, kUMaxLog2 - kUMaxSmallLog2>{});
 constexpr int kULds = kULdsSmall > kULdsLarge ? kULdsSmall : kULdsLarge;
-static_assert(kULds * 8 <= (kUThreadsLog2 >= 10 ? 160 : 80) * 1024, "work-queue LDS over budget");
+static_assert(kULds * 8 <= 79 * 1024, "two workgroups per CU");
 
 template <int L, int DIR>
 __device__ __forceinline__ void small_item(const UArgs &a, const UItem &it, float2 *lds) {
@@ -90,6 +99,7 @@ __device__ __forceinline__ void small_item(const UArgs &a, const UItem &it, floa
 template <int L, int DIR>
 __device__ __forceinline__ void large_item(const UArgs &a, const UItem &it, float2 *lds) {
     constexpr int B1 = ULarge<L>::B1, B2 = ULarge<L>::B2, T1 = ULarge<L>::T1, T2 = ULarge<L>::T2;
+    constexpr bool WIDE = ULarge<L>::wide;
     const long off = a.offs[it.first];
     PassArgs p1{};
     p1.batch = 1;
@@ -97,10 +107,19 @@ __device__ __forceinline__ void large_item(const UArgs &a, const UItem &it, floa
     p1.log2n = L;
     p1.log2S = L - B1;
     p1.scale = 1.0f;
-    p1.tw_local = a.tw.pow[B1];
+    if constexpr (WIDE) {
+        p1.lobits = B1;
+        p1.tw_lo = a.tw.first[B1];
+        p1.tw_hi = a.tw.one;
+    } else {
+        p1.tw_local = a.tw.pow[B1];
+    }
 #pragma unroll 1
-    for (long tile = 0; tile < (1L << (L - B1 - T1)); ++tile)
-        pass_tile<B1, DIR, T1>(a.in + off, a.scratch + off, p1, tile, lds, true);
+    for (long tile = 0; tile < (1L << (L - B1 - T1)); ++tile) {
+        if constexpr (WIDE)
+            wide_tile<B1, DIR, T1, kWideFirst>(a.in + off, a.scratch + off, p1, tile, reinterpret_cast<float *>(lds), true);
+        else pass_tile<B1, DIR, T1>(a.in + off, a.scratch + off, p1, tile, lds, true);
+    }
     __syncthreads();  // this workgroup's scratch writes are visible to all its threads
     PassArgs p2{};
     p2.batch = 1;
@@ -109,12 +128,15 @@ __device__ __forceinline__ void large_item(const UArgs &a, const UItem &it, floa
     p2.log2S = 0;
     p2.lobits = a.tw.lobits[L];
     p2.scale = a.scale;
-    p2.tw_local = a.tw.pow[B2];
+    if constexpr (!WIDE) p2.tw_local = a.tw.pow[B2];
     p2.tw_lo = a.tw.lo[L];
     p2.tw_hi = a.tw.hi[L];
 #pragma unroll 1
-    for (long tile = 0; tile < (1L << (L - B2 - T2)); ++tile)
-        pass_tile<B2, DIR, T2>(a.scratch + off, a.out + off, p2, tile, lds, true);
+    for (long tile = 0; tile < (1L << (L - B2 - T2)); ++tile) {
+        if constexpr (WIDE)
+            wide_tile<B2, DIR, T2, kWideLast>(a.scratch + off, a.out + off, p2, tile, reinterpret_cast<float *>(lds), true);
+        else pass_tile<B2, DIR, T2>(a.scratch + off, a.out + off, p2, tile, lds, true);
+    }
 }
 
 // waves per SIMD the register budget is held to (0: the compiler's choice)
@@ -151,13 +173,7 @@ k_ubatch(UArgs a) {
 #define LARGE(L) \
     case L: large_item<L, DIR>(a, it, lds); break;
             SMALL(1) SMALL(2) SMALL(3) SMALL(4) SMALL(5) SMALL(6) SMALL(7) SMALL(8) SMALL(9) SMALL(10) SMALL(11)
-            SMALL(12)
-#if ESTL_UBATCH_TLOG >= 10
-            SMALL(13)
-#else
-            LARGE(13)
-#endif
-            LARGE(14) LARGE(15) LARGE(16) LARGE(17) LARGE(18) LARGE(19) LARGE(20)
+            SMALL(12) SMALL(13) LARGE(14) LARGE(15) LARGE(16) LARGE(17) LARGE(18) LARGE(19) LARGE(20)
 #undef SMALL
 #undef LARGE
             default: break;
@@ -186,9 +202,7 @@ int ubatch_small_rows_per_item(int log2n) {
 #define TPWC(L) \
     case L: return USmall<L>::TPW;
         TPWC(1) TPWC(2) TPWC(3) TPWC(4) TPWC(5) TPWC(6) TPWC(7) TPWC(8) TPWC(9) TPWC(10) TPWC(11) TPWC(12)
-#if ESTL_UBATCH_TLOG >= 10
         TPWC(13)
-#endif
 #undef TPWC
         default: return 1;
     }
