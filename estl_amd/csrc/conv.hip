@@ -34,6 +34,7 @@ namespace estl {
 __device__ __forceinline__ float filter_l1_256(const float *__restrict__ h, long k, float *part) {
     if (threadIdx.x < 256) {
         float acc = 0.0f;
+#pragma unroll 8
         for (long i = threadIdx.x; i < k; i += 256) acc += fabsf(h[i]);
         part[threadIdx.x] = acc;
     }
@@ -79,7 +80,7 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
                   float2 *__restrict__ dc, float2 *__restrict__ l1_single) {
     using G = BlockGeom<LOG2N>;
     constexpr int N = G::N, E = G::E, TPT = G::TPT;
-    __shared__ float2 lds[G::uses_lds ? Lds<kLdsPad>::size(N) : 1];
+    __shared__ float2 lds[G::uses_lds ? Lds::size(N) : 1];
     __shared__ float s_dc;
     __shared__ float s_part[TPT >= 256 ? 256 : 1];
     const int tl = opaque_lane(threadIdx.x);
@@ -102,8 +103,7 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
 #pragma unroll
         for (int i = 0; i < E; ++i) v[i] = make_float2(fold_tap(h, k, N, shift, tl + TPT * i), 0.0f);
     }
-    // kSpecTw: the power table below 4096 points, the block table from 4096
-    block_fft<LOG2N, -1, kLdsPad, false, kSpecTw<LOG2N>>(v, lds, tl, tw, false);
+    block_fft<LOG2N, -1>(v, lds, tl, tw, false);
     if (normalize) {
         if (tl == 0) {
             s_dc = v[0].x;  // bin 0
@@ -136,7 +136,7 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
     }
     if constexpr (LOG2N >= kWaveMinLog2) {
         // bins to the order k_conv_rows and k_conv_ols of this length read them in
-        using P = Lds<kLdsPad>;
+        using P = Lds;
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < E; ++i) lds[P::idx(tl + TPT * i)] = v[i];
@@ -195,8 +195,9 @@ __device__ __forceinline__ void multiply_spectrum(float2 (&v)[32], const float2 
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Pairs of real rows of N >= 2^10 values, TPW = max(1, 256 / T) pairs per workgroup and
-// one workgroup per group of pairs: forward transform, multiply, inverse transform in
+// Pairs of real rows of N >= 2^10 values, TPW = max(1, 64 / T) pairs per workgroup (the
+// smallest ones are done and replaced soonest: 256-thread workgroups were 7 % slower at
+// 2^10 and 2^11 values and 2000 rows, 13 % at 2000 rows of 2^10) and one workgroup per group of pairs: forward transform, multiply, inverse transform in
 // registers (wave_fft), each value read and written once.  With a request group, `rows`
 // counts the group's pairs twice and each slot takes its pair's member: input rows,
 // spectrum and output rows.  R: the stored real type, float or _Float16 (FP16 storage: the
@@ -204,7 +205,7 @@ __device__ __forceinline__ void multiply_spectrum(float2 (&v)[32], const float2 
 // [-1, 1] (|y| <= sum |h| max |x|); the caller's per-row scales carry the magnitudes).
 // Bound by HBM and VALU alike: 65 vector instructions per complex value at 2^10 points and
 // no barrier (16 values per thread and three exchanges across the workgroup took 105).
-// 30001 rows of 1024 values: 55.3 -> 49.7 us (4.44 -> 4.94 TB/s); 4001 rows of 8192: 83 -> 59 us.
+// 30001 rows of 1024 values: 54.2 -> 45.3 us (4.53 -> 5.43 TB/s); 4001 rows of 8192: 84 -> 59 us.
 template <int LOG2N, int TPW, bool CORR, typename R>
 __global__ void __launch_bounds__(WaveGeom<LOG2N>::T * TPW) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 *__restrict__ spec,
@@ -255,7 +256,7 @@ k_conv_rows(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
             const float2 *__restrict__ tw, float scale, const ConvGroup *__restrict__ group) {
     using G = BlockGeom<LOG2N>;
     constexpr int N = G::N, E = G::E, TPT = G::TPT;
-    constexpr int SLICE = G::uses_lds ? Lds<kLdsPad>::size(N) : 0;
+    constexpr int SLICE = G::uses_lds ? Lds::size(N) : 0;
     constexpr int LDS = G::uses_lds ? TPW * SLICE : 1;
     __shared__ float2 lds[LDS];
     const long pairs = (rows + 1) / 2;
@@ -280,13 +281,13 @@ k_conv_rows(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
 #pragma unroll
         for (int i = 0; i < E; ++i)
             v[i] = make_float2(ld_real(x1 + TPT * i), two ? ld_real(x1 + N + TPT * i) : 0.0f);
-        block_fft<LOG2N, -1, kLdsPad, false, kTwPowers>(v, lds + w * SLICE, tl, tw, true);
+        block_fft<LOG2N, -1>(v, lds + w * SLICE, tl, tw, true);
 #pragma unroll
         for (int i = 0; i < E; ++i) {
             const float2 hk = spec[tl + TPT * i];
             v[i] = CORR ? cmulc(v[i], hk) : cmul(v[i], hk);
         }
-        block_fft<LOG2N, +1, kLdsPad, false, kTwPowers>(v, lds + w * SLICE, tl, tw, true);
+        block_fft<LOG2N, +1>(v, lds + w * SLICE, tl, tw, true);
         if (active) {
             R *y1 = y + r1 * N + tl;
 #pragma unroll
@@ -616,7 +617,7 @@ static hipError_t launch_conv_rows_t(const R *x, R *y, long rows, const float2 *
                                      hipStream_t st, const ConvGroup *group) {
     if constexpr (LOG2N >= kWaveMinLog2) {
         using G = WaveGeom<LOG2N>;
-        constexpr int TPW = (G::T >= 256) ? 1 : 256 / G::T;
+        constexpr int TPW = (G::T >= 64) ? 1 : 64 / G::T;
         const long pairs = (rows + 1) / 2, groups = (pairs + TPW - 1) / TPW;
         if (groups > 0x7fffffffL) return hipErrorInvalidValue;
         hipLaunchKernelGGL((k_conv_wave<LOG2N, TPW, CORR, R>), dim3((unsigned)groups), dim3(G::T * TPW), 0, st, x, y,

@@ -162,10 +162,7 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
     } else if (c->spec_plan.kind != Plan::ROWS) {
         return set_error(ESTL_ERR_UNSUPPORTED, "convolution of n=%ld: no spectrum plan", n);
     } else {
-        // k_filter_spectrum's table (kSpecTw): the rows plan's power table below 4096
-        // points, the block table from 4096
-        c->tw_spec = c->spec_plan.tw_rows;
-        if (c->log2n >= kSpecBlockTwLog2 && (rc = block_table(current_device(), c->log2n, &c->tw_spec))) return rc;
+        c->tw_spec = c->spec_plan.tw_rows;  // k_filter_spectrum's table: the rows plan's powers
     }
     if (c->log2n <= kMaxRowsLog2) {
         c->fused = true;
@@ -175,7 +172,7 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
     }
     for (int w = 0; w < 2; ++w) {
         if (c->log2n <= kOlsLog2 + w) break;
-        if ((rc = block_table(current_device(), kOlsLog2 + w, &c->tw_ols[w]))) return rc;
+        if ((rc = power_table(current_device(), kOlsLog2 + w, &c->tw_ols[w]))) return rc;
         if ((rc = wave_table(current_device(), kOlsLog2 + w, &c->tw_ols_roots[w]))) return rc;
     }
     // forward passes with the default split; the inverse runs the radices in the reverse

@@ -81,7 +81,7 @@ static hipStream_t table_stream(int device) {
     return s;
 }
 
-// Power table of BlockGeom<log2n> (block_fft's kTwPowers): W_{N_q}^g at powoff(q) + g,
+// Power table of BlockGeom<log2n> (block_fft): W_{N_q}^g at powoff(q) + g,
 // g in [0, A_q), per pass q >= 1, then their fourth powers in the same order; FP64 on the
 // device, rounded once.
 int power_table(int device, int log2n, const float2 **out) {
@@ -104,7 +104,7 @@ int power_table(int device, int log2n, const float2 **out) {
             long A;
             int B;
             rows_pass_params(log2n, q, &A, &B);
-            HIP_TRY(launch_twiddle(d + off, A, 1, A, e, A * B, ts));
+            HIP_TRY(launch_twiddle(d + off, A, 0, A, e, A * B, ts));
             off += A;
         }
     HIP_TRY(hipStreamSynchronize(ts));
@@ -132,40 +132,10 @@ int wave_table(int device, int log2n, const float2 **out) {
     HIP_TRY(hipMalloc(&d, sizeof(float2) * (point + 3 * T)));
     for (int e = 0; e < 3; ++e) {
         const long power = 1L << (2 * e);
-        HIP_TRY(launch_twiddle(d + 32 * e, 32, 1, 1, N / 1024 * power, N, ts));
-        if (e < 2) HIP_TRY(launch_twiddle(d + bin + 1024 * e, 1024, 2, Q, power, N, ts));
-        HIP_TRY(launch_twiddle(d + pos + Q * e, Q, 1, 1, 32 * power, N, ts));
-        HIP_TRY(launch_twiddle(d + point + T * e, T, 1, 1, power, N, ts));
-    }
-    HIP_TRY(hipStreamSynchronize(ts));
-    c.tables[key] = d;
-    *out = d;
-    return ESTL_OK;
-}
-
-// Table of BlockGeom<log2n>: W_{N_q}^{g s} at [(s-1) A_q + g] per pass q >= 1.
-int block_table(int device, int log2n, const float2 **out) {
-    auto &c = twcache();
-    std::lock_guard<std::mutex> lk(c.mu);
-    auto key = std::make_tuple(device, 0, (long)log2n, 0L, 0L);
-    auto it = c.tables.find(key);
-    if (it != c.tables.end()) {
-        *out = it->second;
-        return ESTL_OK;
-    }
-    long count = rows_twiddle_count(log2n);
-    if (count < 0) return set_error(ESTL_ERR_UNSUPPORTED, "no block kernel for log2n=%d", log2n);
-    float2 *d = nullptr;
-    hipStream_t ts = table_stream(device);
-    HIP_TRY(hipMalloc(&d, sizeof(float2) * (count > 0 ? count : 1)));
-    long off = 0;
-    for (int q = 1; q < rows_pass_count(log2n); ++q) {
-        long A;
-        int B;
-        rows_pass_params(log2n, q, &A, &B);
-        long cnt = (long)(B - 1) * A;
-        HIP_TRY(launch_twiddle(d + off, cnt, 0, A, 0, A * B, ts));
-        off += cnt;
+        HIP_TRY(launch_twiddle(d + 32 * e, 32, 0, 1, N / 1024 * power, N, ts));
+        if (e < 2) HIP_TRY(launch_twiddle(d + bin + 1024 * e, 1024, 1, Q, power, N, ts));
+        HIP_TRY(launch_twiddle(d + pos + Q * e, Q, 0, 1, 32 * power, N, ts));
+        HIP_TRY(launch_twiddle(d + point + T * e, T, 0, 1, power, N, ts));
     }
     HIP_TRY(hipStreamSynchronize(ts));
     c.tables[key] = d;
@@ -186,7 +156,7 @@ int linear_table(int device, long count, long mult, long nq, const float2 **out)
     float2 *d = nullptr;
     hipStream_t ts = table_stream(device);
     HIP_TRY(hipMalloc(&d, sizeof(float2) * count));
-    HIP_TRY(launch_twiddle(d, count, 1, 1, mult, nq, ts));
+    HIP_TRY(launch_twiddle(d, count, 0, 1, mult, nq, ts));
     HIP_TRY(hipStreamSynchronize(ts));
     c.tables[key] = d;
     *out = d;
@@ -317,7 +287,6 @@ int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned fla
     }
     if (p->log2n <= kMaxRowsLog2 && !(split && !split->empty())) {
         p->kind = Plan::ROWS;
-        // the rows kernels' twiddle source (kRowsTw): powers
         return power_table(p->device, p->log2n, &p->tw_rows);
     }
     p->kind = Plan::PASSES;

@@ -35,15 +35,7 @@ struct BlockGeom {
         for (int p = 0; p < q; ++p) a *= radix(p);
         return a;
     }
-    // offset of pass q's twiddles in the table; pass q stores W_{N_q}^{g s} at
-    // [(s - 1) * A_q + g] for s in [1, B_q), g in [0, A_q) (pass 0 needs none)
-    static constexpr long twoff(int q) {
-        long o = 0;
-        for (int p = 1; p < q; ++p) o += (radix(p) - 1) * A(p);
-        return o;
-    }
-    static constexpr long twsize = twoff(P);
-    // the power table (TwPowers): W_{N_q}^g for g in [0, A_q) per pass q >= 1, at
+    // the power table: W_{N_q}^g for g in [0, A_q) per pass q >= 1, at
     // powoff(q), and their fourth powers powsum further on
     static constexpr long powoff(int q) {
         long o = 0;
@@ -54,42 +46,19 @@ struct BlockGeom {
     static constexpr bool uses_lds = TPT > 1;
 };
 
-// Twiddle sources of block_fft's passes q >= 1 (each butterfly of pass q, group g, needs
-// W_{N_q}^{g s} for s in [1, B_q)):
-//   kTwBlock:  every W_{N_q}^{g s} read from the block table (B_q - 1 reads per
-//              butterfly; the table is N values, 128 KiB at N = 2^14);
-//   kTwPowers: two reads, w = W_{N_q}^g and w^4 from the power table (twice the sum of the
-//              A_q, 68 KiB at 2^14, mostly cache-resident); w^2 and w^8 by squaring, and the
-//              twiddles of each level of the DFT from them (dft_twiddled).  Trades the long-latency reads of
-//              a table too big for L1 for VALU work.
-enum { kTwBlock = 0, kTwPowers = 1 };
-// Twiddle source of the rows kernels (k_fft_rows, _planar, _h): powers at every
-// row length (a rows plan's table is the power table, estl_c.cpp).  The block table's
-// twiddles kept in registers across rows needed 167-206 VGPRs and measured 6-9 % slower at
-// 4096 and 8192 points, and read again for each row from L2 they cost more.  Rel-L2
-// against FP64 is 1.6e-7 at 4096 points (the bound is 1.2e-5): 3.0e-7 when every power
-// came from w alone, 1.2e-7 with the block table's rounded values.
-template <int LOG2N>
-constexpr int kRowsTw = kTwPowers;
-// Twiddle source of the filter spectrum (k_filter_spectrum): the block table from 4096
-// points.  A spectrum is computed once per request or registration, so its speed hardly
-// matters, and the correctly rounded twiddles keep, e.g., a delayed unit impulse's
-// spectrum -- and the convolution by it -- within 2e-6 of the shifted input.
-template <int LOG2N>
-constexpr int kSpecTw = LOG2N < kSpecBlockTwLog2 ? kTwPowers : kTwBlock;
-// LDS layouts of a sequence's exchange buffer.
-//  kLdsPad: one float2 of padding after every 16 values; addresses stay base + constant,
-//           so the exchange reads use immediate offsets (fewest VGPRs);
-//  kLdsXor: no padding, value i sits in row i/16 at column (i mod 16) XOR (row mod 16).
-//           Every exchange of these passes touches, per 16 lanes, either 16 consecutive
-//           values of one row or one value from each of 16 rows at a fixed column; the
-//           XOR spreads both over 16 distinct columns (all 32 four-byte banks for 8-byte
-//           values) and a 4096-value sequence needs exactly 32 KiB.
-enum { kLdsPad = 0, kLdsXor = 1 };
-template <int LAYOUT>
-struct Lds;
-template <>
-struct Lds<kLdsPad> {
+// Twiddles of block_fft's passes q >= 1 (a butterfly of pass q, group g, needs W_{N_q}^{g s}
+// for s in [1, B_q)): w = W_{N_q}^g and w^4 read from the power table (twice the sum of the
+// A_q, 68 KiB at 2^14, mostly cache-resident), w^2 and w^8 by squaring, the twiddles of
+// each level of the DFT from them (dft_twiddled).  A table of every W_{N_q}^{g s} (128 KiB
+// at 2^14, B_q - 1 reads per butterfly) held in registers across rows needed 167-206 VGPRs
+// and was 6-9 % slower at 4096 and 8192 points, and read again for each row slower still;
+// the filter spectra of 2^14 and binary16 storage took 15.8 us with it, 12.0 with powers.
+// Rel-L2 against FP64 is 1.6e-7 at 4096 points (the bound is 1.2e-5): 3.0e-7 when every
+// power came from w alone, 1.2e-7 with that table's rounded values.
+
+// LDS layout of a sequence's exchange buffer: one float2 of padding after every 16 values;
+// addresses stay base + constant, so the exchanges use immediate offsets.
+struct Lds {
     static constexpr int size(int n) { return n + (n >> 4); }
     static __device__ __forceinline__ int idx(int i) { return i + (i >> 4); }
     // idx(i + off), given idx(i), where adding off to i carries nothing into bit 4 (off a
@@ -99,23 +68,14 @@ struct Lds<kLdsPad> {
     // with these and dft_dit's folded twiddles).
     static __device__ __forceinline__ constexpr int step(int at, int off) { return at + off + (off >> 4); }
 };
-template <>
-struct Lds<kLdsXor> {
-    static constexpr int size(int n) { return n; }
-    static __device__ __forceinline__ int idx(int i) { return i ^ ((i >> 4) & 15); }
-};
 
 // On entry v[i] = x[tl + TPT*i]; on exit v[i] = X[tl + TPT*i] (X = DFT of x, sign DIR).
-// `lds` is this sequence's LDS slice (Lds<LAYOUT>::size(N) float2); `tw` the size-N block
-// table (TWSRC = kTwBlock) or the power table (kTwPowers).
+// `lds` is this sequence's LDS slice (Lds::size(N) float2); `tw` the size-N power table.
 // All threads of the workgroup must call it together (it holds workgroup barriers).
 // If `lds_busy` is set, the slice is still being read on entry and a barrier is placed
-// before the first LDS write.  HOIST_TW lets the compiler keep the twiddles of every pass
-// in registers across calls made from a loop over one size; callers that dispatch many
-// sizes in one loop pass false so each size's twiddles are reloaded (from L1/L2)
-// instead of all staying live.  No kernel sets it at present: the rows kernels, its
-// last user, run faster at one row per workgroup with twiddles by powers (k_fft_rows).
-template <int LOG2N, int DIR, int LAYOUT = kLdsPad, bool HOIST_TW = false, int TWSRC = kTwBlock>
+// before the first LDS write.  Twiddles are read anew at each use (from L1/L2): callers that
+// run many rows or sizes in one loop would otherwise have all of them live.
+template <int LOG2N, int DIR>
 __device__ __forceinline__ void block_fft(float2 (&v)[BlockGeom<LOG2N>::E], float2 *lds, int tl,
                                           const float2 *__restrict__ tw, bool lds_busy = false) {
     using G = BlockGeom<LOG2N>;
@@ -136,11 +96,11 @@ __device__ __forceinline__ void block_fft(float2 (&v)[BlockGeom<LOG2N>::E], floa
             });
         } else {
             if (q > 1 || lds_busy) __syncthreads();
-            const int at = Lds<LAYOUT>::idx(tl);
+            const int at = Lds::idx(tl);
 #pragma unroll
             for (int i = 0; i < E; ++i) {
-                if constexpr (LAYOUT == kLdsPad && TPT % 16 == 0) lds[Lds<kLdsPad>::step(at, TPT * i)] = v[i];
-                else lds[Lds<LAYOUT>::idx(tl + TPT * i)] = v[i];
+                if constexpr (TPT % 16 == 0) lds[Lds::step(at, TPT * i)] = v[i];
+                else lds[Lds::idx(tl + TPT * i)] = v[i];
             }
             __syncthreads();
             StaticFor<0, NB>::run([&](auto bc) {
@@ -149,23 +109,13 @@ __device__ __forceinline__ void block_fft(float2 (&v)[BlockGeom<LOG2N>::E], floa
                 const int g = j / S, z = j % S;   // S is a power of two
                 const int base = S * B * g + z;
                 float2 u[B];
-                const int from = Lds<LAYOUT>::idx(base);
+                const int from = Lds::idx(base);
+                // base is a multiple of S B plus z < S: S s is a multiple of 16, or less
+                // than 16 - z within the aligned 16 of S B >= 16 or S B < 16 values
 #pragma unroll
-                for (int s = 0; s < B; ++s) {
-                    // base is a multiple of S B plus z < S: S s (a multiple of 16, or less
-                    // than 16 - z within the aligned 16 of S B >= 16 or S B < 16 values)
-                    if constexpr (LAYOUT == kLdsPad) u[s] = lds[Lds<kLdsPad>::step(from, S * s)];
-                    else u[s] = lds[Lds<LAYOUT>::idx(base + S * s)];
-                }
-                if constexpr (TWSRC == kTwPowers) {
-                    const float2 *w = (HOIST_TW ? tw : opaque(tw)) + G::powoff(q) + g;
-                    dft_twiddled<B, DIR>(u, w, w + G::powsum);
-                } else {
-                    const float2 *twq = (HOIST_TW ? tw : opaque(tw)) + G::twoff(q) + g;
-#pragma unroll
-                    for (int s = 1; s < B; ++s) u[s] = ctw<DIR>(u[s], twq[(s - 1) * Aq]);
-                    Dft<B, DIR>::run(u);
-                }
+                for (int s = 0; s < B; ++s) u[s] = lds[Lds::step(from, S * s)];
+                const float2 *w = opaque(tw) + G::powoff(q) + g;
+                dft_twiddled<B, DIR>(u, w, w + G::powsum);
 #pragma unroll
                 for (int h = 0; h < B; ++h) v[b + NB * h] = u[h];
             });

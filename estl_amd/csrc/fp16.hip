@@ -213,7 +213,7 @@ k_fft_rows_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, long batch, 
              float scale, const float *__restrict__ s_in, float *__restrict__ s_out, float s_factor) {
     using G = BlockGeom<LOG2N>;
     constexpr int N = G::N, E = G::E, TPT = G::TPT;
-    constexpr int SLICE = G::uses_lds ? Lds<kLdsPad>::size(N) : 0;
+    constexpr int SLICE = G::uses_lds ? Lds::size(N) : 0;
     constexpr int LDS = G::uses_lds ? TPW * SLICE : 1;
     __shared__ float2 lds[LDS];
     if constexpr (TPW == 1) {
@@ -226,7 +226,7 @@ k_fft_rows_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, long batch, 
         const f16x2 *src = in + row * N + tl;
 #pragma unroll
         for (int i = 0; i < E; ++i) v[i] = ld_elem(src + TPT * i);
-        block_fft<LOG2N, DIR, kLdsPad, false, kRowsTw<LOG2N>>(v, lds, tl, tw, false);
+        block_fft<LOG2N, DIR>(v, lds, tl, tw, false);
         f16x2 *dst = out + row * N + tl;
 #pragma unroll
         for (int i = 0; i < E; ++i) st_elem(dst + TPT * i, cscale(v[i], scale));
@@ -244,7 +244,7 @@ k_fft_rows_h(const f16x2 *__restrict__ in, f16x2 *__restrict__ out, long batch, 
         const f16x2 *src = in + row * N + tl;
 #pragma unroll
         for (int i = 0; i < E; ++i) v[i] = ld_elem(src + TPT * i);
-        block_fft<LOG2N, DIR, kLdsPad, false, kRowsTw<LOG2N>>(v, lds + w * SLICE, tl, tw, busy);
+        block_fft<LOG2N, DIR>(v, lds + w * SLICE, tl, tw, busy);
         busy = true;
         if (want < batch) {
             f16x2 *dst = out + row * N + tl;

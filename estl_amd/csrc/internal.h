@@ -41,7 +41,7 @@ struct PassArgs {
     int xcd_remap;           // deal consecutive tiles to the same XCD
     int wide;                // run by k_pass_wide (complex rows, no io_in or io_out mode)
     float scale;             // applied to the stored values (1 = none)
-    const float2 *tw_local;  // power table of the radix-B DFT (block_fft kTwPowers)
+    const float2 *tw_local;  // power table of the radix-B DFT (block_fft)
     const float2 *tw_lo;     // W_{A B}^{lo}, lo < 2^lobits
     const float2 *tw_hi;     // W_{A B}^{hi << lobits}
     // I/O modes of the convolution pipeline (0 = plain complex rows in and out):
@@ -124,13 +124,11 @@ hipError_t launch_fill_uniform(float *dst, long count, uint64_t seed, uint64_t o
 // copy n16 blocks of 16 bytes (16-byte aligned), nontemporal or plain loads and stores
 hipError_t launch_stream_copy(const void *src, void *dst, long n16, bool nontemporal, hipStream_t st);
 
-long rows_twiddle_count(int log2n);
 long rows_power_count(int log2n);  // entries of BlockGeom<log2n>'s power table
 void rows_pass_params(int log2n, int q, long *A, int *B);
 int rows_pass_count(int log2n);
 
 constexpr int kMaxRowsLog2 = 13;   // largest single-launch row length
-constexpr int kSpecBlockTwLog2 = 12;  // filter spectra of at least 2^12 points read the block table
 constexpr int kMaxPassLog2 = 13;   // largest radix of a global pass
 constexpr int kMaxSplitLog2Fp16 = 9;  // largest radix of an FP16 pass that a caller can ask for
 constexpr int kMaxPassTileLog2 = 14;  // a pass tile holds at most 2^14 values (~139 KiB of LDS)

@@ -20,19 +20,15 @@
 namespace estl {
 
 // ------------------------------------------------------------------ twiddles
-// mode 0 (per-pass layout of BlockGeom): entry e -> s = e / A + 1, g = e % A, m = g*s
-// mode 1 (linear): entry e -> m = e * mult
-// mode 2 (the bin roots of WaveRoots, Q = A): entry e = r T + u, T = 32 Q ->
+// mode 0 (linear): entry e -> m = e * mult
+// mode 1 (the bin roots of WaveRoots, Q = A): entry e = r T + u, T = 32 Q ->
 //         m = mult * bin, bin = u / Q + 32 (r + (32 / Q) (u mod Q))
 // value = exp(-2 pi i m / nq), computed as sincospi(2 m / nq) in double.
 __global__ void k_twiddle(float2 *__restrict__ dst, long count, int mode, long A, long mult, long nq) {
     long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
     long m;
-    if (mode == 0) {
-        long s = e / A + 1, g = e % A;
-        m = (g * s) % nq;
-    } else if (mode == 2) {
+    if (mode == 1) {
         const long r = e / (32 * A), u = e % (32 * A);
         m = (u / A + 32 * (r + 32 / A * (u % A))) * mult % nq;
     } else {
@@ -103,11 +99,11 @@ hipError_t launch_stream_copy(const void *src, void *dst, long n16, bool nontemp
 // whole transform in registers and padded LDS, one HBM read and one HBM write per
 // value, nontemporal loads and stores.  A partial last group computes its missing rows
 // on a copy of the last row and stores nothing for them.  With twiddles by powers
-// (kRowsTw) the kernel holds 58 VGPRs at 4096 and 8192 points, so LDS alone bounds
+// the kernel holds 58 VGPRs at 4096 and 8192 points, so LDS alone bounds
 // residency (four 34 KiB groups per CU; two 8192-point rows), and it runs at the copy's
 // rate: 4096 x 16384 in 167-175 us between devices, 6.1-6.4 TB/s of the copy's 6.55.  Measured against
 // the earlier persistent grid (four resident rounds of workgroups, the next group
-// prefetched into registers; at 4096 and 8192 points the block table's twiddles held in
+// prefetched into registers; at 4096 and 8192 points a table of all twiddles held in
 // registers across rows, 167 / 206 VGPRs): 6.5 % faster at 4096 x 16384 and 9 % at
 // 8192 x 8192, 3-6 % at 512-2048 points -- many short-lived workgroups keep more loads
 // in flight, and the grid's last round is one group deep.
@@ -126,7 +122,7 @@ k_fft_rows(const float2 *__restrict__ in, float2 *__restrict__ out, long batch,
            const float2 *__restrict__ tw, float scale) {
     using G = BlockGeom<LOG2N>;
     constexpr int N = G::N, E = G::E, TPT = G::TPT;
-    constexpr int SLICE = G::uses_lds ? Lds<kLdsPad>::size(N) : 0;
+    constexpr int SLICE = G::uses_lds ? Lds::size(N) : 0;
     constexpr int LDS = G::uses_lds ? TPW * SLICE : 1;
     __shared__ float2 lds[LDS];
     float2 v[E];
@@ -138,7 +134,7 @@ k_fft_rows(const float2 *__restrict__ in, float2 *__restrict__ out, long batch,
 #pragma unroll
         for (int i = 0; i < E; ++i) v[i] = ld_stream(src + TPT * i);
         rows_loaded<LOG2N>();
-        block_fft<LOG2N, DIR, kLdsPad, false, kRowsTw<LOG2N>>(v, lds, tl, tw, false);
+        block_fft<LOG2N, DIR>(v, lds, tl, tw, false);
         float2 *dst = out + row * N + tl;
 #pragma unroll
         for (int i = 0; i < E; ++i) st_stream(dst + TPT * i, SCALED ? cscale(v[i], scale) : v[i]);
@@ -153,7 +149,7 @@ k_fft_rows(const float2 *__restrict__ in, float2 *__restrict__ out, long batch,
         rows_loaded<LOG2N>();
         {
             const int to = opaque_lane(t);
-            block_fft<LOG2N, DIR, kLdsPad, false, kRowsTw<LOG2N>>(v, lds + (to / TPT) * SLICE, to % TPT, tw, false);
+            block_fft<LOG2N, DIR>(v, lds + (to / TPT) * SLICE, to % TPT, tw, false);
         }
         if (want < batch) {
             float2 *dst = out + row * N + tl;
@@ -173,7 +169,7 @@ k_fft_rows_planar(const float2 *__restrict__ in, float2 *__restrict__ out, long 
                   float scale) {
     using G = BlockGeom<LOG2N>;
     constexpr int N = G::N, E = G::E, TPT = G::TPT;
-    constexpr int SLICE = G::uses_lds ? Lds<kLdsPad>::size(N) : 0;
+    constexpr int SLICE = G::uses_lds ? Lds::size(N) : 0;
     constexpr int LDS = G::uses_lds ? TPW * SLICE : 1;
     __shared__ float2 lds[LDS];
     const long groups = (batch + TPW - 1) / TPW;
@@ -186,7 +182,7 @@ k_fft_rows_planar(const float2 *__restrict__ in, float2 *__restrict__ out, long 
         float2 v[E];
 #pragma unroll
         for (int i = 0; i < E; ++i) v[i] = ld_planar(in, row * N + tl + TPT * i);
-        block_fft<LOG2N, DIR, kLdsPad, false, kRowsTw<LOG2N>>(v, lds + w * SLICE, tl, tw, busy);
+        block_fft<LOG2N, DIR>(v, lds + w * SLICE, tl, tw, busy);
         busy = true;
         if (want < batch) {
 #pragma unroll
@@ -279,17 +275,6 @@ hipError_t launch_rows_planar(int log2n, int dir, const float2 *in, float2 *out,
                    : launch_rows_planar_d<+1>(log2n, in, out, batch, tw, scale, st);
 }
 
-long rows_twiddle_count(int log2n) {
-    switch (log2n) {
-#define TW_CASE(L) \
-    case L: return BlockGeom<L>::twsize;
-        TW_CASE(1) TW_CASE(2) TW_CASE(3) TW_CASE(4) TW_CASE(5) TW_CASE(6) TW_CASE(7) TW_CASE(8)
-        TW_CASE(9) TW_CASE(10) TW_CASE(11) TW_CASE(12) TW_CASE(13) TW_CASE(14)
-#undef TW_CASE
-        default: return -1;
-    }
-}
-
 long rows_power_count(int log2n) {
     switch (log2n) {
 #define POW_CASE(L) \
@@ -301,7 +286,7 @@ long rows_power_count(int log2n) {
     }
 }
 
-// per-pass parameters of the block table (for building it): A_q and B_q of pass q
+// per-pass parameters of the power table (for building it): A_q and B_q of pass q
 void rows_pass_params(int log2n, int q, long *A, int *B) {
     const int nfull = log2n / 4, rem = log2n % 4;
     long a = 1;

@@ -32,7 +32,7 @@ struct PassTile {
     // Adjacent lanes serve adjacent columns, so column slices are strided by an odd
     // number of float2: 16 lanes at the same offset in 16 columns then land on 16
     // distinct 8-byte bank pairs (all 32 banks).
-    static constexpr int ldsp = Lds<kLdsPad>::size(B) | 1;
+    static constexpr int ldsp = Lds::size(B) | 1;
     static constexpr int lds_size = T * ldsp;
     static constexpr int threads = BlockGeom<LOG2B>::TPT << LOG2T;
 };
@@ -208,11 +208,11 @@ __device__ __forceinline__ void pass_tile_finish(ST *__restrict__ out, const Pas
             const int o = P.t + NT * k;
             const int gl = o >> (ls + LOG2B), rem = o & sbmask;
             const int s = rem >> ls, zz = rem & smask;
-            lds[((gl << ls) + zz) * LDSP + Lds<kLdsPad>::idx(s)] = v[k];
+            lds[((gl << ls) + zz) * LDSP + Lds::idx(s)] = v[k];
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < E; ++i) v[i] = lds[c * LDSP + Lds<kLdsPad>::idx(tl + TPT * i)];
+        for (int i = 0; i < E; ++i) v[i] = lds[c * LDSP + Lds::idx(tl + TPT * i)];
         busy = true;
     }
     if (a.A > 1) {
@@ -240,7 +240,7 @@ __device__ __forceinline__ void pass_tile_finish(ST *__restrict__ out, const Pas
             v[i] = ctw<DIR>(v[i], w);
         }
     }
-    block_fft<LOG2B, DIR, kLdsPad, false, kTwPowers>(v, lds + c * LDSP, tl, a.tw_local, busy);
+    block_fft<LOG2B, DIR>(v, lds + c * LDSP, tl, a.tw_local, busy);
     if (a.io_out == 2) {
         // re / im to real rows 2 row and 2 row + 1 of rout (FP32 or binary16); in a
         // request group, the member's pair and rows
@@ -280,7 +280,7 @@ __device__ __forceinline__ void pass_tile_finish(ST *__restrict__ out, const Pas
             const float2 hk = spec[j + ((tl + TPT * i) << lcpr)];
             v[i] = a.corr ? cmulc(v[i], hk) : cmul(v[i], hk);
         }
-        block_fft<LOG2B, -DIR, kLdsPad, false, kTwPowers>(v, lds + c * LDSP, tl, a.tw_local, true);
+        block_fft<LOG2B, -DIR>(v, lds + c * LDSP, tl, a.tw_local, true);
     }
     if (F32 && a.planar_out) {
         const long e0 = (P.row << a.log2n) + j;

@@ -71,8 +71,7 @@ inline size_t planar_bytes(long count) {
     } while (0)
 
 int current_device();
-int block_table(int device, int log2n, const float2 **out);
-int power_table(int device, int log2n, const float2 **out);  // block_fft's kTwPowers table
+int power_table(int device, int log2n, const float2 **out);  // block_fft's table
 int wave_table(int device, int log2n, const float2 **out);   // fft_wave.h's roots, log2n = 10..14
 int linear_table(int device, long count, long mult, long nq, const float2 **out);
 // Split log2n into passes of at most 9 bits, as evenly as possible, smaller radices first
@@ -130,7 +129,7 @@ struct ConvShape {
     bool half = false;
     Plan half_fwd, half_inv;
     // tables of the overlap-save windows of 2^13 (n > 2^13) and 2^14 (n > 2^14) values:
-    // block tables (the filter's window spectrum, kSpecTw) and roots (k_conv_ols)
+    // power tables (the filter's window spectrum) and roots (k_conv_ols)
     const float2 *tw_ols[2] = {nullptr, nullptr};
     const float2 *tw_ols_roots[2] = {nullptr, nullptr};
 };

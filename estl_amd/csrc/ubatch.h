@@ -31,7 +31,7 @@ struct UItem {
 
 // Device tables of every size class.
 struct UTables {
-    // power tables (block_fft kTwPowers) of BlockGeom<log2>, log2 0..kUMaxSmallLog2: the
+    // power tables of BlockGeom<log2>, log2 0..kUMaxSmallLog2: the
     // small transforms and the radices of the large ones' passes
     const float2 *pow[kUMaxSmallLog2 + 1];
     // W_B^m, m < B = 2^log2, of the first passes in k_pass_wide's form, and the one entry

@@ -31,7 +31,7 @@ template <int L>
 struct USmall {
     using G = BlockGeom<L>;
     static constexpr int TPW = kUThreads / G::TPT;
-    static constexpr int slice = G::uses_lds ? Lds<kLdsPad>::size(G::N) : 0;
+    static constexpr int slice = G::uses_lds ? Lds::size(G::N) : 0;
     static constexpr int lds = TPW * slice;
 };
 // Transforms of 2^17 values and more keep 32 values per thread (wide_tile, tiles of 2^14
@@ -86,7 +86,7 @@ __device__ __forceinline__ void small_item(const UArgs &a, const UItem &it, floa
     const float2 *src = a.in + off + tl;
 #pragma unroll
     for (int i = 0; i < E; ++i) v[i] = ld_stream(src + TPT * i);
-    block_fft<L, DIR, kLdsPad, false, kTwPowers>(v, lds + w * USmall<L>::slice, tl, a.tw.pow[L], true);
+    block_fft<L, DIR>(v, lds + w * USmall<L>::slice, tl, a.tw.pow[L], true);
     if (active) {
         float2 *dst = a.out + off + tl;
 #pragma unroll
