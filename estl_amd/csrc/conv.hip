@@ -27,10 +27,10 @@
 
 namespace estl {
 
-// sum |h_t| over k filter taps by the first 256 threads of a workgroup in a fixed
-// summation order (thread t adds taps t, t + 256, ...; then a tree over the 256
-// partial sums), so every caller gets the same value; every thread of the workgroup
-// must call it (it holds barriers); the result is valid in every thread.
+// sum |h_t| over k filter taps by the first 256 threads of a workgroup, in the summation
+// order of filter_l1 (thread t adds taps t, t + 256, ...; then a tree over the 256 partial
+// sums), so every caller gets the same value; every thread of the workgroup must call it
+// (it holds barriers); the result is valid in every thread.  `part` holds 257 floats.
 __device__ __forceinline__ float filter_l1_256(const float *__restrict__ h, long k, float *part) {
     if (threadIdx.x < 256) {
         float acc = 0.0f;
@@ -39,11 +39,15 @@ __device__ __forceinline__ float filter_l1_256(const float *__restrict__ h, long
         part[threadIdx.x] = acc;
     }
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) part[threadIdx.x] += part[threadIdx.x + s];
-        __syncthreads();
+    if (threadIdx.x < 64) {  // the first wave takes the tree, in registers after two levels
+        const int t = threadIdx.x;
+        float acc = (part[t] + part[t + 128]) + (part[t + 64] + part[t + 192]);
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) acc += __shfl_down(acc, s);
+        if (t == 0) part[256] = acc;
     }
-    return part[0];
+    __syncthreads();
+    return part[256];
 }
 
 // spectrum /= Re spectrum[0] (the kernel sum), read from a copy `dc` taken beforehand
@@ -66,23 +70,30 @@ __device__ __forceinline__ int conv_group_member(const ConvGroup *g, long pair) 
     return q;
 }
 
-// The spectrum of a filter of length n <= 2^13 in one workgroup: fold the taps on
-// load, forward FFT (the rows kernel's block_fft and table, so the bins are those of the
-// rows plan), optionally divide by the kernel sum Re K^[0] (Convolution.h:141), store.
-// With a request group, workgroup q builds member q's filter into its spectrum, divided
-// by the member's L (group->l1[q].x) for FP16 storage when divide_l1 is set.  With
-// normalisation the kernel sum K^[0] is also written to dc (the FP16 L1 bound divides
-// by it).
+// The threads of a filter's spectrum: those of wave_fft from 2^10 values, whose order of bins
+// k_conv_wave and k_conv_ols read, of block_fft and in natural order below.
 template <int LOG2N>
-__global__ void __launch_bounds__(BlockGeom<LOG2N>::TPT)
+constexpr int kSpecThreads = LOG2N >= kWaveMinLog2 ? (1 << LOG2N) / 32 : BlockGeom<LOG2N>::TPT;
+
+// The spectrum of a filter of length n <= 2^13 (or a window of 2^14 values) in one workgroup:
+// fold the taps on load, forward FFT, optionally divide by the kernel sum Re K^[0]
+// (Convolution.h:141), store.  With a request group, workgroup q builds member q's filter
+// into its spectrum, divided by the member's L (group->l1[q].x) for FP16 storage when
+// divide_l1 is set.  With normalisation the kernel sum K^[0] is also written to dc (the FP16
+// L1 bound divides by it).
+// Bound by its latency (one workgroup): taps, exchanges and barriers in a row.  With 16
+// values per thread, an exchange more across the workgroup and one to the convolutions'
+// order of bins, a 2^14 spectrum took 10.0 us per set_filter where this one takes 8.2, and 12.0
+// against 9.7 with the L1 norm (FP16 storage), which was summed after the transform.
+template <int LOG2N>
+__global__ void __launch_bounds__(kSpecThreads<LOG2N>)
 k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__restrict__ spec,
                   const float2 *__restrict__ tw, int normalize, const ConvGroup *__restrict__ group, int divide_l1,
                   float2 *__restrict__ dc, float2 *__restrict__ l1_single) {
-    using G = BlockGeom<LOG2N>;
-    constexpr int N = G::N, E = G::E, TPT = G::TPT;
-    __shared__ float2 lds[G::uses_lds ? Lds::size(N) : 1];
+    constexpr bool wave = LOG2N >= kWaveMinLog2;
+    constexpr int N = 1 << LOG2N, TPT = kSpecThreads<LOG2N>, E = N / TPT;
     __shared__ float s_dc;
-    __shared__ float s_part[TPT >= 256 ? 256 : 1];
+    __shared__ float s_part[LOG2N >= kOlsLog2 ? 257 : 1];
     const int tl = opaque_lane(threadIdx.x);
     if (group) {
         const int q = blockIdx.x;
@@ -103,7 +114,18 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
 #pragma unroll
         for (int i = 0; i < E; ++i) v[i] = make_float2(fold_tap(h, k, N, shift, tl + TPT * i), 0.0f);
     }
-    block_fft<LOG2N, -1>(v, lds, tl, tw, false);
+    [[maybe_unused]] float l1 = 0.0f;
+    if constexpr (LOG2N >= kOlsLog2) {
+        // the taps are on their way; their sum meanwhile
+        if (l1_single) l1 = filter_l1_256(h, k, s_part);
+    }
+    if constexpr (wave) {
+        __shared__ float lds[WaveGeom<LOG2N>::lds_floats];
+        wave_fft<LOG2N>(v, lds, tl, tw, false);
+    } else {
+        __shared__ float2 lds[BlockGeom<LOG2N>::uses_lds ? Lds::size(N) : 1];
+        block_fft<LOG2N, -1>(v, lds, tl, tw, false);
+    }
     if (normalize) {
         if (tl == 0) {
             s_dc = v[0].x;  // bin 0
@@ -119,12 +141,11 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
 #pragma unroll
         for (int i = 0; i < E; ++i) v[i] = make_float2(v[i].x * s, v[i].y * s);
     }
-    if constexpr (TPT >= 256) {
-        if (!group && l1_single) {
+    if constexpr (LOG2N >= kOlsLog2) {
+        if (l1_single) {
             // FP16 storage, one filter: L = sum |h| (divided by |kernel sum| when
             // normalised), the spectrum times 1 / L, and (L, sum |h|) after it -- the
             // values of k_filter_l1 then k_spec_l1, in one launch
-            const float l1 = filter_l1_256(h, k, s_part);
             float L = l1;
             if (normalize) L /= fabsf(s_dc);
             if (!(L > 0.0f)) L = 1.0f;
@@ -134,36 +155,22 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
             if (tl == 0) *l1_single = make_float2(L, l1);
         }
     }
-    if constexpr (LOG2N >= kWaveMinLog2) {
-        // bins to the order k_conv_rows and k_conv_ols of this length read them in
-        using P = Lds;
-        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < E; ++i) lds[P::idx(tl + TPT * i)] = v[i];
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const int pos = tl + TPT * i;
-            spec[pos] = lds[P::idx(wave_bin<LOG2N>(pos))];
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < E; ++i) spec[tl + TPT * i] = v[i];
-    }
+    for (int i = 0; i < E; ++i) spec[tl + TPT * i] = v[i];
 }
 
-// l1_single (one filter, FP16 storage, N >= 2^12): the spectrum divided by its L and
+// l1_single (one filter, FP16 storage, a window's spectrum): the spectrum divided by its L and
 // (L, sum |h|) stored there, in place of launch_conv_fp16_filter's two launches
 hipError_t launch_filter_spectrum(int log2n, const float *h, long k, long shift, float2 *spec, const float2 *tw,
                                   bool normalize, hipStream_t st, const ConvGroup *group, int members,
                                   bool divide_l1, float2 *dc, float2 *l1_single) {
     if (group && (members < 1 || members > kGroupMax || normalize)) return hipErrorInvalidValue;
-    if (l1_single && (group || log2n < 12)) return hipErrorInvalidValue;
+    if (l1_single && (group || log2n < kOlsLog2)) return hipErrorInvalidValue;
     const unsigned blocks = group ? (unsigned)members : 1u;
     switch (log2n) {
 #define FS(L)                                                                                                   \
     case L:                                                                                                     \
-        hipLaunchKernelGGL(k_filter_spectrum<L>, dim3(blocks), dim3(BlockGeom<L>::TPT), 0, st, h, k, shift, spec, \
+        hipLaunchKernelGGL(k_filter_spectrum<L>, dim3(blocks), dim3(kSpecThreads<L>), 0, st, h, k, shift, spec, \
                            tw, normalize ? 1 : 0, group, divide_l1 ? 1 : 0, dc, l1_single);                      \
         break;
         FS(1) FS(2) FS(3) FS(4) FS(5) FS(6) FS(7) FS(8) FS(9) FS(10) FS(11) FS(12) FS(13) FS(14)

@@ -161,8 +161,6 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
         s0.args.io_in = 3;
     } else if (c->spec_plan.kind != Plan::ROWS) {
         return set_error(ESTL_ERR_UNSUPPORTED, "convolution of n=%ld: no spectrum plan", n);
-    } else {
-        c->tw_spec = c->spec_plan.tw_rows;  // k_filter_spectrum's table: the rows plan's powers
     }
     if (c->log2n <= kMaxRowsLog2) {
         c->fused = true;
@@ -172,8 +170,7 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
     }
     for (int w = 0; w < 2; ++w) {
         if (c->log2n <= kOlsLog2 + w) break;
-        if ((rc = power_table(current_device(), kOlsLog2 + w, &c->tw_ols[w]))) return rc;
-        if ((rc = wave_table(current_device(), kOlsLog2 + w, &c->tw_ols_roots[w]))) return rc;
+        if ((rc = wave_table(current_device(), kOlsLog2 + w, &c->tw_ols[w]))) return rc;
     }
     // forward passes with the default split; the inverse runs the radices in the reverse
     // order, so the last forward pass and the first inverse pass cover the same columns
@@ -249,7 +246,7 @@ int conv_filter(const ConvShape &c, const ConvBuffers &b, const float *h, long k
     }
     if (c.spec_plan.kind == Plan::ROWS) {
         // fold, transform and normalise in one launch (the kernel sum to b.dc)
-        e = launch_filter_spectrum(c.log2n, h, k, shift, b.spec, c.tw_spec, normalize, st, nullptr, 0,
+        e = launch_filter_spectrum(c.log2n, h, k, shift, b.spec, c.tw_rows, normalize, st, nullptr, 0,
                                    false, b.dc);
         if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "filter spectrum launch: %s", hipGetErrorString(e));
     } else {
@@ -352,10 +349,10 @@ static int conv_run_ols(const ConvShape &c, const ConvBuffers &b, const void *x,
     // result moves back by the shift, a correlation's forward
     const long oshift = c.corr ? shift : -shift;
     const int lw = b.ols;
-    if (lw != kOlsLog2 && !(lw == kOlsWideLog2 && c.tw_ols_roots[1]))
+    if (lw != kOlsLog2 && !(lw == kOlsWideLog2 && c.tw_ols[1]))
         return set_error(ESTL_ERR_INVALID, "no overlap-save window of 2^%d values for n=%ld", lw, c.n);
     hipError_t e = launch_conv_ols(fp16, c.corr, lw, x, y, c.rows, c.log2n, b.k, oshift, b.spec,
-                                   c.tw_ols_roots[lw - kOlsLog2], s_in, s_out, st);
+                                   c.tw_ols[lw - kOlsLog2], s_in, s_out, st);
     if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "k_conv_ols launch: %s", hipGetErrorString(e));
     return ESTL_OK;
 }
@@ -381,7 +378,7 @@ int conv_run(const ConvShape &c, const ConvBuffers &b, const float *x, float *y,
 int conv_filter_group_rows(const ConvShape &c, const ConvGroup *d_group, int members, bool divide_l1,
                            hipStream_t st) {
     if (!c.fused || c.spec_plan.kind != Plan::ROWS) return set_error(ESTL_ERR_INVALID, "not a fused shape");
-    hipError_t e = launch_filter_spectrum(c.log2n, nullptr, 0, 0, nullptr, c.tw_spec, false, st, d_group,
+    hipError_t e = launch_filter_spectrum(c.log2n, nullptr, 0, 0, nullptr, c.tw_rows, false, st, d_group,
                                           members, divide_l1);
     if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group filter spectra: %s", hipGetErrorString(e));
     return ESTL_OK;

@@ -51,8 +51,7 @@ struct BlockGeom {
 // A_q, 68 KiB at 2^14, mostly cache-resident), w^2 and w^8 by squaring, the twiddles of
 // each level of the DFT from them (dft_twiddled).  A table of every W_{N_q}^{g s} (128 KiB
 // at 2^14, B_q - 1 reads per butterfly) held in registers across rows needed 167-206 VGPRs
-// and was 6-9 % slower at 4096 and 8192 points, and read again for each row slower still;
-// the filter spectra of 2^14 and binary16 storage took 15.8 us with it, 12.0 with powers.
+// and was 6-9 % slower at 4096 and 8192 points, and read again for each row slower still.
 // Rel-L2 against FP64 is 1.6e-7 at 4096 points (the bound is 1.2e-5): 3.0e-7 when every
 // power came from w alone, 1.2e-7 with that table's rounded values.
 

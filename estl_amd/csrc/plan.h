@@ -115,10 +115,9 @@ struct ConvShape {
     unsigned flags = 0;
     bool corr = false, fused = false;
     float scale = 1.0f;
-    const float2 *tw_rows = nullptr;  // table of the fused rows kernel (n <= 2^13): roots from
-                                      // 2^10 values (k_conv_wave), the power table below
+    const float2 *tw_rows = nullptr;  // table of the fused rows kernel and the filter's spectrum
+                                      // (n <= 2^13): roots from 2^10 values, powers below
     Plan spec_plan;                  // forward FFT of the folded filter (batch 1)
-    const float2 *tw_spec = nullptr;  // k_filter_spectrum's table when spec_plan is a rows plan
     std::vector<PassStep> fwd, inv;  // multi-pass pipeline (n > 2^13): fwd, mid, inv
     PassStep mid{};                  // last forward + multiply + first inverse pass
     size_t scratch_bytes = 0;        // bytes of each of the two scratch buffers
@@ -128,10 +127,8 @@ struct ConvShape {
     // k_conv_half_merge, taken when the row's input and output are 8-byte aligned
     bool half = false;
     Plan half_fwd, half_inv;
-    // tables of the overlap-save windows of 2^13 (n > 2^13) and 2^14 (n > 2^14) values:
-    // power tables (the filter's window spectrum) and roots (k_conv_ols)
+    // roots of the overlap-save windows of 2^13 (n > 2^13) and 2^14 (n > 2^14) values
     const float2 *tw_ols[2] = {nullptr, nullptr};
-    const float2 *tw_ols_roots[2] = {nullptr, nullptr};
 };
 bool conv_half_path(long n, long rows, int precision);
 // Rows longer than an overlap-save window convolved with a filter of at most
