@@ -93,6 +93,36 @@ hipError_t launch_stream_copy(const void *src, void *dst, long n16, bool nontemp
     return hipGetLastError();
 }
 
+// A served output's copy as the streaming copy's kernel instead of the runtime's, whose copies
+// of 8-32 MiB outlast the host's calls for them: a burst of 24 requests of up to 32 MiB, each
+// output copied out, 990-1039 -> 884-977 us.  Smaller ones are hidden behind the host either
+// way (15 requests of up to 4 MiB: 470-630 us both) and stay with the runtime, which needs
+// none of the queries below.  Taken from kOutputCopyMin for whole 16-byte
+// values on 16-byte boundaries between buffers of `device`, with the stream and the caller
+// on it, and only inside dst's allocation; *queued stays false otherwise (host or managed
+// memory, another device's, odd sizes), and the caller leaves it to the runtime.
+constexpr size_t kOutputCopyMin = size_t(8) << 20;
+hipError_t launch_output_copy(const void *src, void *dst, size_t bytes, int device, hipStream_t st, bool *queued) {
+    *queued = false;
+    if (bytes < kOutputCopyMin || bytes % 16 || (uintptr_t)src % 16 || (uintptr_t)dst % 16) return hipSuccess;
+    int on = -1;
+    if (hipGetDevice(&on) != hipSuccess || on != device) return hipSuccess;
+    hipDevice_t on_stream = device;
+    if (st && (hipStreamGetDevice(st, &on_stream) != hipSuccess || on_stream != device)) return hipSuccess;
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, dst) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != device ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)dst) != hipSuccess ||
+        (uintptr_t)dst + bytes > (uintptr_t)base + size) {
+        (void)hipGetLastError();  // a query's error is not the copy's
+        return hipSuccess;
+    }
+    const hipError_t e = launch_stream_copy(src, dst, (long)(bytes / 16), true, st);
+    *queued = e == hipSuccess;
+    return e;
+}
+
 // ------------------------------------------------------------------ batched rows
 // Rows of N <= 2^13 points: a group of TPW = max(1, 256 / TPT) rows, one per TPT = N/16
 // threads (16 values per thread), per workgroup, and one workgroup per group -- the

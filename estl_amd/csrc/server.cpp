@@ -62,6 +62,10 @@
 
 namespace estl {
 
+// kernels.hip; weak, as this file is also built without device code (the runtime then copies)
+__attribute__((weak)) hipError_t launch_output_copy(const void *src, void *dst, size_t bytes, int device,
+                                                    hipStream_t st, bool *queued);
+
 using Clock = std::chrono::steady_clock;
 
 // First-fit allocator over one device allocation (offsets aligned to 256 bytes).
@@ -356,7 +360,11 @@ class Server {
         // block out of the arena until it has run, whenever the request is released
         hipEvent_t done = nullptr;
         if (int rc = get_event(&done)) return rc;
-        if (hipMemcpyAsync(dst, r.out, (size_t)bytes, hipMemcpyDeviceToDevice, st) != hipSuccess) {
+        bool queued = false;
+        hipError_t e = hipSuccess;
+        if (launch_output_copy) e = launch_output_copy(r.out, dst, (size_t)bytes, device_, st, &queued);
+        if (e == hipSuccess && !queued) e = hipMemcpyAsync(dst, r.out, (size_t)bytes, hipMemcpyDeviceToDevice, st);
+        if (e != hipSuccess) {
             put_event(done);
             return set_error(ESTL_ERR_HIP, "output copy failed");
         }
