@@ -236,8 +236,10 @@ int finish_pass(PassStep *s, int device, bool tiled, bool fp16) {
 }
 
 // The passes of a plan of `batch` rows.  Up to 2^18 values two passes; 2^19 and 2^20 two of
-// radices 2^9 and 2^10 where k_pass_wide fills the device (2^20 x 33: 300 us in three
-// passes, 210 in two; a single 2^20 is 10 % faster in three), then as few as radices of 2^9
+// radices 2^9 and 2^10 where k_pass_wide has tiles enough: in FP32 from 2^21 values (2^20 x 33:
+// 300 us in three passes, 210 in two; 2^20 x 2 23.1 and 21.9, 2^19 x 4 23.2 and 21.2; below, 2^19
+// x 3 19.6 and 21.1, 2^20 x 1 19.7 and 21.1), in FP16 from two rows (2^19 x 2 16.9 and 14.6, x 3
+// 18.4 and 16.0); buffers new with each call, then as few as radices of 2^9
 // allow, evenly split, smaller ones first (a first pass has no pre-twiddles).  A last pass
 // of radix 2^9 reads runs of 16 values per column where smaller ones read 8 or less, which
 // counts where a value is 4 bytes (binary16 2^16 x 300: 75 us as 2^8 2^8, 65 as 2^7 2^9;
@@ -245,7 +247,7 @@ int finish_pass(PassStep *s, int device, bool tiled, bool fp16) {
 // 186 -> 177 us).
 static std::vector<int> plan_pass_split(int log2n, long batch, bool fp16) {
     const long values = batch << log2n;
-    if ((log2n == 19 || log2n == 20) && batch > 1) return {log2n - 10, 10};
+    if ((log2n == 19 || log2n == 20) && (fp16 ? batch > 1 : values >= (1L << 21))) return {log2n - 10, 10};
     const int P = std::max(2, (log2n + 8) / 9);
     const bool last9 = fp16 ? P <= 3 && values >= (1L << 20) : P == 2 && log2n >= 15 && values >= (1L << 23);
     if (!last9 || (log2n - 9 + P - 2) / (P - 1) > 9) return conv_pass_split(log2n);

@@ -39,7 +39,7 @@ def sizes(split):
 def test_fp32(gpu, split, tiles, direction):
     import torch
     for n in sizes(split):
-        for batch, in_place in ((1, False), (3, True)):
+        for batch, in_place in ((1, False), (3, True), (4, False)):
             x = torch.empty(batch, n, dtype=torch.complex64, device=gpu)
             estl_amd.fill_uniform(x, 95)
             want = oracle.fft64(x.cpu().numpy(), direction)
