@@ -480,14 +480,36 @@ struct OlsArgs {
     int pre;      // first valid position in a window
 };
 
+// `count` outputs at p (uniform across the wave) as a raw buffer, which drops stores at other
+// offsets: no lane test and no branch where a window's valid outputs begin and end.
+template <typename R>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t out_piece(R *p, int count) {
+    return __builtin_amdgcn_make_buffer_rsrc(p, 0, count * (int)sizeof(R), 4 << 15 /* 32-bit data */);
+}
+// Output i + step; the sum is formed before it becomes a byte offset (opaque), where the
+// compiler would put a part of it into the instruction's own offset, added to an i below 0.
+template <typename R>
+__device__ __forceinline__ void st_piece(__amdgpu_buffer_rsrc_t piece, int i, int step, float v) {
+    const int at = opaque_lane((i + step) * (int)sizeof(R));
+    if constexpr (sizeof(R) == 4) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), piece, at, 0, 2 /* nontemporal */);
+    } else {
+        const _Float16 h = (_Float16)v;
+        unsigned short u;
+        __builtin_memcpy(&u, &h, 2);
+        __builtin_amdgcn_raw_buffer_store_b16(u, piece, at, 0, 0);
+    }
+}
+
 // One workgroup per pair of windows, 32 values per thread, at most 128 VGPRs and 33 / 66
 // KiB of LDS: four waves per SIMD, four workgroups per CU at L = 2^13 and two at 2^14, so
-// one's loads and stores overlap another's arithmetic.  Bound by the vector instructions
-// (~92 per complex value and two transforms; 16 values per thread took ~148, with twelve
-// barriers a window pair instead of seven), which keep the SIMDs 96 % busy while four
-// waves each are resident, at a clock that power holds to 2.0-2.3 GHz; the rest is the last
-// round.  63 rows of 2^20 values and 2049 taps (2^13 windows): 201 -> 147 us; 101 binary16
-// rows of 2^18 and 6001 taps (2^14), spectrum included: 153 -> 94 us.
+// one's loads and stores overlap another's arithmetic.  Bound by the vector instructions,
+// at a clock that power holds to 2.0-2.3 GHz, then by the last round of workgroups; a call of
+// a few windows by one wave's chain of them.  Nothing is spilled, and the stores have no
+// lane tests: with 24 bytes of scratch and a branch per store a call took 14.5 us for one row of
+// 2^14 values (12.7 with 16 values per thread), 11.1 without; 63 rows of 2^20 and 2049
+// taps (2^13 windows) 146 -> 135 us (201), 101 binary16 rows of 2^18 and 6001 taps (2^14) 74 -> 66
+// (122).
 template <int LOG2L, bool CORR, typename R>
 __global__ void __launch_bounds__(WaveGeom<LOG2L>::T) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *__restrict__ spec,
@@ -500,7 +522,7 @@ k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *
         // FP16 storage: the output row scales, s_in times L (the value after the
         // spectrum's L bins), as k_conv_scales computes them
         const float l1 = spec[(size_t)L].x;
-        for (long r = t; r < a.rows; r += T) a.s_out[r] = a.s_in[r] * l1;
+        for (unsigned r = t; r < (unsigned)a.rows; r += T) a.s_out[r] = a.s_in[r] * l1;
     }
     // rows and windows in scalar registers, offsets inside a row in 32 bits (n <= 2^30):
     // loads and stores take a scalar base and a 32-bit lane offset
@@ -535,34 +557,27 @@ k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *
     wave_fft<LOG2L>(v, lds, t, tw, false);
     multiply_spectrum<CORR, T>(v, spec, t);
     wave_ifft<LOG2L>(v, lds, t, tw);
-    const int osh = (int)a.oshift;
+    // both windows' outputs before the first is stored: the compiler would otherwise move
+    // the second's last butterflies past the branch, and spill
+#pragma unroll
+    for (int e = 0; e < 32; ++e) asm volatile("" : "+v"(v[e].x), "+v"(v[e].y));
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
         if (half && !two) break;
         const int m = half ? m1 : m0;
-        R *yr = half ? y1 : y0;
+        int to = m + (int)a.oshift;  // where its first output goes
+        if (to >= n) to -= n;
         const int live = n - m < a.M ? n - m : a.M;  // outputs of this window
-        if (m + osh + live <= n || m + osh >= n) {
-            // no output wraps: a scalar base, and a lane test only where the valid part ends
-            R *base = yr + (m + osh >= n ? m + osh - n : m + osh) - a.pre;
+        // one piece, two where the rotation carries it past the row's end
+#pragma unroll 1
+        for (int q = 0; q < live;) {
+            const int count = live - q < n - to ? live - q : n - to;
+            const auto piece = out_piece((half ? y1 : y0) + to, count);
 #pragma unroll
-            for (int e = 0; e < 32; ++e) {
-                const int lo = T * e;
-                if (lo + T <= a.pre || lo >= a.pre + live) continue;
-                const float o = (half ? v[e].y : v[e].x) * scale;
-                if (lo >= a.pre && lo + T <= a.pre + live) {
-                    st_real(base + lo + t, o);
-                } else if (lo + t >= a.pre && lo + t < a.pre + live) {
-                    st_real(base + lo + t, o);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 32; ++e) {
-                const int q = t + T * e - a.pre;  // position in the window's valid outputs
-                if (q >= 0 && q < live)
-                    st_real(yr + ((unsigned)(m + q + osh) & nm), (half ? v[e].y : v[e].x) * scale);
-            }
+            for (int e = 0; e < 32; ++e)
+                st_piece<R>(piece, t - (a.pre + q), T * e, (half ? v[e].y : v[e].x) * scale);
+            q += count;
+            to = 0;
         }
     }
 }
