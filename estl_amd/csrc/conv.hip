@@ -187,16 +187,26 @@ __device__ __forceinline__ void st_real(float *p, float v) { st_stream_f(p, v); 
 __device__ __forceinline__ void st_real(_Float16 *p, float v) { *p = (_Float16)v; }
 
 // v[r] times bin r T + t of a spectrum (its conjugate with CORR), eight bins in flight at a
-// time: the compiler's schedule has all 32 and spills for them.
-template <bool CORR, int T>
+// time, or with AHEAD the next eight already on their way while these are used (where that
+// spills nothing: at 2^10 and 2^12 values it does): the compiler's schedule has all 32 and
+// spills for them.
+template <bool CORR, int T, bool AHEAD>
 __device__ __forceinline__ void multiply_spectrum(float2 (&v)[32], const float2 *__restrict__ spec, int t) {
+    float2 h[2][8];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) h[c / 8 % 2][r] = spec[t + T * (c + r)];
+    };
+    if constexpr (AHEAD) load(0);
 #pragma unroll
     for (int c = 0; c < 32; c += 8) {
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!AHEAD) load(c);
+        else if (c < 24) load(c + 8);
 #pragma unroll
-        for (int r = c; r < c + 8; ++r) {
-            const float2 hk = spec[t + T * r];
-            v[r] = CORR ? cmulc(v[r], hk) : cmul(v[r], hk);
+        for (int r = 0; r < 8; ++r) {
+            const float2 hk = h[c / 8 % 2][r];
+            v[c + r] = CORR ? cmulc(v[c + r], hk) : cmul(v[c + r], hk);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -242,7 +252,7 @@ k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
     for (int i = 0; i < 32; ++i) v[i] = make_float2(ld_real(x1 + T * i), ld_real(x2 + T * i));
     float *slice = lds + w * G::lds_floats;
     wave_fft<LOG2N>(v, slice, t, tw, false);
-    multiply_spectrum<CORR, T>(v, spec, t);
+    multiply_spectrum<CORR, T, LOG2N == 11 || LOG2N == 13>(v, spec, t);
     wave_ifft<LOG2N>(v, slice, t, tw);
     if (active) {
         R *y1 = global_ptr(y) + r1 * N + t;
@@ -555,7 +565,7 @@ k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *
         for (int e = 0; e < 32; ++e) v[e].y = ld_real(x1 + ((unsigned)(s1 + t + T * e) & nm));
     }
     wave_fft<LOG2L>(v, lds, t, tw, false);
-    multiply_spectrum<CORR, T>(v, spec, t);
+    multiply_spectrum<CORR, T, true>(v, spec, t);
     wave_ifft<LOG2L>(v, lds, t, tw);
     // both windows' outputs before the first is stored: the compiler would otherwise move
     // the second's last butterflies past the branch, and spill

@@ -80,31 +80,43 @@ struct WaveRoots {
     static constexpr int size = point + 3 * WaveGeom<LOG2N>::T;
 };
 
-// In-place DFT of v[i] w^i (conjugated for DIR > 0), i < 32; w, w^4, w^16 at roots[t],
-// [STRIDE + t], [2 STRIDE + t].
-template <int DIR, int STRIDE>
-__device__ __forceinline__ void dft32_rooted(float2 (&v)[32], const float2 *__restrict__ roots, int t) {
+// w, w^4, w^16 of a 32-point step: at roots[t], [STRIDE + t], [2 STRIDE + t].  A step's roots
+// are loaded before the exchange ahead of it, which needs few registers, and arrive
+// meanwhile: loaded where they are used, each step of a lone wave waited for the L2 (a call of
+// one row of 2^14 values 11.1 -> 10.6 us, 1000 rows of 2^11 8.9 -> 8.25, 63 rows of 2^20 at 4097
+// taps 154 -> 145).
+struct Roots32 {
+    float2 w1, w4, w16;
+};
+template <int STRIDE>
+__device__ __forceinline__ Roots32 load_roots(const float2 *__restrict__ roots, int t) {
     // read anew at each use: kept from one use to the next their powers would take
     // tens of registers
     const float2 *q = opaque(roots);
-    float2 p[5];
-    p[0] = q[t];
-    p[2] = q[STRIDE + t];
-    p[4] = q[2 * STRIDE + t];
-    p[1] = csquare(p[0]);
-    p[3] = csquare(p[2]);
+    return {q[t], q[STRIDE + t], q[2 * STRIDE + t]};
+}
+
+// In-place DFT of v[i] w^i (conjugated for DIR > 0), i < 32.
+template <int DIR>
+__device__ __forceinline__ void dft32_rooted(float2 (&v)[32], const Roots32 &w) {
+    const float2 p[5] = {w.w1, csquare(w.w1), w.w4, csquare(w.w4), w.w16};
     const LevelTw<32> tw(p);
     dft_dit<32, DIR, true>(v, tw.t);
 }
 
-// The same for x[i] w^i, i < Q <= 16; w and w^4 at roots[t] and [1024 + t].
+// w and w^4 (Q > 4 only) of a Q-point step, at roots[t] and [1024 + t].
+struct RootsQ {
+    float2 w1, w4;
+};
+
+// In-place DFT of x[i] w^i, i < Q <= 16.
 template <int Q, int DIR>
-__device__ __forceinline__ void dft_rooted(float2 *x, const float2 *__restrict__ roots, int t) {
+__device__ __forceinline__ void dft_rooted(float2 *x, const RootsQ &w) {
     constexpr int LQ = __builtin_ctz(Q);
     float2 p[4], y[Q];
-    p[0] = roots[t];
+    p[0] = w.w1;
     p[1] = csquare(p[0]);
-    if constexpr (LQ > 2) p[2] = roots[1024 + t];
+    if constexpr (LQ > 2) p[2] = w.w4;
     if constexpr (LQ > 3) p[3] = csquare(p[2]);
     const LevelTw<Q> tw(p);
     StaticFor<0, Q>::run([&](auto ic) { y[decltype(ic)::value] = x[decltype(ic)::value]; });
@@ -123,6 +135,7 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
     const int tq = t % Q;
     using W = WaveRoots<LOG2N>;
     Dft<32, -1>::run(v);
+    const Roots32 wr = load_roots<32>(tw + W::row, t / Q);
     if (lds_busy) exchange_sync<G::in_wave>();
 #pragma unroll
     for (int k = 0; k < 32; ++k) lds[k * RS + t] = v[k].x;
@@ -135,8 +148,15 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
     exchange_sync<G::in_wave>();
 #pragma unroll
     for (int i = 0; i < 32; ++i) v[i].y = row[tq + Q * i];
-    dft32_rooted<-1, 32>(v, tw + W::row, t / Q);
+    dft32_rooted<-1>(v, wr);
     if constexpr (Q > 1) {
+        RootsQ wb[32 / Q];
+        const float2 *bin = opaque(tw + W::bin);
+#pragma unroll
+        for (int m = 0; m < 32 / Q; ++m) {
+            wb[m].w1 = bin[T * m + t];
+            if constexpr (Q > 4) wb[m].w4 = bin[1024 + T * m + t];
+        }
         wave_lds_fence();
 #pragma unroll
         for (int k = 0; k < 32; ++k) row[k * Q + (k * Q >> 5) + tq] = v[k].x;
@@ -151,7 +171,7 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
         for (int r = 0; r < 32; ++r) v[r].y = row[33 * tq + r];
         StaticFor<0, 32 / Q>::run([&](auto mc) {
             constexpr int m = decltype(mc)::value;
-            dft_rooted<Q, -1>(v + Q * m, tw + W::bin + T * m, t);
+            dft_rooted<Q, -1>(v + Q * m, wb[m]);
         });
     }
 }
@@ -166,6 +186,7 @@ __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, co
     float *row = lds + (t / Q) * RS;
     const int tq = t % Q;
     if constexpr (Q > 1) {
+        const Roots32 wp = load_roots<Q>(tw + W::pos, tq);
         StaticFor<0, 32 / Q>::run([&](auto mc) { Dft<Q, +1>::run(v + Q * decltype(mc)::value); });
         wave_lds_fence();
 #pragma unroll
@@ -179,10 +200,11 @@ __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, co
         wave_lds_fence();
 #pragma unroll
         for (int k = 0; k < 32; ++k) v[k].y = row[k * Q + (k * Q >> 5) + tq];
-        dft32_rooted<+1, Q>(v, tw + W::pos, tq);
+        dft32_rooted<+1>(v, wp);
     } else {
         Dft<32, +1>::run(v);
     }
+    const Roots32 wn = load_roots<T>(tw + W::point, t);
     wave_lds_fence();
 #pragma unroll
     for (int i = 0; i < 32; ++i) row[tq + Q * i] = v[i].x;
@@ -195,7 +217,7 @@ __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, co
     exchange_sync<G::in_wave>();
 #pragma unroll
     for (int k = 0; k < 32; ++k) v[k].y = lds[k * RS + t];
-    dft32_rooted<+1, T>(v, tw + W::point, t);
+    dft32_rooted<+1>(v, wn);
 }
 
 }  // namespace estl
