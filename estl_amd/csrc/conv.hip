@@ -70,10 +70,10 @@ __device__ __forceinline__ int conv_group_member(const ConvGroup *g, long pair) 
     return q;
 }
 
-// The threads of a filter's spectrum: those of wave_fft from 2^10 values, whose order of bins
-// k_conv_wave and k_conv_ols read, of block_fft and in natural order below.
-template <int LOG2N>
-constexpr int kSpecThreads = LOG2N >= kWaveMinLog2 ? (1 << LOG2N) / 32 : BlockGeom<LOG2N>::TPT;
+// The threads of a filter's spectrum: those of wave_fft (WAVE), whose order of bins k_conv_wave
+// and k_conv_ols read, or of block_fft, in natural order for k_conv_rows.
+template <int LOG2N, bool WAVE>
+constexpr int kSpecThreads = WAVE ? (1 << LOG2N) / 32 : BlockGeom<LOG2N>::TPT;
 
 // The spectrum of a filter of length n <= 2^13 (or a window of 2^14 values) in one workgroup:
 // fold the taps on load, forward FFT, optionally divide by the kernel sum Re K^[0]
@@ -85,13 +85,12 @@ constexpr int kSpecThreads = LOG2N >= kWaveMinLog2 ? (1 << LOG2N) / 32 : BlockGe
 // values per thread, an exchange more across the workgroup and one to the convolutions'
 // order of bins, a 2^14 spectrum took 10.0 us per set_filter where this one takes 8.2, and 12.0
 // against 9.7 with the L1 norm (FP16 storage), which was summed after the transform.
-template <int LOG2N>
-__global__ void __launch_bounds__(kSpecThreads<LOG2N>)
+template <int LOG2N, bool WAVE>
+__global__ void __launch_bounds__((kSpecThreads<LOG2N, WAVE>))
 k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__restrict__ spec,
                   const float2 *__restrict__ tw, int normalize, const ConvGroup *__restrict__ group, int divide_l1,
                   float2 *__restrict__ dc, float2 *__restrict__ l1_single) {
-    constexpr bool wave = LOG2N >= kWaveMinLog2;
-    constexpr int N = 1 << LOG2N, TPT = kSpecThreads<LOG2N>, E = N / TPT;
+    constexpr int N = 1 << LOG2N, TPT = kSpecThreads<LOG2N, WAVE>, E = N / TPT;
     __shared__ float s_dc;
     __shared__ float s_part[LOG2N >= kOlsLog2 ? 257 : 1];
     const int tl = opaque_lane(threadIdx.x);
@@ -119,7 +118,7 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
         // the taps are on their way; their sum meanwhile
         if (l1_single) l1 = filter_l1_256(h, k, s_part);
     }
-    if constexpr (wave) {
+    if constexpr (WAVE) {
         __shared__ float lds[WaveGeom<LOG2N>::lds_floats];
         wave_fft<LOG2N>(v, lds, tl, tw, false);
     } else {
@@ -161,19 +160,20 @@ k_filter_spectrum(const float *__restrict__ h, long k, long shift, float2 *__res
 
 // l1_single (one filter, FP16 storage, a window's spectrum): the spectrum divided by its L and
 // (L, sum |h|) stored there, in place of launch_conv_fp16_filter's two launches
-hipError_t launch_filter_spectrum(int log2n, const float *h, long k, long shift, float2 *spec, const float2 *tw,
-                                  bool normalize, hipStream_t st, const ConvGroup *group, int members,
+hipError_t launch_filter_spectrum(int log2n, bool wave, const float *h, long k, long shift, float2 *spec,
+                                  const float2 *tw, bool normalize, hipStream_t st, const ConvGroup *group, int members,
                                   bool divide_l1, float2 *dc, float2 *l1_single) {
     if (group && (members < 1 || members > kGroupMax || normalize)) return hipErrorInvalidValue;
     if (l1_single && (group || log2n < kOlsLog2)) return hipErrorInvalidValue;
     const unsigned blocks = group ? (unsigned)members : 1u;
-    switch (log2n) {
-#define FS(L)                                                                                                   \
-    case L:                                                                                                     \
-        hipLaunchKernelGGL(k_filter_spectrum<L>, dim3(blocks), dim3(kSpecThreads<L>), 0, st, h, k, shift, spec, \
-                           tw, normalize ? 1 : 0, group, divide_l1 ? 1 : 0, dc, l1_single);                      \
+    switch (2 * log2n + (wave ? 1 : 0)) {
+#define FS(L, W)                                                                                            \
+    case 2 * L + W:                                                                                         \
+        hipLaunchKernelGGL((k_filter_spectrum<L, W != 0>), dim3(blocks), dim3(kSpecThreads<L, W != 0>), 0, st, h, k, \
+                           shift, spec, tw, normalize ? 1 : 0, group, divide_l1 ? 1 : 0, dc, l1_single);     \
         break;
-        FS(1) FS(2) FS(3) FS(4) FS(5) FS(6) FS(7) FS(8) FS(9) FS(10) FS(11) FS(12) FS(13) FS(14)
+        FS(1, 0) FS(2, 0) FS(3, 0) FS(4, 0) FS(5, 0) FS(6, 0) FS(7, 0) FS(8, 0) FS(9, 0) FS(12, 0)
+        FS(10, 1) FS(11, 1) FS(12, 1) FS(13, 1) FS(14, 1)
 #undef FS
         default: return hipErrorInvalidValue;
     }
@@ -212,7 +212,7 @@ __device__ __forceinline__ void multiply_spectrum(float2 (&v)[32], const float2 
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Pairs of real rows of N >= 2^10 values, TPW = max(1, 64 / T) pairs per workgroup (the
+// Pairs of real rows of N >= 2^10 values (conv_wave), TPW = max(1, 64 / T) pairs per workgroup (the
 // smallest ones are done and replaced soonest: 256-thread workgroups were 7 % slower at
 // 2^10 and 2^11 values and 2000 rows, 13 % at 2000 rows of 2^10) and one workgroup per group of pairs: forward transform, multiply, inverse transform in
 // registers (wave_fft), each value read and written once.  With a request group, `rows`
@@ -265,8 +265,8 @@ k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
     }
 }
 
-// The same for rows of N < 2^10 values (16 values per thread, bins in natural order),
-// persistent over the pairs (four resident rounds of workgroups).
+// The same for the other rows (16 values per thread, bins in natural order), persistent over
+// the pairs (four resident rounds of workgroups).
 template <int LOG2N, int TPW, bool CORR, typename R>
 __global__ void __launch_bounds__(BlockGeom<LOG2N>::TPT * TPW) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_rows(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 *__restrict__ spec,
@@ -647,7 +647,7 @@ hipError_t launch_conv_ols(bool fp16, bool corr, int log2L, const void *x, void 
 template <int LOG2N, bool CORR, typename R>
 static hipError_t launch_conv_rows_t(const R *x, R *y, long rows, const float2 *spec, const float2 *tw, float scale,
                                      hipStream_t st, const ConvGroup *group) {
-    if constexpr (LOG2N >= kWaveMinLog2) {
+    if constexpr (conv_wave(LOG2N, sizeof(R) == 2)) {
         using G = WaveGeom<LOG2N>;
         constexpr int TPW = (G::T >= 64) ? 1 : 64 / G::T;
         const long pairs = (rows + 1) / 2, groups = (pairs + TPW - 1) / TPW;

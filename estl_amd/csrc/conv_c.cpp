@@ -33,8 +33,8 @@ namespace estl {
 // (group: a request group's descriptor in device memory, or null)
 hipError_t launch_conv_rows(int log2n, bool corr, const float *x, float *y, long rows, const float2 *spec,
                             const float2 *tw, float scale, hipStream_t st, const ConvGroup *group = nullptr);
-hipError_t launch_filter_spectrum(int log2n, const float *h, long k, long shift, float2 *spec, const float2 *tw,
-                                  bool normalize, hipStream_t st, const ConvGroup *group = nullptr, int members = 0,
+hipError_t launch_filter_spectrum(int log2n, bool wave, const float *h, long k, long shift, float2 *spec,
+                                  const float2 *tw, bool normalize, hipStream_t st, const ConvGroup *group = nullptr, int members = 0,
                                   bool divide_l1 = false, float2 *dc = nullptr, float2 *l1_single = nullptr);
 hipError_t launch_spec_normalize(float2 *spec, long n, const float2 *dc, hipStream_t st);
 hipError_t launch_conv_rows_fp16(int log2n, bool corr, const void *x, void *y, long rows, const float2 *spec,
@@ -165,8 +165,9 @@ int conv_shape_init(ConvShape *c, long n, long rows, unsigned flags, int precisi
     if (c->log2n <= kMaxRowsLog2) {
         c->fused = true;
         c->scratch_bytes = 0;
-        return c->log2n >= kWaveMinLog2 ? wave_table(current_device(), c->log2n, &c->tw_rows)    // k_conv_wave
-                                        : power_table(current_device(), c->log2n, &c->tw_rows);  // k_conv_rows
+        c->wave = conv_wave(c->log2n, h);
+        return c->wave ? wave_table(current_device(), c->log2n, &c->tw_rows)    // k_conv_wave
+                       : power_table(current_device(), c->log2n, &c->tw_rows);  // k_conv_rows
     }
     for (int w = 0; w < 2; ++w) {
         if (c->log2n <= kOlsLog2 + w) break;
@@ -239,14 +240,14 @@ int conv_filter(const ConvShape &c, const ConvBuffers &b, const float *h, long k
         // launch too
         const long L = 1L << lw;
         const bool h16 = c.precision == ESTL_PRECISION_FP16;
-        e = launch_filter_spectrum(lw, h, k, 0, b.spec, c.tw_ols[lw - kOlsLog2], normalize, st, nullptr, 0, false,
+        e = launch_filter_spectrum(lw, true, h, k, 0, b.spec, c.tw_ols[lw - kOlsLog2], normalize, st, nullptr, 0, false,
                                    b.dc, h16 ? b.spec + L : nullptr);
         if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "filter spectrum launch: %s", hipGetErrorString(e));
         return ESTL_OK;
     }
     if (c.spec_plan.kind == Plan::ROWS) {
         // fold, transform and normalise in one launch (the kernel sum to b.dc)
-        e = launch_filter_spectrum(c.log2n, h, k, shift, b.spec, c.tw_rows, normalize, st, nullptr, 0,
+        e = launch_filter_spectrum(c.log2n, c.wave, h, k, shift, b.spec, c.tw_rows, normalize, st, nullptr, 0,
                                    false, b.dc);
         if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "filter spectrum launch: %s", hipGetErrorString(e));
     } else {
@@ -378,7 +379,7 @@ int conv_run(const ConvShape &c, const ConvBuffers &b, const float *x, float *y,
 int conv_filter_group_rows(const ConvShape &c, const ConvGroup *d_group, int members, bool divide_l1,
                            hipStream_t st) {
     if (!c.fused || c.spec_plan.kind != Plan::ROWS) return set_error(ESTL_ERR_INVALID, "not a fused shape");
-    hipError_t e = launch_filter_spectrum(c.log2n, nullptr, 0, 0, nullptr, c.tw_rows, false, st, d_group,
+    hipError_t e = launch_filter_spectrum(c.log2n, c.wave, nullptr, 0, 0, nullptr, c.tw_rows, false, st, d_group,
                                           members, divide_l1);
     if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group filter spectra: %s", hipGetErrorString(e));
     return ESTL_OK;

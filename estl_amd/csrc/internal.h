@@ -133,9 +133,15 @@ constexpr int kMaxPassLog2 = 13;   // largest radix of a global pass
 constexpr int kMaxSplitLog2Fp16 = 9;  // largest radix of an FP16 pass that a caller can ask for
 constexpr int kMaxPassTileLog2 = 14;  // a pass tile holds at most 2^14 values (~139 KiB of LDS)
 constexpr int kMaxPassCols = 6;    // at most 2^6 columns per tile
-// convolutions of 2^10 values and more (k_conv_wave, k_conv_ols) keep 32 values per thread
-// and a spectrum in the order their transform leaves it (fft_wave.h)
+// Convolutions of 2^10 values and more (k_conv_wave, k_conv_ols) keep 32 values per thread
+// and a spectrum in the order their transform leaves it (fft_wave.h), but for FP32 rows of
+// 2^12 values, which k_conv_rows takes with 16: a lone pair's chain of instructions is shorter
+// there, and its persistent grid has no nearly empty last round (1 row 7.1 us a call against 7.7,
+// 500 rows 7.4 against 8.9, 5000 rows 36.4 against 39; 16000 rows 111 against 101).  Other lengths
+// and binary16 rows are faster in k_conv_wave or within 2 % at any number of rows.  The rule
+// looks at no number of rows: a row's result does not depend on what runs beside it.
 constexpr int kWaveMinLog2 = 10;
+constexpr bool conv_wave(int log2n, bool fp16) { return log2n >= kWaveMinLog2 && (fp16 || log2n != 12); }
 constexpr int kOlsLog2 = 13;       // overlap-save convolution windows of 2^13 values
 constexpr int kOlsWideLog2 = 14;   // and of 2^14 values (rows of n >= 2^15)
 #ifndef ESTL_OLS_MAX_TAPS

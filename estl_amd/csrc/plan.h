@@ -115,8 +115,9 @@ struct ConvShape {
     unsigned flags = 0;
     bool corr = false, fused = false;
     float scale = 1.0f;
+    bool wave = false;                // n <= 2^13: k_conv_wave and its spectra (conv_wave)
     const float2 *tw_rows = nullptr;  // table of the fused rows kernel and the filter's spectrum
-                                      // (n <= 2^13): roots from 2^10 values, powers below
+                                      // (n <= 2^13): roots for k_conv_wave, powers for k_conv_rows
     Plan spec_plan;                  // forward FFT of the folded filter (batch 1)
     std::vector<PassStep> fwd, inv;  // multi-pass pipeline (n > 2^13): fwd, mid, inv
     PassStep mid{};                  // last forward + multiply + first inverse pass
