@@ -148,11 +148,19 @@ __global__ void __launch_bounds__(kUThreads)
 #if ESTL_UBATCH_WAVES
 __attribute__((amdgpu_waves_per_eu(ESTL_UBATCH_WAVES, ESTL_UBATCH_WAVES)))
 #endif
-k_ubatch(UArgs a) {
+k_ubatch(UArgs args) {
     __shared__ float2 lds[kULds];
     __shared__ int s_item;
+    // The arguments are read where an item needs them, from the kernel's argument block:
+    // read ahead of the loop, those of all size classes filled the scalar registers, and each
+    // workgroup started with a dozen waits for them in a row (batches of a few hundred
+    // transforms 7.2 -> 7.9 us a call).
+    using KernArgs = const __attribute__((address_space(4))) UArgs;
+    auto *ap = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
 #pragma unroll 1
     for (;;) {
+        asm volatile("" : "+s"(ap));
+        const UArgs &a = *(const UArgs *)ap;
         if (threadIdx.x == 0) s_item = atomicAdd(&a.counters[0], 1);
         __syncthreads();
         // the ticket and the descriptor are the same for the whole workgroup: say so, so
@@ -180,6 +188,7 @@ k_ubatch(UArgs a) {
         }
     }
     if (threadIdx.x == 0) {
+        const UArgs &a = args;
         __threadfence();
         if (atomicAdd(&a.counters[1], 1) == (int)gridDim.x - 1) {
             atomicExch(&a.counters[0], 0);

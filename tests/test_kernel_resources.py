@@ -41,15 +41,28 @@ def kernels(blob, base):
             p = desc + (descsz + 3) // 4 * 4
 
 
-def test_no_kernel_uses_scratch():
+@pytest.fixture(scope="module")
+def found():
     if not os.path.exists(estl_amd.LIB_PATH):
         pytest.skip("library not built")
     with open(estl_amd.LIB_PATH, "rb") as f:
         blob = f.read()
-    found = [k for base in code_objects(blob) for k in kernels(blob, base)]
-    assert len(found) > 100, "no kernel metadata found in the library"
+    all_kernels = [k for base in code_objects(blob) for k in kernels(blob, base)]
+    assert len(all_kernels) > 100, "no kernel metadata found in the library"
+    return all_kernels
+
+
+def test_no_kernel_uses_scratch(found):
     spilled = {k[".name"]: k[".private_segment_fixed_size"] for k in found if k[".private_segment_fixed_size"]}
     # the convolutions' fused middle pass (k_fft_pass<b, dir, t, true>) keeps tiles of 2^12 values;
     # tiles of 2^14 are compiled beside them and taken by no plan
     spilled = {n: s for n, s in spilled.items() if not ("k_fft_pass" in n and "ELb1E" in n)}
     assert not spilled, spilled
+
+
+def test_work_queue_reads_arguments_where_needed(found):
+    """The arguments of all size classes do not fit the scalar registers: read ahead of the work
+    loop, they are spilled by the dozen, with a wait for each group of them (52 spilled, 0.7 us a
+    call)."""
+    counts = [k[".sgpr_spill_count"] for k in found if "k_ubatch" in k[".name"]]
+    assert len(counts) == 2 and max(counts) <= 8, counts
