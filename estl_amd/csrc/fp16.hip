@@ -73,20 +73,22 @@ __global__ void __launch_bounds__(256) k_maxabs(const float2 *__restrict__ x, in
 
 // y = x / m_t in FP16; scale[t] = m_t (1 for an all-zero transform).  `scale` holds the
 // atomicMax results (float bits) on entry and is rewritten in place with the same bits.
-// A workgroup takes 256 kPackU consecutive values, the workgroups from the last to the first:
-// what k_maxabs read last is still in the memory-side cache.
-// Eight values a thread: one each left the launch bound by its workgroups' dispatch
-// (2^18 x 101 with k_maxabs 98 -> 90 us, 2^26 266 -> 248; chunks that both kernels take in turn
-// were slower).
-constexpr int kPackU = 8;
+// A workgroup takes 256 U consecutive values.  From 2^22 values in all U = 8 (one value per thread
+// leaves the launch bound by its workgroups' dispatch), the workgroups from the last to the
+// first: what k_maxabs read last is still in the memory-side cache (2^18 x 101 with k_maxabs
+// 98 -> 90 us, 2^26 266 -> 248; chunks that both kernels take in turn were slower).  Below, where
+// the values stay cached and a thread's chain of divisions counts, one value per thread, first
+// to last (2^18 x 8 20.9 -> 19.3 us, 2^7 x 20000 17.1 -> 14.8).
+constexpr long kPackWide = 1L << 22;
+template <int U>
 __global__ void __launch_bounds__(256) k_pack(const float2 *__restrict__ x, f16x2 *__restrict__ y, int log2n,
                                               long batch, float *__restrict__ scale) {
     const long count = batch << log2n;
-    const long base = (long)(gridDim.x - 1 - blockIdx.x) * (256 * kPackU) + threadIdx.x;
-    float2 v[kPackU];
-    float m[kPackU];
+    const long base = (long)(U > 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * (256 * U) + threadIdx.x;
+    float2 v[U];
+    float m[U];
 #pragma unroll
-    for (int u = 0; u < kPackU; ++u) {
+    for (int u = 0; u < U; ++u) {
         const long i = base + 256 * u;
         if (i < count) {
             v[u] = ld_stream(x + i);
@@ -94,7 +96,7 @@ __global__ void __launch_bounds__(256) k_pack(const float2 *__restrict__ x, f16x
         }
     }
 #pragma unroll
-    for (int u = 0; u < kPackU; ++u) {
+    for (int u = 0; u < U; ++u) {
         const long i = base + 256 * u;
         if (i < count) {
             const float d = m[u] > 0.0f ? m[u] : 1.0f;
@@ -187,9 +189,14 @@ hipError_t launch_pack_fp16(const float2 *x, void *y16, float *scale, int log2n,
     const int per_log = clog > 8 ? clog - 8 : 0;
     const long blocks = ((batch << log2n) + (1L << (per_log + 8)) - 1) >> (per_log + 8);
     hipLaunchKernelGGL(k_maxabs, dim3((unsigned)blocks), dim3(256), 0, st, x, log2n, batch, umax);
-    const long pb = ((batch << log2n) + 256 * kPackU - 1) / (256 * kPackU);
-    if (pb > 0x7fffffffL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_pack, dim3((unsigned)pb), dim3(256), 0, st, x, y, log2n, batch, scale);
+    const long count = batch << log2n;
+    if (count < kPackWide) {
+        hipLaunchKernelGGL(k_pack<1>, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, st, x, y, log2n, batch, scale);
+    } else {
+        const long pb = (count + 256 * 8 - 1) / (256 * 8);
+        if (pb > 0x7fffffffL) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(k_pack<8>, dim3((unsigned)pb), dim3(256), 0, st, x, y, log2n, batch, scale);
+    }
     return hipGetLastError();
 }
 
