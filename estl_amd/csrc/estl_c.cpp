@@ -243,13 +243,14 @@ int finish_pass(PassStep *s, int device, bool tiled, bool fp16) {
 // allow, evenly split, smaller ones first (a first pass has no pre-twiddles).  A last pass
 // of radix 2^9 reads runs of 16 values per column where smaller ones read 8 or less, which
 // counts where a value is 4 bytes (binary16 2^16 x 300: 75 us as 2^8 2^8, 65 as 2^7 2^9;
-// 2^24 x 2: 178 us as 2^8 2^8 2^8, 165 as 2^7 2^8 2^9) and, in FP32, for rows of 2^15 and 2^16 (2^15 x 1000:
+// 2^24 x 2: 178 us as 2^8 2^8 2^8, 165 as 2^7 2^8 2^9; a third pass pays from 2^22 values: 2^21 x 1
+// 19.3 us as 2^7 2^7 2^7, 20.4 as 2^6 2^6 2^9, 2^21 x 2 27.8 and 25.4) and, in FP32, for rows of 2^15 and 2^16 (2^15 x 1000:
 // 186 -> 177 us).
 static std::vector<int> plan_pass_split(int log2n, long batch, bool fp16) {
     const long values = batch << log2n;
     if ((log2n == 19 || log2n == 20) && (fp16 ? batch > 1 : values >= (1L << 21))) return {log2n - 10, 10};
     const int P = std::max(2, (log2n + 8) / 9);
-    const bool last9 = fp16 ? P <= 3 && values >= (1L << 20) : P == 2 && log2n >= 15 && values >= (1L << 23);
+    const bool last9 = fp16 ? P <= 3 && values >= (P == 3 ? 1L << 22 : 1L << 20) : P == 2 && log2n >= 15 && values >= (1L << 23);
     if (!last9 || (log2n - 9 + P - 2) / (P - 1) > 9) return conv_pass_split(log2n);
     std::vector<int> bits(P, 9);
     const int rest = log2n - 9;

@@ -81,7 +81,6 @@ static int build_plan2d(Plan2D *p, long nx, long ny, long batch, int dir, unsign
             s.args.log2n += lx;
             s.args.log2S += lx;
             s.args.batch = batch;
-            s.args.xcd_remap = 0;
             s.args.scale = (q + 1 == p->cols.steps.size()) ? scale : 1.0f;
             if ((rc = finish_pass(&s, p->cols.device, false, false))) return rc;
             // no tile goes to its neighbour's XCD here, narrow as it may be: with it 1024 x 512 x 4
