@@ -83,9 +83,9 @@ static int build_plan2d(Plan2D *p, long nx, long ny, long batch, int dir, unsign
             s.args.batch = batch;
             s.args.scale = (q + 1 == p->cols.steps.size()) ? scale : 1.0f;
             if ((rc = finish_pass(&s, p->cols.device, false, false))) return rc;
-            // no tile goes to its neighbour's XCD here, narrow as it may be: with it 1024 x 512 x 4
-            // took 22.1 us, without 19.4
-            s.args.xcd_remap = 0;
+            // narrow tiles dealt to the XCDs in runs only while the whole array stays in their L2s
+            // (256 x 256 x 16, 2^20 values: 14.7 us without, 12.0 with; 1024 x 512 x 4: 19.5 and 21.8)
+            if (nx * ny * batch > (1L << 20)) s.args.xcd_remap = 0;
         }
         p->cols.n = nx * ny;
         p->cols.batch = batch;
