@@ -246,7 +246,7 @@ int finish_pass(PassStep *s, int device, bool tiled, bool fp16) {
 // 2^24 x 2: 178 us as 2^8 2^8 2^8, 165 as 2^7 2^8 2^9; a third pass pays from 2^22 values: 2^21 x 1
 // 19.3 us as 2^7 2^7 2^7, 20.4 as 2^6 2^6 2^9, 2^21 x 2 27.8 and 25.4) and, in FP32, for rows of 2^15 and 2^16 (2^15 x 1000:
 // 186 -> 177 us).
-static std::vector<int> plan_pass_split(int log2n, long batch, bool fp16) {
+std::vector<int> plan_pass_split(int log2n, long batch, bool fp16) {
     const long values = batch << log2n;
     if ((log2n == 19 || log2n == 20) && (fp16 ? batch > 1 : values >= (1L << 21))) return {log2n - 10, 10};
     const int P = std::max(2, (log2n + 8) / 9);
@@ -327,6 +327,9 @@ int build_plan(Plan *p, long n, long batch, int dir, int precision, unsigned fla
         if (rc) return rc;
         rc = finish_pass(&st, p->device, tiled, fp16);
         if (rc) return rc;
+        if (fp16 && bits[q] > kMaxSplitLog2Fp16 && !st.args.wide)
+            return set_error(ESTL_ERR_UNSUPPORTED, "no FP16 kernel for radix 2^%d with tiles of 2^%d columns", bits[q],
+                             st.log2t);
         p->steps.push_back(st);
         A *= B;
     }
@@ -528,7 +531,10 @@ int estl_plan_create_split(estl_plan_t *plan, long n, long batch, int direction,
     if (npasses < 0 || npasses > 16 || (npasses > 0 && !log2radices))
         return set_error(ESTL_ERR_INVALID, "bad pass split");
     std::vector<int> split(log2radices, log2radices + npasses);
-    if (precision == ESTL_PRECISION_FP16)
+    // radices above 2^9 in FP16 only as the plan that a caller gets without a split has them
+    const bool own = n > (1L << kMaxRowsLog2) && !(n & (n - 1)) && batch >= 1 &&
+                     split == plan_pass_split(ilog2(n), batch, true);
+    if (precision == ESTL_PRECISION_FP16 && !own)
         for (int b : split)
             if (b > kMaxSplitLog2Fp16)
                 return set_error(ESTL_ERR_UNSUPPORTED, "pass radix 2^%d outside [2^4, 2^%d]", b, kMaxSplitLog2Fp16);

@@ -130,7 +130,7 @@ int rows_pass_count(int log2n);
 
 constexpr int kMaxRowsLog2 = 13;   // largest single-launch row length
 constexpr int kMaxPassLog2 = 13;   // largest radix of a global pass
-constexpr int kMaxSplitLog2Fp16 = 9;  // largest radix of an FP16 pass that a caller can ask for
+constexpr int kMaxSplitLog2Fp16 = 9;  // largest radix of an FP16 pass in any tile
 constexpr int kMaxPassTileLog2 = 14;  // a pass tile holds at most 2^14 values (~139 KiB of LDS)
 constexpr int kMaxPassCols = 6;    // at most 2^6 columns per tile
 // Convolutions of 2^10 values and more (k_conv_wave, k_conv_ols) keep 32 values per thread

@@ -86,6 +86,8 @@ inline std::vector<int> conv_pass_split(int log2n) {
     for (int i = 0; i < log2n % P; ++i) bits[P - 1 - i]++;
     return bits;
 }
+// the passes of a plan of `batch` rows whose caller names no split (estl_c.cpp)
+std::vector<int> plan_pass_split(int log2n, long batch, bool fp16);
 // columns per workgroup (log2) of k_fft_pass (estl_c.cpp)
 int default_pass_tile(int log2b, int log2cpr, long total_cols);
 // a pass's tile (unless `tiled`), kernel (args.wide) and pre-twiddle tables

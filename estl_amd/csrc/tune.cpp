@@ -3,8 +3,8 @@
 // The reference hard-codes one plan per size: radix-16 passes with the remainder last
 // (FFT_OpenCL_Contiguous.h:55-60), each pass a separate generated kernel.  Here the plan
 // space is (a) the single-launch rows kernel when n <= 2^13 and (b) every split of log2 n
-// into 2..4 global passes of radix 2^4..2^13 near the balanced split, each with its
-// default tile width, then the tile widths of the three fastest splits and of the
+// into 2..4 global passes of radix 2^4..2^13 (2^9 in FP16) near the balanced split and the
+// untuned plan's, each with its default tile width, then the tile widths of the three fastest splits and of the
 // fastest split with the fewest passes refined pass by pass.  The tuner times each
 // candidate on the device (HIP events, min of a few runs on zero-filled buffers of the
 // real size) and keeps the fastest per (device, log2 n, batch, direction), preferring
@@ -229,7 +229,15 @@ int tune_plan(long n, long batch, int dir, int precision, bool *rows, std::vecto
         cleanup();
         return set_error(ESTL_ERR_HIP, "tuner set-up failed");
     }
-    std::vector<Choice> cands = candidates(log2n, fp16 ? max_pass_log2_fp16() : kMaxPassLog2);
+    std::vector<Choice> cands = candidates(log2n, fp16 ? kMaxSplitLog2Fp16 : kMaxPassLog2);
+    if (log2n > kMaxRowsLog2) {
+        // the untuned plan too, whatever its radices
+        Choice own;
+        own.split = plan_pass_split(log2n, batch, fp16);
+        bool have = false;
+        for (const Choice &c : cands) have |= c.split == own.split;
+        if (!have) cands.push_back(own);
+    }
     Choice best;
     best.us = 1e30;
     std::vector<Choice> timed;  // pass splits that ran, fastest first after the first stage
