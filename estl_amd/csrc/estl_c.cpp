@@ -446,8 +446,7 @@ std::string describe_plan(const Plan *p) {
         return s;
     }
     if (p->kind == Plan::ROWS) {
-        s += h ? "\"kind\": \"rows\", \"kernel\": \"k_fft_rows_h\", \"radices\": ["
-               : "\"kind\": \"rows\", \"kernel\": \"k_fft_rows\", \"radices\": [";
+        s += std::string("\"kind\": \"rows\", \"kernel\": \"") + rows_kernel(p) + "\", \"radices\": [";
         for (int q = 0; q < rows_pass_count(p->log2n); ++q) {
             long A;
             int B;
@@ -458,14 +457,19 @@ std::string describe_plan(const Plan *p) {
         s += "], \"launches\": 1}";
         return s;
     }
-    s += h ? "\"kind\": \"passes\", \"kernel\": \"k_fft_pass_h\", \"passes\": ["
-           : "\"kind\": \"passes\", \"kernel\": \"k_fft_pass\", \"passes\": [";
+    std::string names, passes;  // the kernels in the order of their first launches
     for (size_t q = 0; q < p->steps.size(); ++q) {
         const auto &st = p->steps[q];
-        snprintf(buf, sizeof buf, "%s{\"radix\": %ld, \"A\": %ld, \"S\": %ld, \"tile\": %d}", q ? ", " : "",
-                 1L << st.log2b, st.args.A, 1L << st.args.log2S, 1 << st.log2t);
-        s += buf;
+        const char *name = pass_kernel(st, h);
+        bool named = false;
+        for (size_t r = 0; r < q; ++r) named = named || pass_kernel(p->steps[r], h) == name;
+        if (!named) names += (q ? std::string(", ") : std::string()) + name;
+        snprintf(buf, sizeof buf,
+                 "%s{\"radix\": %ld, \"A\": %ld, \"S\": %ld, \"tile\": %d, \"kernel\": \"%s\"}", q ? ", " : "",
+                 1L << st.log2b, st.args.A, 1L << st.args.log2S, 1 << st.log2t, name);
+        passes += buf;
     }
+    s += "\"kind\": \"passes\", \"kernel\": \"" + names + "\", \"passes\": [" + passes;
     snprintf(buf, sizeof buf, "], \"launches\": %zu}", p->steps.size());
     s += buf;
     return s;

@@ -86,6 +86,15 @@ inline std::vector<int> conv_pass_split(int log2n) {
     for (int i = 0; i < log2n % P; ++i) bits[P - 1 - i]++;
     return bits;
 }
+// the kernels that a plan's launches run: of a rows plan, and of a pass
+inline const char *rows_kernel(const Plan *p) {
+    return p->precision == ESTL_PRECISION_FP16 ? "k_fft_rows_h"
+           : p->flags & ESTL_FLAG_PLANAR       ? "k_fft_rows_planar"
+                                               : "k_fft_rows";
+}
+inline const char *pass_kernel(const PassStep &s, bool fp16) {
+    return s.args.wide ? "k_pass_wide" : fp16 ? "k_fft_pass_h" : "k_fft_pass";
+}
 // the passes of a plan of `batch` rows whose caller names no split (estl_c.cpp)
 std::vector<int> plan_pass_split(int log2n, long batch, bool fp16);
 // columns per workgroup (log2) of k_fft_pass (estl_c.cpp)

@@ -54,11 +54,11 @@ std::string plan_kernel_info(const Plan *p, int q) {
             snprintf(buf, sizeof buf, "%s%d", k ? "x" : "", B);
             r += buf;
         }
-        snprintf(buf, sizeof buf, "%s, radices %s in registers", h ? "k_fft_rows_h" : "k_fft_rows", r.c_str());
+        snprintf(buf, sizeof buf, "%s, radices %s in registers", rows_kernel(p), r.c_str());
         return buf;
     }
     const PassStep &s = p->steps[q];
-    snprintf(buf, sizeof buf, "%s, radix %ld, %d columns per workgroup", h ? "k_fft_pass_h" : "k_fft_pass",
+    snprintf(buf, sizeof buf, "%s, radix %ld, %d columns per workgroup", pass_kernel(s, h),
              1L << s.log2b, 1 << s.log2t);
     return buf;
 }

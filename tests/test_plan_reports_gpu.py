@@ -1,8 +1,6 @@
 """What a plan reports can be given back: the radices and tiles of every default plan make the
 same plan through an explicit split, and so do the tuner's; and the kernels that the
 reports name are the ones that run."""
-import json
-
 import pytest
 
 import estl_amd
@@ -63,3 +61,27 @@ def test_tuned_fp16_plan_round_trip(gpu, log2n, batch):
     assert log2s([p["radix"] for p in default["passes"]]) in [c["plan"] for c in report["candidates"]]
     desc = estl_amd.Plan(n, batch, estl_amd.FORWARD, estl_amd.FP16, flags=estl_amd.FLAG_AUTOTUNE).describe()
     assert rebuilt(desc, n, batch, estl_amd.FP16).describe() == desc
+
+
+@pytest.mark.parametrize("precision,plain", [(estl_amd.FP32, "k_fft_pass"), (estl_amd.FP16, "k_fft_pass_h")])
+def test_reports_name_the_kernels_that_run(gpu, precision, plain):
+    """The wide kernel has radices 2^7 .. 2^10 in its own tiles; every other pass is the plain
+    one's.  describe() and the profile's lines say which runs each pass."""
+    for split, tiles, want in [([9, 9], [5, 5], ["k_pass_wide"] * 2), ([9, 9], [3, 3], [plain] * 2),
+                               ([6, 8], [6, 5], [plain, "k_pass_wide"])]:
+        p = estl_amd.Plan(1 << sum(split), 4, estl_amd.FORWARD, precision, split=split, tiles=tiles)
+        desc = p.describe()
+        assert [q["kernel"] for q in desc["passes"]] == want
+        assert desc["kernel"] == ", ".join(dict.fromkeys(want))
+        info = [k["info"] for k in p.profile(1)["kernels"]]
+        assert [i.split(",")[0] for i in info] == want
+    names = [q["kernel"] for q in estl_amd.Plan(1 << 20, 33, estl_amd.FORWARD, precision).describe()["passes"]]
+    assert names == ["k_pass_wide"] * 2
+
+
+def test_reports_name_the_rows_kernels(gpu):
+    for precision, flags, want in [(estl_amd.FP32, 0, "k_fft_rows"), (estl_amd.FP16, 0, "k_fft_rows_h"),
+                                   (estl_amd.FP32, estl_amd.FLAG_PLANAR, "k_fft_rows_planar")]:
+        p = estl_amd.Plan(1 << 10, 64, estl_amd.FORWARD, precision, flags=flags)
+        assert p.describe()["kernel"] == want
+        assert p.profile(1)["kernels"][0]["info"].split(",")[0] == want
