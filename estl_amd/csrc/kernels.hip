@@ -95,26 +95,30 @@ hipError_t launch_stream_copy(const void *src, void *dst, long n16, bool nontemp
 
 // A served output's copy as the streaming copy's kernel instead of the runtime's, whose copies
 // of 8-32 MiB outlast the host's calls for them: a burst of 24 requests of up to 32 MiB, each
-// output copied out, 990-1039 -> 884-977 us.  Smaller ones are hidden behind the host either
-// way (15 requests of up to 4 MiB: 470-630 us both) and stay with the runtime, which needs
-// none of the queries below.  Taken from kOutputCopyMin for whole 16-byte
-// values on 16-byte boundaries between buffers of `device`, with the stream and the caller
-// on it, and only inside dst's allocation; *queued stays false otherwise (host or managed
-// memory, another device's, odd sizes), and the caller leaves it to the runtime.
+// output copied out, 975 -> 937 us (medians of eight processes a side in turn, 962-990 and
+// 920-964), of 8 requests 388 -> 363.  Smaller ones are hidden behind the host either way (15
+// requests of up to 4 MiB: 520-670 us both) and stay with the runtime, which needs none of the
+// queries below.  Taken from kOutputCopyMin for whole 16-byte values on 16-byte boundaries
+// between buffers of `device`, with the stream and the caller on it, and only inside dst's
+// allocation; *queued stays false otherwise (host or managed memory, another device's, odd
+// sizes), and the caller leaves it to the runtime.
 constexpr size_t kOutputCopyMin = size_t(8) << 20;
-hipError_t launch_output_copy(const void *src, void *dst, size_t bytes, int device, hipStream_t st, bool *queued) {
-    *queued = false;
-    if (bytes < kOutputCopyMin || bytes % 16 || (uintptr_t)src % 16 || (uintptr_t)dst % 16) return hipSuccess;
+static bool output_copy_fits(const void *dst, size_t bytes, int device, hipStream_t st) {
     int on = -1;
-    if (hipGetDevice(&on) != hipSuccess || on != device) return hipSuccess;
     hipDevice_t on_stream = device;
-    if (st && (hipStreamGetDevice(st, &on_stream) != hipSuccess || on_stream != device)) return hipSuccess;
     hipPointerAttribute_t at{};
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
-    if (hipPointerGetAttributes(&at, dst) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != device ||
-        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)dst) != hipSuccess ||
-        (uintptr_t)dst + bytes > (uintptr_t)base + size) {
+    return hipGetDevice(&on) == hipSuccess && on == device &&
+           (!st || hipStreamGetDevice(st, &on_stream) == hipSuccess) && on_stream == device &&
+           hipPointerGetAttributes(&at, dst) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == device &&
+           hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)dst) == hipSuccess &&
+           (uintptr_t)dst + bytes <= (uintptr_t)base + size;
+}
+hipError_t launch_output_copy(const void *src, void *dst, size_t bytes, int device, hipStream_t st, bool *queued) {
+    *queued = false;
+    if (bytes < kOutputCopyMin || bytes % 16 || (uintptr_t)src % 16 || (uintptr_t)dst % 16) return hipSuccess;
+    if (!output_copy_fits(dst, bytes, device, st)) {
         (void)hipGetLastError();  // a query's error is not the copy's
         return hipSuccess;
     }
