@@ -12,14 +12,15 @@
 //                   the taps (fold_tap): for n <= 2^13 k_filter_spectrum (fold, forward
 //                   FFT and the kernel-sum normalisation in one workgroup), above that
 //                   the first pass of the spectrum plan; the spectrum stays resident;
-//   * k_conv_rows   for n <= 2^13: two real rows enter as one complex row (re = row 2p,
-//                   im = row 2p + 1 -- the filter is real, so the two convolutions stay
-//                   separate), forward FFT, multiply by the spectrum (its conjugate for
+//   * k_conv_wave   for n = 2^10 .. 2^13, k_conv_rows for the other n <= 2^13 (conv_wave):
+//                   two real rows enter as one complex row (re = row 2p, im = row 2p + 1
+//                   -- the filter is real, so the two convolutions stay separate),
+//                   forward FFT, multiply by the spectrum (its conjugate for
 //                   correlation, Convolution.h:125-131), inverse FFT, scale, and the
 //                   re / im parts go back to the two rows: one HBM read and one write
 //                   per value, one launch for the whole batch;
 //   * larger n runs the same pipeline as global passes with fused I/O (pass_tile.h);
-//   * k_conv_rows on binary16 rows, k_filter_l1, k_spec_l1, k_conv_scales: the FP16-storage
+//   * the same on binary16 rows, k_filter_l1, k_spec_l1, k_conv_scales: the FP16-storage
 //                   variant (and group forms of the last three for request groups).
 #include "fft_block.h"
 #include "fft_wave.h"

@@ -2,7 +2,7 @@
 // real rows of length n, a real filter of any length, a batch of rows) and its C ABI.
 //
 // A ConvShape (immutable per n, rows, flags) picks the pipeline:
-//   n <= 2^13: k_conv_rows, one launch (pair-pack, forward FFT, spectrum multiply,
+//   n <= 2^13: k_conv_wave or k_conv_rows (conv_wave), one launch (pair-pack, forward FFT, spectrum multiply,
 //              inverse FFT, scale, unpack);
 //   n >  2^13: the forward global passes (the first reading real pairs), one middle
 //              pass fusing the last forward pass, the spectrum multiply and the first
@@ -367,7 +367,7 @@ int conv_run(const ConvShape &c, const ConvBuffers &b, const float *x, float *y,
         return conv_half_chain(c, b.spec, x, y, b.scratch[0], b.scratch[1], st);
     if (c.fused) {
         hipError_t e = launch_conv_rows(c.log2n, c.corr, x, y, c.rows, b.spec, c.tw_rows, c.scale, st);
-        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "k_conv_rows launch: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "row convolution launch: %s", hipGetErrorString(e));
         return ESTL_OK;
     }
     return conv_pass_chain(c, x, y, b.spec, nullptr, 0, b.scratch[0], b.scratch[1], st);
@@ -407,7 +407,7 @@ int conv_run_group(const ConvShape &c, const ConvGroup *d_group, long pairs, flo
     if (c.fused) {  // one launch over the group's pairs
         hipError_t e = launch_conv_rows(c.log2n, c.corr, nullptr, nullptr, 2 * pairs, nullptr, c.tw_rows, c.scale, st,
                                         d_group);
-        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group k_conv_rows launch: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group row convolution launch: %s", hipGetErrorString(e));
         return ESTL_OK;
     }
     return conv_pass_chain(c, nullptr, nullptr, nullptr, d_group, pairs, scratch0, scratch1, st);
@@ -481,7 +481,7 @@ int conv_run_group_fp16(const ConvShape &c, ConvGroup *d_group, int members, lon
     if (c.fused) {
         e = launch_conv_rows_fp16(c.log2n, c.corr, nullptr, nullptr, 2 * pairs, nullptr, c.tw_rows, c.scale, st,
                                   d_group);
-        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group FP16 k_conv_rows launch: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "group FP16 row convolution launch: %s", hipGetErrorString(e));
     } else if (int rc = conv_pass_chain(c, nullptr, nullptr, nullptr, d_group, pairs, scratch0, scratch1, st)) {
         return rc;
     }
@@ -500,7 +500,7 @@ int conv_run_fp16(const ConvShape &c, const ConvBuffers &b, const void *x16, con
     }
     if (c.fused) {
         e = launch_conv_rows_fp16(c.log2n, c.corr, x16, y16, c.rows, b.spec, c.tw_rows, c.scale, st);
-        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "FP16 k_conv_rows launch: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return set_error(ESTL_ERR_HIP, "FP16 row convolution launch: %s", hipGetErrorString(e));
     } else if (int rc = conv_pass_chain(c, x16, y16, b.spec, nullptr, 0, b.scratch[0], b.scratch[1], st)) {
         return rc;
     }

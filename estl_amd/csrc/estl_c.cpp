@@ -6,9 +6,10 @@
 // per radix-16 pass and compiles a program per FFT object, a plan here picks among
 // precompiled gfx950 kernels:
 //   * rows plan   (n <= 2^13): one launch of k_fft_rows, all passes in LDS;
-//   * pass plan   (n > 2^13): P launches of k_fft_pass, radix up to 2^13 each, the
-//                 Stockham pass formula of FFT_OpenCL_Contiguous.h:167-180 with its
-//                 A_q / N_q prefix products (computeParameters, OpenCLFFTAlgorithm.h:9-12).
+//   * pass plan   (n > 2^13): P launches of k_pass_wide (radices 2^7 .. 2^10, where there
+//                 are tiles enough) or k_fft_pass (radices up to 2^13), the Stockham pass
+//                 formula of FFT_OpenCL_Contiguous.h:167-180 with its A_q / N_q prefix
+//                 products (computeParameters, OpenCLFFTAlgorithm.h:9-12).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -125,17 +126,17 @@ int wave_table(int device, int log2n, const float2 **out) {
     }
     if (log2n < kWaveMinLog2 || log2n > kOlsWideLog2)
         return set_error(ESTL_ERR_UNSUPPORTED, "no roots table for log2n=%d", log2n);
-    const long N = 1L << log2n, T = N / 32, Q = T / 32;
+    const WaveLayout at(log2n);
+    const long N = 1L << log2n;
     float2 *d = nullptr;
     hipStream_t ts = table_stream(device);
-    const long bin = 96, pos = bin + 2048, point = pos + 3 * Q;
-    HIP_TRY(hipMalloc(&d, sizeof(float2) * (point + 3 * T)));
+    HIP_TRY(hipMalloc(&d, sizeof(float2) * at.size));
     for (int e = 0; e < 3; ++e) {
         const long power = 1L << (2 * e);
-        HIP_TRY(launch_twiddle(d + 32 * e, 32, 0, 1, N / 1024 * power, N, ts));
-        if (e < 2) HIP_TRY(launch_twiddle(d + bin + 1024 * e, 1024, 1, Q, power, N, ts));
-        HIP_TRY(launch_twiddle(d + pos + Q * e, Q, 0, 1, 32 * power, N, ts));
-        HIP_TRY(launch_twiddle(d + point + T * e, T, 0, 1, power, N, ts));
+        HIP_TRY(launch_twiddle(d + at.row + 32 * e, 32, 0, 1, N / 1024 * power, N, ts));
+        if (e < 2) HIP_TRY(launch_twiddle(d + at.bin + 1024 * e, 1024, 1, at.Q, power, N, ts));
+        HIP_TRY(launch_twiddle(d + at.pos + at.Q * e, at.Q, 0, 1, 32 * power, N, ts));
+        HIP_TRY(launch_twiddle(d + at.point + at.T * e, at.T, 0, 1, power, N, ts));
     }
     HIP_TRY(hipStreamSynchronize(ts));
     c.tables[key] = d;

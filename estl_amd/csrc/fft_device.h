@@ -214,12 +214,13 @@ struct StaticFor {
 // 16-point transform: 217 instructions with its twiddles' generation; as radix 4 after
 // 15 products by powers of w: 276).
 
-// a + w b and a - w b; w as tabulated for the forward direction (DIR > 0 takes its
+// a + w b and a - w b (as 2 a less the sum: a sum that overflows, or is of infinities, takes the
+// difference with it); w as tabulated for the forward direction (DIR > 0 takes its
 // conjugate), a quarter turn further with ROT.
 template <int DIR, bool ROT>
 __device__ __forceinline__ void butterfly(float2 a, float2 b, float2 w, float2 &sum, float2 &diff) {
     // the twiddle's real part c, and s: w = c + i s
-    const float c = ROT ? (DIR < 0 ? w.y : w.y) : w.x;
+    const float c = ROT ? w.y : w.x;
     const float s = ROT ? (DIR < 0 ? -w.x : w.x) : (DIR < 0 ? w.y : -w.y);
     const float2 t = make_float2(fmaf(-s, b.y, fmaf(c, b.x, a.x)), fmaf(s, b.x, fmaf(c, b.y, a.y)));
     sum = t;

@@ -41,14 +41,6 @@ struct WaveGeom {
     static constexpr int lds_floats = 32 * RS;
 };
 
-// the bin that position pos = r T + u of such a spectrum holds
-template <int LOG2N>
-__host__ __device__ constexpr int wave_bin(int pos) {
-    using G = WaveGeom<LOG2N>;
-    const int r = pos / G::T, u = pos % G::T;
-    return u / G::Q + 32 * (r / G::Q + (32 / G::Q) * (u % G::Q)) + 1024 * (r % G::Q);
-}
-
 // Orders this wave's LDS accesses (a wave's LDS operations execute in order; the
 // compiler must not move them across).
 __device__ __forceinline__ void wave_lds_fence() {
@@ -71,13 +63,14 @@ __device__ __forceinline__ void exchange_sync() {
 // rounded, with the fourth and sixteenth powers beside the roots so that no power is
 // squared twice:
 //   row:   W_1024^{e k1}, k1 < 32, for e = 1, 4, 16
-//   bin:   W_N^{e (k1 + 32 k2)} at (k2 mod 32 / Q) T + thread, for e = 1, 4
+//   bin:   W_N^{e (k1 + 32 k2)} at (k2 mod 32 / Q) T + thread (wave_bin), for e = 1, 4
 //   pos:   W_T^{e t'}, t' < Q, for e = 1, 4, 16
 //   point: W_N^{e t}, t < T, for e = 1, 4, 16
 template <int LOG2N>
 struct WaveRoots {
-    static constexpr int row = 0, bin = 96, pos = bin + 2048, point = pos + 3 * WaveGeom<LOG2N>::Q;
-    static constexpr int size = point + 3 * WaveGeom<LOG2N>::T;
+    static constexpr WaveLayout at{LOG2N};
+    static_assert(at.T == WaveGeom<LOG2N>::T && at.Q == WaveGeom<LOG2N>::Q, "the table's geometry is the kernel's");
+    static constexpr int row = at.row, bin = at.bin, pos = at.pos, point = at.point;
 };
 
 // w, w^4, w^16 of a 32-point step: at roots[t], [STRIDE + t], [2 STRIDE + t].  A step's roots

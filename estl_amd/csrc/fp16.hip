@@ -318,7 +318,7 @@ constexpr int kMaxPassLog2Fp16 = 10;
 
 template <int LOG2B, int DIR, int LOG2T, bool MID>
 static hipError_t launch_pass_h_t(const f16x2 *in, f16x2 *out, const PassArgs &a, hipStream_t st) {
-    if constexpr (LOG2B + LOG2T > kMaxPassTileLog2) {
+    if constexpr (LOG2B + LOG2T > (MID ? kMaxMidTileLog2 + 1 : kMaxPassTileLog2)) {
         return hipErrorInvalidValue;
     } else {
         const int lcpr = a.log2n - LOG2B;

@@ -132,6 +132,8 @@ constexpr int kMaxRowsLog2 = 13;   // largest single-launch row length
 constexpr int kMaxPassLog2 = 13;   // largest radix of a global pass
 constexpr int kMaxSplitLog2Fp16 = 9;  // largest radix of an FP16 pass in any tile
 constexpr int kMaxPassTileLog2 = 14;  // a pass tile holds at most 2^14 values (~139 KiB of LDS)
+constexpr int kMaxMidTileLog2 = 12;   // a convolution's middle pass: radices up to 2^9 (conv_pass_split) in tiles of
+                                      // at most 2^12 values, 2^13 in FP16 storage
 constexpr int kMaxPassCols = 6;    // at most 2^6 columns per tile
 // Convolutions of 2^10 values and more (k_conv_wave, k_conv_ols) keep 32 values per thread
 // and a spectrum in the order their transform leaves it (fft_wave.h), but for FP32 rows of
@@ -142,6 +144,17 @@ constexpr int kMaxPassCols = 6;    // at most 2^6 columns per tile
 // looks at no number of rows: a row's result does not depend on what runs beside it.
 constexpr int kWaveMinLog2 = 10;
 constexpr bool conv_wave(int log2n, bool fp16) { return log2n >= kWaveMinLog2 && (fp16 || log2n != 12); }
+// The roots' table of wave_fft for 2^log2n values: T = 2^log2n / 32 threads, Q = T / 32 per row,
+// and where each kind of root begins (fft_wave.h says what they are).
+struct WaveLayout {
+    int T, Q, row, bin, pos, point, size;
+    constexpr explicit WaveLayout(int log2n)
+        : T((1 << log2n) / 32), Q(T / 32), row(0), bin(row + 3 * 32), pos(bin + 2 * 1024), point(pos + 3 * Q),
+          size(point + 3 * T) {}
+};
+// k1 + 32 k2 of the values that thread u = k1 Q + t' holds after the second step, in group m:
+// k2 = m + (32 / Q) t'
+constexpr int wave_bin(int m, int u, int Q) { return u / Q + 32 * (m + 32 / Q * (u % Q)); }
 constexpr int kOlsLog2 = 13;       // overlap-save convolution windows of 2^13 values
 constexpr int kOlsWideLog2 = 14;   // and of 2^14 values (rows of n >= 2^15)
 #ifndef ESTL_OLS_MAX_TAPS

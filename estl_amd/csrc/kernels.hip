@@ -21,16 +21,14 @@ namespace estl {
 
 // ------------------------------------------------------------------ twiddles
 // mode 0 (linear): entry e -> m = e * mult
-// mode 1 (the bin roots of WaveRoots, Q = A): entry e = r T + u, T = 32 Q ->
-//         m = mult * bin, bin = u / Q + 32 (r + (32 / Q) (u mod Q))
+// mode 1 (the bin roots of WaveRoots, Q = A): entry e = r T + u, T = 32 Q -> m = mult * wave_bin
 // value = exp(-2 pi i m / nq), computed as sincospi(2 m / nq) in double.
 __global__ void k_twiddle(float2 *__restrict__ dst, long count, int mode, long A, long mult, long nq) {
     long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
     long m;
     if (mode == 1) {
-        const long r = e / (32 * A), u = e % (32 * A);
-        m = (u / A + 32 * (r + 32 / A * (u % A))) * mult % nq;
+        m = wave_bin(int(e / (32 * A)), int(e % (32 * A)), int(A)) * mult % nq;
     } else {
         m = (e * mult) % nq;
     }
@@ -314,7 +312,7 @@ long rows_power_count(int log2n) {
 #define POW_CASE(L) \
     case L: return BlockGeom<L>::powsize;
         POW_CASE(1) POW_CASE(2) POW_CASE(3) POW_CASE(4) POW_CASE(5) POW_CASE(6) POW_CASE(7) POW_CASE(8)
-        POW_CASE(9) POW_CASE(10) POW_CASE(11) POW_CASE(12) POW_CASE(13) POW_CASE(14)
+        POW_CASE(9) POW_CASE(10) POW_CASE(11) POW_CASE(12) POW_CASE(13)
 #undef POW_CASE
         default: return -1;
     }

@@ -35,7 +35,7 @@ k_fft_pass(const float2 *__restrict__ in, float2 *__restrict__ out, PassArgs a) 
 
 template <int LOG2B, int LOG2T, bool MID>
 static hipError_t launch_t(const float2 *in, float2 *out, const PassArgs &a, hipStream_t st) {
-    if constexpr (LOG2B + LOG2T > kMaxPassTileLog2) {
+    if constexpr (LOG2B + LOG2T > (MID ? kMaxMidTileLog2 : kMaxPassTileLog2)) {
         return hipErrorInvalidValue;
     } else {
         const int lcpr = a.log2n - LOG2B;
@@ -98,10 +98,6 @@ hipError_t launch_pass_mid(int log2b, int log2t, const float2 *in, float2 *out, 
         case 7: return launch_b<7, true>(log2t, in, out, a, st);
         case 8: return launch_b<8, true>(log2t, in, out, a, st);
         case 9: return launch_b<9, true>(log2t, in, out, a, st);
-        case 10: return launch_b<10, true>(log2t, in, out, a, st);
-        case 11: return launch_b<11, true>(log2t, in, out, a, st);
-        case 12: return launch_b<12, true>(log2t, in, out, a, st);
-        case 13: return launch_b<13, true>(log2t, in, out, a, st);
         default: return hipErrorInvalidValue;
     }
 }

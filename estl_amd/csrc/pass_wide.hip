@@ -23,8 +23,11 @@ static hipError_t launch_t(const void *in, void *out, const PassArgs &a, hipStre
     const long tiles = a.batch << (lcpr - LOG2T);
     if (tiles > 0x7fffffffL) return hipErrorInvalidValue;
     auto kernel = a.A == 1 ? k_pass_wide<LOG2B, ESTL_PASS_DIR, LOG2T, kWideFirst, ST>
-                  : a.log2S >= LOG2T ? k_pass_wide<LOG2B, ESTL_PASS_DIR, LOG2T, kWideMiddle, ST>
-                                     : k_pass_wide<LOG2B, ESTL_PASS_DIR, LOG2T, kWideLast, ST>;
+                           : k_pass_wide<LOG2B, ESTL_PASS_DIR, LOG2T, kWideMiddle, ST>;
+    if (a.A > 1 && a.log2S < LOG2T) {
+        if constexpr (LOG2B > 7) kernel = k_pass_wide<LOG2B, ESTL_PASS_DIR, LOG2T, kWideLast, ST>;
+        else return hipErrorInvalidValue;  // pass_is_wide: k_fft_pass's
+    }
     hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(WideTile<LOG2B, LOG2T, 0>::threads), 0, st,
                        static_cast<const ST *>(in), static_cast<ST *>(out), a);
     return hipGetLastError();

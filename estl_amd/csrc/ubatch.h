@@ -19,6 +19,7 @@ constexpr int kUMaxSmallLog2 = kUThreadsLog2 + 4;
 __host__ __device__
 #endif
 constexpr int ubatch_split(int L) { return L / 2; }
+constexpr int kUWideLog2 = 17;  // from here both passes keep 32 values per thread (workqueue.hip)
 
 // One work item: `count` transforms of size 2^log2n, the `first`-th.. of the
 // size-sorted offset list (count = 1 for large sizes).

@@ -149,15 +149,11 @@ static int ubatch_create(UBatch **out, int count, const long *sizes, const long 
         for (auto &it : u->items) used |= (it.log2n == L);
         if (!used) continue;
         const int b = ubatch_split(L);
-        int rf = linear_table(u->device, 1L << b, 1, 1L << b, &tw.first[b]);
-        if (!rf) rf = linear_table(u->device, 1, 1, 1, &tw.one);
-        if (rf) {
-            ubatch_free(u);
-            return rf;
-        }
         const long nq = 1L << L;
         tw.lobits[L] = (L + 1) / 2;
-        int rc = linear_table(u->device, 1L << tw.lobits[L], 1, nq, &tw.lo[L]);
+        int rc = L >= kUWideLog2 ? linear_table(u->device, 1L << b, 1, 1L << b, &tw.first[b]) : ESTL_OK;
+        if (!rc && L >= kUWideLog2) rc = linear_table(u->device, 1, 1, 1, &tw.one);
+        if (!rc) rc = linear_table(u->device, 1L << tw.lobits[L], 1, nq, &tw.lo[L]);
         if (!rc) rc = linear_table(u->device, nq >> tw.lobits[L], 1L << tw.lobits[L], nq, &tw.hi[L]);
         if (rc) {
             ubatch_free(u);

@@ -41,7 +41,7 @@ struct USmall {
 // second radix of 2^9).
 template <int L>
 struct ULarge {
-    static constexpr bool wide = L >= 17;
+    static constexpr bool wide = L >= kUWideLog2;
     static constexpr int B1 = ubatch_split(L), B2 = L - B1;
     static constexpr int per = kUThreadsLog2 + (wide ? 5 : 4);  // values of a tile
     static constexpr int T1 = per - B1, T2 = per - B2;
