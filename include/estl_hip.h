@@ -57,7 +57,8 @@ extern "C" {
 #define ESTL_CONV_FP16 0x80u             /* server: binary16 rows with per-row scales         */
 #define ESTL_CONV_FULL_LENGTH 0x100u     /* transform whole rows even where overlap-save      */
                                          /* windows would serve (rows longer than 2^13 with   */
-                                         /* filters of at most 4097 taps)                     */
+                                         /* filters of at most 4097 taps, longer than 2^14    */
+                                         /* with at most 8193)                                */
 
 typedef struct estl_plan_s *estl_plan_t;
 typedef struct estl_ubatch_s *estl_ubatch_t;
@@ -81,11 +82,16 @@ int estl_init(int device);
  * plan at :55-61) and the factory call FFTFactorySpecific::newFFT (FFT.h:51).
  * direction: ESTL_FORWARD / ESTL_BACKWARD.  precision: ESTL_PRECISION_*.
  * flags: ESTL_FLAG_* bits.  Twiddle tables are built on the device (FP64, rounded to
- * FP32) and shared by all plans of the same size on that device. */
+ * FP32) and shared by all plans of the same size on that device.
+ * The number of passes and the kernels of a plan of n > 2^13 are chosen by n and batch, so a
+ * row's last bits may differ between plans of different batch (both within the transform's
+ * error); a plan of one split and its tiles, or of n <= 2^13, computes a row the same in any
+ * batch, and every execution of a plan computes the same values. */
 int estl_plan_create(estl_plan_t *plan, long n, long batch, int direction, int precision, unsigned flags);
 
 /* Same as estl_plan_create with an explicit pass split: npasses global passes of radix
- * 2^log2radices[q] (each in [4, 13], summing to log2 n), each computed by workgroups
+ * 2^log2radices[q] (each in [1, 13], in FP16 [4, 9] and whatever the default plan has,
+ * summing to log2 n), each computed by workgroups
  * owning 2^log2tiles[q] adjacent columns (log2tiles may be NULL: default widths).
  * npasses = 0 picks the default plan.  The reference fixes the split to radix-16
  * passes with the remainder last (BGs, FFT_OpenCL_Contiguous.h:55-60); here it is the
