@@ -77,7 +77,8 @@ struct WaveRoots {
 // are loaded before the exchange ahead of it, which needs few registers, and arrive
 // meanwhile: loaded where they are used, each step of a lone wave waited for the L2 (a call of
 // one row of 2^14 values 11.1 -> 10.6 us, 1000 rows of 2^11 8.9 -> 8.25, 63 rows of 2^20 at 4097
-// taps 154 -> 145).
+// taps 154 -> 145).  At 2^10 values (Q = 1, no exchange but one inside the wave) they are
+// loaded at their use: 30001 rows 46.2 us with them ahead, 45.5 so.
 struct Roots32 {
     float2 w1, w4, w16;
 };
@@ -128,7 +129,8 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
     const int tq = t % Q;
     using W = WaveRoots<LOG2N>;
     Dft<32, -1>::run(v);
-    const Roots32 wr = load_roots<32>(tw + W::row, t / Q);
+    Roots32 wr;
+    if constexpr (Q > 1) wr = load_roots<32>(tw + W::row, t / Q);
     if (lds_busy) exchange_sync<G::in_wave>();
 #pragma unroll
     for (int k = 0; k < 32; ++k) lds[k * RS + t] = v[k].x;
@@ -141,6 +143,7 @@ __device__ __forceinline__ void wave_fft(float2 (&v)[32], float *lds, int t, con
     exchange_sync<G::in_wave>();
 #pragma unroll
     for (int i = 0; i < 32; ++i) v[i].y = row[tq + Q * i];
+    if constexpr (Q == 1) wr = load_roots<32>(tw + W::row, t / Q);
     dft32_rooted<-1>(v, wr);
     if constexpr (Q > 1) {
         RootsQ wb[32 / Q];
@@ -197,7 +200,8 @@ __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, co
     } else {
         Dft<32, +1>::run(v);
     }
-    const Roots32 wn = load_roots<T>(tw + W::point, t);
+    Roots32 wn;
+    if constexpr (Q > 1) wn = load_roots<T>(tw + W::point, t);
     wave_lds_fence();
 #pragma unroll
     for (int i = 0; i < 32; ++i) row[tq + Q * i] = v[i].x;
@@ -210,6 +214,7 @@ __device__ __forceinline__ void wave_ifft(float2 (&v)[32], float *lds, int t, co
     exchange_sync<G::in_wave>();
 #pragma unroll
     for (int k = 0; k < 32; ++k) v[k].y = lds[k * RS + t];
+    if constexpr (Q == 1) wn = load_roots<T>(tw + W::point, t);
     dft32_rooted<+1>(v, wn);
 }
 

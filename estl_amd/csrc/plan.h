@@ -146,17 +146,20 @@ bool conv_half_path(long n, long rows, int precision);
 // Rows longer than an overlap-save window convolved with a filter of at most
 // kOlsWideMaxTaps taps run overlap-save unless ESTL_CONV_FULL_LENGTH asks for whole-row
 // transforms: one launch (conv.hip k_conv_ols) over windows of L = 2^13 values (K <= 4097
-// taps; 512-thread workgroups, two per CU) or 2^14 values (n >= 2^15, K <= 8193; 1024
-// threads, one per CU), each giving M = L - K + 1 outputs, with the filter's L-point
+// taps; 256-thread workgroups, four per CU) or 2^14 values (n >= 2^15, K <= 8193; 512
+// threads, two per CU), each giving M = L - K + 1 outputs, with the filter's L-point
 // spectrum.  Returns log2 L, or 0 for whole-row transforms.
 //
-// Between the two window lengths (both possible) the choice is a cost model fitted to
-// MI355X timings of the two kernels (68 shapes of 2^22 to 2^28 values, K = 16..4097; the
-// choice is within 1.5 % of the faster length at each, where the two differ by up to
-// 30 %).  Window pairs are dealt to the `cus` CUs and the time is that of the CU with the
-// most: with T the time a CU takes for two concurrent 2^13 pairs (four windows), a lone
-// 2^13 pair takes 0.35 T and a 2^14 pair (one per CU) 1.10 T -- or 0.90 T when every CU
-// has at most one (a single short round).  cus = 0: the windows' count and size alone.
+// Between the two window lengths (both possible) the choice is a cost model: window pairs
+// are dealt to the `cus` CUs and the time is that of the CU with the most: with T the time a
+// CU takes for two 2^13 pairs (four windows), a lone 2^13 pair takes 0.35 T and a 2^14 pair
+// 1.10 T -- or 0.90 T when every CU has at most one (a single short round).  cus = 0: the
+// windows' count and size alone.  The ratios were fitted to kernels with 16 values per thread,
+// two 2^13 pairs or one 2^14 pair per CU.  The present ones timed at 161 shapes (2^15 to 2^28
+// values, K = 16..4097, FP32 and binary16): the choice is within 5.7 % of the faster length
+// (within 1.5 % at all but six) outside one region.  Where a CU has one 2^14 pair or two 2^13
+// pairs, the model takes 2^14, and 2^13 is 3-15 % faster (2^22 x 1 and 16 taps: 15.5 us against
+// 17.2; 2^16 x 64 and 2048 taps: 15.5 against 16.8).
 // 2^13 windows read fewer padding values for short filters (L/M near 1 for either length,
 // and the last window of a row less wasted); 2^14 windows read each input value fewer
 // times for long filters (L/M = 1.14 against 1.33 at K = 2048).
