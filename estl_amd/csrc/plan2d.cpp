@@ -83,9 +83,12 @@ static int build_plan2d(Plan2D *p, long nx, long ny, long batch, int dir, unsign
             s.args.batch = batch;
             s.args.scale = (q + 1 == p->cols.steps.size()) ? scale : 1.0f;
             if ((rc = finish_pass(&s, p->cols.device, false, false))) return rc;
-            // narrow tiles dealt to the XCDs in runs only while the whole array stays in their L2s
-            // (256 x 256 x 16, 2^20 values: 14.7 us without, 12.0 with; 1024 x 512 x 4: 19.5 and 21.8)
-            if (nx * ny * batch > (1L << 20)) s.args.xcd_remap = 0;
+            // Narrow tiles go to the XCDs in runs (finish_pass), which is worth 5-20 % (256 x 256 x 16
+            // 14.7 -> 12.0 us, 512 x 512 x 5 19.7 -> 17.2, 1024 x 512 x 7 32.5 -> 29.4) but for arrays of
+            // 3 2^19 to 2^21 values, which lose 3-12 % by it (1024 x 512 x 3 19.3 -> 20.5, x 4 19.5 ->
+            // 21.8, 256 x 256 x 31 18.7 -> 20.4).
+            const long values = nx * ny * batch;
+            if (values >= (3L << 19) && values <= (1L << 21)) s.args.xcd_remap = 0;
         }
         p->cols.n = nx * ny;
         p->cols.batch = batch;
