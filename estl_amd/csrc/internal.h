@@ -138,10 +138,11 @@ constexpr int kMaxPassCols = 6;    // at most 2^6 columns per tile
 // Convolutions of 2^10 values and more (k_conv_wave, k_conv_ols) keep 32 values per thread
 // and a spectrum in the order their transform leaves it (fft_wave.h), but for FP32 rows of
 // 2^12 values, which k_conv_rows takes with 16: a lone pair's chain of instructions is shorter
-// there, and its persistent grid has no nearly empty last round (1 row 7.1 us a call against 7.7,
-// 500 rows 7.4 against 8.9, 5000 rows 36.4 against 39; 16000 rows 111 against 101).  Other lengths
-// and binary16 rows are faster in k_conv_wave or within 2 % at any number of rows.  The rule
-// looks at no number of rows: a row's result does not depend on what runs beside it.
+// there, and its persistent grid has no nearly empty last round (1 row 7.3 us a call against 8.0,
+// 500 rows 7.7 against 9.2, 2000 rows 13.9 against 14.8, 5000 rows 36.4 against 38.7; the other way
+// 4000 rows 29.2 against 27.9, one full round, and 16000 rows 111 against 102).  Other lengths and
+// binary16 rows are faster in k_conv_wave or within 2 % at any number of rows.  The rule looks at
+// no number of rows: a row's result does not depend on what runs beside it.
 constexpr int kWaveMinLog2 = 10;
 constexpr bool conv_wave(int log2n, bool fp16) { return log2n >= kWaveMinLog2 && (fp16 || log2n != 12); }
 // The roots' table of wave_fft for 2^log2n values: T = 2^log2n / 32 threads, Q = T / 32 per row,
