@@ -223,7 +223,8 @@ __device__ __forceinline__ void multiply_spectrum(float2 (&v)[32], const float2 
 // [-1, 1] (|y| <= sum |h| max |x|); the caller's per-row scales carry the magnitudes).
 // Bound by HBM and VALU alike: 65 vector instructions per complex value at 2^10 points and
 // no barrier (16 values per thread and three exchanges across the workgroup took 105).
-// 30001 rows of 1024 values: 54.2 -> 45.3 us (4.53 -> 5.43 TB/s); 4001 rows of 8192: 84 -> 59 us.
+// 30001 rows of 1024 values, new with each call: 54.4 -> 47.9 us (4.5 -> 5.13 TB/s); 4000 rows of
+// 8192: 82.5 -> 57 us.
 template <int LOG2N, int TPW, bool CORR, typename R>
 __global__ void __launch_bounds__(WaveGeom<LOG2N>::T * TPW) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 *__restrict__ spec,
@@ -514,13 +515,14 @@ __device__ __forceinline__ void st_piece(__amdgpu_buffer_rsrc_t piece, int i, in
 
 // One workgroup per pair of windows, 32 values per thread, at most 128 VGPRs and 33 / 66
 // KiB of LDS: four waves per SIMD, four workgroups per CU at L = 2^13 and two at 2^14, so
-// one's loads and stores overlap another's arithmetic.  Bound by the vector instructions,
-// at a clock that power holds to 2.0-2.3 GHz, then by the last round of workgroups; a call of
-// a few windows by one wave's chain of them.  Nothing is spilled, and the stores have no
-// lane tests: with 24 bytes of scratch and a branch per store a call took 14.5 us for one row of
-// 2^14 values (12.7 with 16 values per thread), 11.1 without; 63 rows of 2^20 and 2049
-// taps (2^13 windows) 146 -> 135 us (201), 101 binary16 rows of 2^18 and 6001 taps (2^14) 74 -> 66
-// (122).
+// one's loads and stores overlap another's arithmetic.  Bound by the vector instructions (90
+// per complex value at 2^13, 96 at 2^14), at a clock that power holds to 2.0-2.3 GHz, then by
+// the last round of workgroups; a call of a few windows by one wave's chain of them.  Nothing is
+// spilled, and the stores have no lane tests: with 24 bytes of scratch and a branch per store a
+// call took 14.5 us for one row of 2^14 values (12.7 with 16 values per thread), 11.1 without,
+// 10.6 with the roots loaded ahead (fft_wave.h); 63 rows of 2^20 and 2049 taps (2^13 windows)
+// 146 -> 135 -> 131 us (201 with 16 values), 101 binary16 rows of 2^18 and 6001 taps (2^14)
+// 74 -> 66 -> 64 (122).
 template <int LOG2L, bool CORR, typename R>
 __global__ void __launch_bounds__(WaveGeom<LOG2L>::T) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_ols(const R *__restrict__ x, R *__restrict__ y, OlsArgs a, const float2 *__restrict__ spec,

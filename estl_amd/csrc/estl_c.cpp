@@ -175,7 +175,7 @@ static int ilog2(long n) {
 // contiguous runs per load and store), capped at 64, narrowed while that leaves fewer
 // than 512 tiles to spread over the CUs (small problems are latency-bound), to 8: narrower
 // ones share their 128-byte lines three ways and more (2^18 x 4: 22.4 us with 4 columns,
-// 13.6 with 8).  Tiles of radices above 2^11 hold 2^14 values, not to be narrower still.
+// 13.6 with 8).  Tiles of radices above 2^10 hold 2^14 values, not to be narrower still.
 int default_pass_tile(int log2b, int log2cpr, long total_cols) {
     int lt = (log2b > 10 ? 14 : 13) - log2b;
     if (lt > kMaxPassCols) lt = kMaxPassCols;

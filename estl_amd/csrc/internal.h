@@ -6,7 +6,7 @@
 
 namespace estl {
 
-// Arguments of one global Stockham pass (k_fft_pass).
+// Arguments of one global Stockham pass (k_fft_pass, k_pass_wide).
 // A group of convolution requests of one length n run as one batch (the server's
 // continuous batching): request q owns pair rows [pair_start[q], pair_start[q + 1]) of
 // the batch.  Its real rows are read from x[q] and written to y[q] (real_rows[q] of

@@ -132,8 +132,8 @@ hipError_t launch_output_copy(const void *src, void *dst, size_t bytes, int devi
 // value, nontemporal loads and stores.  A partial last group computes its missing rows
 // on a copy of the last row and stores nothing for them.  With twiddles by powers
 // the kernel holds 58 VGPRs at 4096 and 8192 points, so LDS alone bounds
-// residency (four 34 KiB groups per CU; two 8192-point rows), and it runs at the copy's
-// rate: 4096 x 16384 in 167-175 us between devices, 6.1-6.4 TB/s of the copy's 6.55.  Measured against
+// residency (four 34 KiB groups per CU; two 8192-point rows), and it runs near the copy's
+// rate: 4096 x 16384 in 167-180 us between devices, 6.0-6.4 TB/s, 0.93-0.97 of the copy.  Measured against
 // the earlier persistent grid (four resident rounds of workgroups, the next group
 // prefetched into registers; at 4096 and 8192 points a table of all twiddles held in
 // registers across rows, 167 / 206 VGPRs): 6.5 % faster at 4096 x 16384 and 9 % at
@@ -141,7 +141,7 @@ hipError_t launch_output_copy(const void *src, void *dst, size_t bytes, int devi
 // in flight, and the grid's last round is one group deep.
 // With its loads issued a wave goes before those still issuing theirs (up to 4096 points):
 // rows leave the CU as soon as they are done instead of in bursts, 177.9 -> 174.3 us at
-// 4096 x 16384 and 175.5 -> 173.2 at 2048 x 32768; 8192 points, two workgroups per CU,
+// 4096 x 16384 (which is what fewer instructions had cost on such devices) and 175.5 -> 173.2 at 2048 x 32768; 8192 points, two workgroups per CU,
 // would lose 1 %.
 template <int LOG2N>
 __device__ __forceinline__ void rows_loaded() {
