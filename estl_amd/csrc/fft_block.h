@@ -90,7 +90,8 @@ __device__ __forceinline__ void block_fft(float2 (&v)[BlockGeom<LOG2N>::E], floa
                 constexpr int b = decltype(bc)::value;
                 float2 u[B];
                 StaticFor<0, B>::run([&](auto sc) { u[decltype(sc)::value] = v[b + NB * decltype(sc)::value]; });
-                Dft<B, DIR>::run(u);
+                if constexpr (G::P == 1) DftApart<B, DIR>::run(u);
+                else Dft<B, DIR>::run(u);
                 StaticFor<0, B>::run([&](auto hc) { v[b + NB * decltype(hc)::value] = u[decltype(hc)::value]; });
             });
         } else {

@@ -288,6 +288,58 @@ struct Dft {
     }
 };
 
+// a + w b and a - w b, each by itself: 8 instructions instead of butterfly's 6.
+template <int K, int R, int DIR>
+__device__ __forceinline__ void butterfly_apart(float2 a, float2 b, float2 &sum, float2 &diff) {
+    if constexpr ((4 * K) % R == 0) {
+        const float2 t = twc<K, R, DIR>(b);
+        sum = cadd(a, t);
+        diff = csub(a, t);
+    } else {
+        constexpr float c = float(ct::cos2pi(K, R)), s = float(DIR) * float(ct::sin2pi(K, R));
+        sum = make_float2(fmaf(-s, b.y, fmaf(c, b.x, a.x)), fmaf(s, b.x, fmaf(c, b.y, a.y)));
+        diff = make_float2(fmaf(s, b.y, fmaf(-c, b.x, a.x)), fmaf(-s, b.x, fmaf(-c, b.y, a.y)));
+    }
+}
+
+// The DFT of a whole transform of R <= 16 values: no sum takes another along when it overflows,
+// and no value meets two rotations by other than quarter turns, so an infinite input gives
+// infinities of the right signs and no NaN.  Such transforms are HBM-bound (16 values per
+// thread, no exchange).
+template <int R, int DIR>
+struct DftApart {
+    static_assert(R <= 16, "one register DFT");
+    static __device__ __forceinline__ void run(float2 *x) {
+        if constexpr (R < 8) {
+            Dft<R, DIR>::run(x);
+        } else {
+            // R / 4 apart: S transforms of 4 or 2 x 4 values, joined with one rotation each
+            constexpr int S = R / 4;
+            float2 e[S][4];
+            StaticFor<0, S>::run([&](auto sc) {
+                constexpr int s = decltype(sc)::value;
+                StaticFor<0, 4>::run([&](auto mc) { e[s][decltype(mc)::value] = x[S * decltype(mc)::value + s]; });
+                Dft<4, DIR>::run(e[s]);
+            });
+            StaticFor<0, 4>::run([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                if constexpr (S == 2) {
+                    butterfly_apart<k, R, DIR>(e[0][k], e[1][k], x[k], x[k + 4]);
+                } else {
+                    float2 a, b, c, d;
+                    butterfly_apart<2 * k, R, DIR>(e[0][k], e[2][k], a, b);
+                    butterfly_apart<3 * k, R, DIR>(twc<k, R, DIR>(e[1][k]), e[3][k], c, d);
+                    const float2 t = twc<1, 4, DIR>(d);
+                    x[k] = cadd(a, c);
+                    x[k + 4] = cadd(b, t);
+                    x[k + 8] = csub(a, c);
+                    x[k + 12] = csub(b, t);
+                }
+            });
+        }
+    }
+};
+
 __device__ __forceinline__ float2 csquare(float2 a) {
     return make_float2(fmaf(a.x, a.x, -a.y * a.y), 2.0f * a.x * a.y);
 }
