@@ -142,10 +142,11 @@ hipError_t launch_output_copy(const void *src, void *dst, size_t bytes, int devi
 // With its loads issued a wave goes before those still issuing theirs (up to 4096 points):
 // rows leave the CU as soon as they are done instead of in bursts, 177.9 -> 174.3 us at
 // 4096 x 16384 (which is what fewer instructions had cost on such devices) and 175.5 -> 173.2 at 2048 x 32768; 8192 points, two workgroups per CU,
-// would lose 1 %.
+// would lose 1 %, and 32 points, whose loads bring 16 bytes of each row at a time, 14 % (2^20 rows
+// 215 -> 241 us, 210 without it).
 template <int LOG2N>
 __device__ __forceinline__ void rows_loaded() {
-    if constexpr (LOG2N <= 12) __builtin_amdgcn_s_setprio(3);
+    if constexpr (LOG2N >= 6 && LOG2N <= 12) __builtin_amdgcn_s_setprio(3);
 }
 
 template <int LOG2N, int DIR, int TPW, bool SCALED>
