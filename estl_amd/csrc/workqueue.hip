@@ -76,7 +76,7 @@ constexpr int kULds = kULdsSmall > kULdsLarge ? kULdsSmall : kULdsLarge;
 static_assert(kULds * 8 <= 79 * 1024, "two workgroups per CU");
 
 template <int L, int DIR>
-__device__ __forceinline__ void small_item(const UArgs &a, const UItem &it, float2 *lds) {
+__device__ __forceinline__ void small_item(const UArgs &a, const UTables &tw, const UItem &it, float2 *lds) {
     using G = BlockGeom<L>;
     constexpr int N = G::N, E = G::E, TPT = G::TPT, TPW = USmall<L>::TPW;
     const int t = opaque_lane(threadIdx.x), w = t / TPT, tl = t % TPT;
@@ -86,7 +86,7 @@ __device__ __forceinline__ void small_item(const UArgs &a, const UItem &it, floa
     const float2 *src = a.in + off + tl;
 #pragma unroll
     for (int i = 0; i < E; ++i) v[i] = ld_stream(src + TPT * i);
-    block_fft<L, DIR>(v, lds + w * USmall<L>::slice, tl, a.tw.pow[L], true);
+    block_fft<L, DIR>(v, lds + w * USmall<L>::slice, tl, tw.pow[L], true);
     if (active) {
         float2 *dst = a.out + off + tl;
 #pragma unroll
@@ -97,7 +97,7 @@ __device__ __forceinline__ void small_item(const UArgs &a, const UItem &it, floa
 }
 
 template <int L, int DIR>
-__device__ __forceinline__ void large_item(const UArgs &a, const UItem &it, float2 *lds) {
+__device__ __forceinline__ void large_item(const UArgs &a, const UTables &tw, const UItem &it, float2 *lds) {
     constexpr int B1 = ULarge<L>::B1, B2 = ULarge<L>::B2, T1 = ULarge<L>::T1, T2 = ULarge<L>::T2;
     constexpr bool WIDE = ULarge<L>::wide;
     const long off = a.offs[it.first];
@@ -109,10 +109,10 @@ __device__ __forceinline__ void large_item(const UArgs &a, const UItem &it, floa
     p1.scale = 1.0f;
     if constexpr (WIDE) {
         p1.lobits = B1;
-        p1.tw_lo = a.tw.first[B1];
-        p1.tw_hi = a.tw.one;
+        p1.tw_lo = tw.first[B1];
+        p1.tw_hi = tw.one;
     } else {
-        p1.tw_local = a.tw.pow[B1];
+        p1.tw_local = tw.pow[B1];
     }
 #pragma unroll 1
     for (long tile = 0; tile < (1L << (L - B1 - T1)); ++tile) {
@@ -126,11 +126,11 @@ __device__ __forceinline__ void large_item(const UArgs &a, const UItem &it, floa
     p2.A = 1L << B1;
     p2.log2n = L;
     p2.log2S = 0;
-    p2.lobits = a.tw.lobits[L];
+    p2.lobits = tw.lobits[L];
     p2.scale = a.scale;
-    if constexpr (!WIDE) p2.tw_local = a.tw.pow[B2];
-    p2.tw_lo = a.tw.lo[L];
-    p2.tw_hi = a.tw.hi[L];
+    if constexpr (!WIDE) p2.tw_local = tw.pow[B2];
+    p2.tw_lo = tw.lo[L];
+    p2.tw_hi = tw.hi[L];
 #pragma unroll 1
     for (long tile = 0; tile < (1L << (L - B2 - T2)); ++tile) {
         if constexpr (WIDE)
@@ -148,19 +148,20 @@ __global__ void __launch_bounds__(kUThreads)
 #if ESTL_UBATCH_WAVES
 __attribute__((amdgpu_waves_per_eu(ESTL_UBATCH_WAVES, ESTL_UBATCH_WAVES)))
 #endif
-k_ubatch(UArgs args) {
+k_ubatch(UArgs a) {
     __shared__ float2 lds[kULds];
     __shared__ int s_item;
-    // The arguments are read where an item needs them, from the kernel's argument block:
-    // read ahead of the loop, those of all size classes filled the scalar registers, and each
-    // workgroup started with a dozen waits for them in a row (batches of a few hundred
-    // transforms 7.2 -> 7.9 us a call).
+    // The tables' addresses are read where an item needs them, from the kernel's argument
+    // block: read ahead of the loop, those of all size classes filled the scalar registers, and
+    // each workgroup started with a dozen waits for them in a row (batches of a few hundred
+    // transforms 7.2 -> 7.9 us a call).  The other arguments stay in registers (all of them read
+    // for each item: 100000 transforms of 2^4 .. 2^6 82.2 us, so 80.7).
     using KernArgs = const __attribute__((address_space(4))) UArgs;
     auto *ap = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
 #pragma unroll 1
     for (;;) {
         asm volatile("" : "+s"(ap));
-        const UArgs &a = *(const UArgs *)ap;
+        const UTables &tw = ((const UArgs *)ap)->tw;
         if (threadIdx.x == 0) s_item = atomicAdd(&a.counters[0], 1);
         __syncthreads();
         // the ticket and the descriptor are the same for the whole workgroup: say so, so
@@ -177,9 +178,9 @@ k_ubatch(UArgs args) {
         it.pad = 0;
         switch (it.log2n) {
 #define SMALL(L) \
-    case L: small_item<L, DIR>(a, it, lds); break;
+    case L: small_item<L, DIR>(a, tw, it, lds); break;
 #define LARGE(L) \
-    case L: large_item<L, DIR>(a, it, lds); break;
+    case L: large_item<L, DIR>(a, tw, it, lds); break;
             SMALL(1) SMALL(2) SMALL(3) SMALL(4) SMALL(5) SMALL(6) SMALL(7) SMALL(8) SMALL(9) SMALL(10) SMALL(11)
             SMALL(12) SMALL(13) LARGE(14) LARGE(15) LARGE(16) LARGE(17) LARGE(18) LARGE(19) LARGE(20)
 #undef SMALL
@@ -188,7 +189,6 @@ k_ubatch(UArgs args) {
         }
     }
     if (threadIdx.x == 0) {
-        const UArgs &a = args;
         __threadfence();
         if (atomicAdd(&a.counters[1], 1) == (int)gridDim.x - 1) {
             atomicExch(&a.counters[0], 0);
