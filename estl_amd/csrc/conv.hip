@@ -268,7 +268,9 @@ k_conv_wave(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
 }
 
 // The same for the other rows (16 values per thread, bins in natural order), persistent over
-// the pairs (four resident rounds of workgroups).
+// the pairs (four resident rounds of workgroups).  The pointers are said to be global (a
+// request group's come from its descriptor): with flat accesses 300000 rows of 64 values took
+// 166 us, with global ones 159, 5000 rows of 4096 37.7 and 36.4.
 template <int LOG2N, int TPW, bool CORR, typename R>
 __global__ void __launch_bounds__(BlockGeom<LOG2N>::TPT * TPW) __attribute__((amdgpu_waves_per_eu(4)))
 k_conv_rows(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 *__restrict__ spec,
@@ -295,7 +297,8 @@ k_conv_rows(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
             spec = group->spec[q];
         }
         const bool two = active && r1 + 1 < nrows;
-        const R *x1 = x + r1 * N + tl;
+        const R *x1 = global_ptr(x) + r1 * N + tl;
+        const float2 *bins = global_ptr(spec) + tl;
         float2 v[E];
 #pragma unroll
         for (int i = 0; i < E; ++i)
@@ -303,12 +306,12 @@ k_conv_rows(const R *__restrict__ x, R *__restrict__ y, long rows, const float2 
         block_fft<LOG2N, -1>(v, lds + w * SLICE, tl, tw, true);
 #pragma unroll
         for (int i = 0; i < E; ++i) {
-            const float2 hk = spec[tl + TPT * i];
+            const float2 hk = bins[TPT * i];
             v[i] = CORR ? cmulc(v[i], hk) : cmul(v[i], hk);
         }
         block_fft<LOG2N, +1>(v, lds + w * SLICE, tl, tw, true);
         if (active) {
-            R *y1 = y + r1 * N + tl;
+            R *y1 = global_ptr(y) + r1 * N + tl;
 #pragma unroll
             for (int i = 0; i < E; ++i) {
                 st_real(y1 + TPT * i, v[i].x * scale);
